@@ -3,230 +3,359 @@
 // 947-1030): particles are visited in index order; a particle that changed cell is removed
 // from its old table by swap-with-last (Swarm_RemoveParticleFromCell) and appended to its
 // new one (Swarm_AddParticleToCell).  The edits that touch one cell are exactly that
-// cell's removals and additions in particle-index order, so every cell can replay its own
-// events independently: stable radix sorts group the moved particles by old and by new
-// cell, and one thread per cell replays the merged sequence.
+// cell's removals and additions in particle-index order, so every cell replays its own
+// events independently.  The removals are the table's own entries whose owner changed; the
+// additions are gathered per cell with a counting pass (per-cell atomics whose order does not
+// matter: the replay takes a cell's additions by increasing index).  A cell that gains more
+// particles than that search is good for sends the call to a stable radix sort of the movers.
+#include <algorithm>
+#include <utility>
+
 #include <hipcub/hipcub.hpp>
 
+#include "uwg_geom.h"
 #include "uwg_internal.h"
 
 namespace uwg {
 
+// additions per cell up to which the replay finds them in index order by scanning; above it
+// the movers are sorted (one step of a 3D swarm at the CFL limit adds about a third of a
+// cell's particles; the scan costs na^2 / 8 reads per cell, the sort 5-6 launches per step)
+constexpr int kMaxScanAdd = 48;
+
 struct RelocWork {
   long P, E;
   int* new_owner;
-  uint8_t* moved;
-  int* ids;        // 0..P-1
-  int* mv;         // moved particle ids (ascending)
-  int* nmv;        // [1] on device
-  int* key_a;      // new owner of moved
-  int* key_r;      // old owner of moved
-  int* key_a_s;
-  int* key_r_s;
-  int* val_a_s;    // moved ids sorted by new owner (stable)
-  int* val_r_s;    // moved ids sorted by old owner (stable)
-  int* cnt_a;      // [E+1]
-  int* cnt_r;      // [E+1]
-  int* off_a;      // [E+1]
-  int* off_r;      // [E+1]
-  int* new_cnt;    // [E+1]
-  int* new_ptr;    // [E+1]
-  int* tmp_ptr;    // [E+1] scratch offsets (old + additions)
-  int* tmp_cnt;
-  int* tmp;        // scratch tables, size P + P
-  int* new_pid;    // [P]
-  int* outside;    // [1]
-  void* cub_tmp;
-  size_t cub_bytes;
+  int* rank;       // position of a mover among its new cell's additions (unordered)
+  int* cnt;        // [2][E+2]: additions, removals per cell
+  unsigned long long* off;  // [E+1]: start of a cell's new table (high word) and additions (low)
+  int* add;        // movers grouped by new cell
+  int* tmp;        // lists too long for LDS, [2 P]
+  int* ptr;        // [E+1] the new tables, exchanged with the swarm's
+  int* pid;        // [cap]
+  int* stat;       // outside count, large-cell flag, caller's two counters
+  // movers sorted by new cell (allocated on first use)
+  int *ids = nullptr, *mv = nullptr, *key = nullptr, *key_s = nullptr;
+  uint8_t* moved = nullptr;
+  void* cub_tmp = nullptr;
+  size_t cub_bytes = 0;
 };
 
 static inline unsigned nb(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-__global__ void k_iota(long n, int* x) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = (int)i;
-}
-__global__ void k_moved(long P, const int* oldo, const int* newo, uint8_t* moved) {
-  long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < P) moved[p] = oldo[p] != newo[p];
-}
-__global__ void k_keys(const int* nmv, const int* mv, const int* oldo, const int* newo, int* ka, int* kr) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < *nmv) {
-    int p = mv[i];
-    ka[i] = newo[p];
-    kr[i] = oldo[p];
-  }
-}
-__global__ void k_hist(const int* nmv, const int* keys, int* cnt) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < *nmv) atomicAdd(&cnt[keys[i]], 1);
-}
-__global__ void k_newcnt(long E, const int* ptr, const int* ca, const int* cr, int* nc, int* tc) {
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < E) {
-    int old = ptr[e + 1] - ptr[e];
-    nc[e] = old - cr[e] + ca[e];
-    tc[e] = old + ca[e];
-  }
-}
-// Per cell, replay removals/additions in particle-index order.  Eight lanes per cell copy the
-// cell's list in and out (consecutive lanes, consecutive entries); the edits themselves are
-// sequential (a removal moves the list's last entry into the hole) and run on the cell's first
-// lane between two workgroup barriers, which also make the lanes' global writes of the list
-// visible to each other.
-constexpr int kReplayLanes = 8, kReplayBlock = 256;
-__global__ __launch_bounds__(kReplayBlock) void k_replay(long E, const int* ptr, const int* pid, const int* off_a,
-                                                         const int* cnt_a, const int* val_a, const int* off_r,
-                                                         const int* cnt_r, const int* val_r, const int* tmp_ptr,
-                                                         int* tmp, const int* new_ptr, int* new_pid) {
-  __shared__ int nfin[kReplayBlock / kReplayLanes];
-  const int lane = threadIdx.x & (kReplayLanes - 1), c = threadIdx.x / kReplayLanes;
-  const long e = ((long)blockIdx.x * blockDim.x + threadIdx.x) / kReplayLanes;
-  const bool live = e < E;
-  int s0 = 0, n = 0, na = 0, nr = 0;
-  int* out = nullptr;
-  int* L = nullptr;
-  if (live) {
-    s0 = ptr[e];
-    n = ptr[e + 1] - s0;
-    na = cnt_a[e];
-    nr = cnt_r[e];
-    out = new_pid + new_ptr[e];
-    L = tmp + tmp_ptr[e];
-  }
-  const bool edit = live && (na != 0 || nr != 0);
-  if (live) {
-    int* dst = edit ? L : out;
-    for (int k = lane; k < n; k += kReplayLanes) dst[k] = pid[s0 + k];
-  }
-  __syncthreads();
-  if (edit && lane == 0) {
-    const int* A = val_a + off_a[e];
-    const int* R = val_r + off_r[e];
-    int ia = 0, ir = 0, m = n;
-    while (ia < na || ir < nr) {
-      bool take_r = ir < nr && (ia >= na || R[ir] < A[ia]);
-      if (take_r) {
-        int p = R[ir++];
-        int k = 0;
-        while (k < m && L[k] != p) k++;
-        if (k < m) {
-          L[k] = L[m - 1];
-          m--;
-        }
-      } else {
-        L[m++] = A[ia++];
-      }
+struct CellGrid {
+  int res[3];
+  double lo[3], hi[3];
+  long E;
+};
+
+// Lanes of a wave that hold the same key as this one: *leader its lowest lane, *rank this lane's
+// position among them, returned their number.  Neighbouring particles share cells, so a wave
+// meets few distinct keys, and one atomic per key (all leaders at once) replaces up to 64
+// serialised ones on one address: 0.74 ms -> 0.05 ms for the counts of 5.2 M particles.
+__device__ __forceinline__ int same_key(bool on, int key, int* leader, int* rank) {
+  const int lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  unsigned long long todo = __ballot(on);
+  int n = 0;
+  while (todo) {
+    const int first = __ffsll((long long)todo) - 1;
+    const int k = __builtin_amdgcn_readlane(key, first);
+    const unsigned long long same = __ballot(on && key == k);
+    if (on && key == k) {
+      *leader = first;
+      *rank = __popcll(same & below);
+      n = __popcll(same);
     }
-    nfin[c] = m;
+    todo &= ~same;
   }
-  __syncthreads();
-  if (edit) {
-    const int m = nfin[c], nmax = new_ptr[e + 1] - new_ptr[e];
-    for (int k = lane; k < m && k < nmax; k += kReplayLanes) out[k] = L[k];
-  }
-}
-__global__ void k_count_outside(long P, const int* owner, long E, int* out) {
-  long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < P && owner[p] >= E) atomicAdd(out, 1);
+  return n;
 }
 
-RelocWork* reloc_create(long P, long E) {
+// New owner of every particle, additions and removals per cell, and each mover's position among
+// its new cell's additions.  HBM-bound: coordinates and owner in, owner and rank out.
+template <int DIM>
+__global__ __launch_bounds__(256) void k_moves(CellGrid g, long P, const double* __restrict__ coords,
+                                               const int* __restrict__ owner, int* __restrict__ new_owner,
+                                               int* __restrict__ rank, int* __restrict__ cnt_a,
+                                               int* __restrict__ cnt_r, int* __restrict__ stat) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool live = p < P;
+  int nw = 0, old = 0;
+  if (live) {
+    double x[3];
+    for (int d = 0; d < DIM; d++) x[d] = coords[p * DIM + d];
+    nw = (int)cell_of<DIM>(g.res, g.lo, g.hi, x, g.E);
+    old = owner[p];
+    new_owner[p] = nw;
+  }
+  const int lane = threadIdx.x & 63;
+  const unsigned long long out = __ballot(live && nw >= (int)g.E);
+  if (out && lane == __ffsll((long long)out) - 1) atomicAdd(&stat[0], __popcll(out));
+  const bool moved = live && nw != old;
+  int leader = lane, r = 0;
+  const int na = same_key(moved, nw, &leader, &r);
+  int base = 0;
+  if (moved && lane == leader) base = atomicAdd(&cnt_a[nw], na);
+  base = __shfl(base, leader);
+  if (moved) {
+    rank[p] = base + r;
+    if (base + r >= kMaxScanAdd && nw < (int)g.E) stat[1] = 1;
+  }
+  const bool leaves = moved && old < (int)g.E;
+  const int nr = same_key(leaves, old, &leader, &r);
+  if (leaves && lane == leader) atomicAdd(&cnt_r[old], nr);
+}
+
+// (new table size, additions) of a cell, scanned together
+struct CellCounts {
+  const int* ptr;
+  const int* ca;
+  const int* cr;
+  int E;
+  __host__ __device__ unsigned long long operator()(int e) const {
+    if (e >= E) return 0ull;
+    const int n = ptr[e + 1] - ptr[e] - cr[e] + ca[e];
+    return ((unsigned long long)(unsigned)n << 32) | (unsigned)ca[e];
+  }
+};
+
+__global__ void k_group(long P, int E, const int* __restrict__ owner, const int* __restrict__ new_owner,
+                        const int* __restrict__ rank, const unsigned long long* __restrict__ off,
+                        int* __restrict__ add) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  const int nw = new_owner[p];
+  if (nw == owner[p] || nw >= E) return;
+  add[(unsigned)off[nw] + rank[p]] = (int)p;
+}
+
+// Per cell, replay removals/additions in particle-index order.  Eight lanes per cell: they copy
+// the table in (an entry whose owner changed carries the top bit), find the next removal and the
+// next addition by a scan and a three-step minimum, and copy the table out; the edits themselves
+// are sequential and made by the cell's first lane.  The list lives in LDS (global memory where
+// it is longer).  Latency-bound on the dependent loads table -> owner.
+constexpr int kReplayLanes = 8, kReplayBlock = 256, kReplayList = 96;
+constexpr int kReplayCells = kReplayBlock / kReplayLanes;
+constexpr unsigned kGone = 0x80000000u, kNone = 0x7fffffffu;
+template <bool SORTED>
+__global__ __launch_bounds__(kReplayBlock) void k_replay(int E, const int* __restrict__ ptr,
+                                                         const int* __restrict__ pid,
+                                                         const int* __restrict__ new_owner,
+                                                         const unsigned long long* __restrict__ off,
+                                                         const int* __restrict__ cnt_r, const int* __restrict__ add,
+                                                         int* tmp, int* __restrict__ new_ptr,
+                                                         int* __restrict__ new_pid, const int* __restrict__ stat) {
+  __shared__ unsigned list[kReplayCells][kReplayList + 1];
+  if (!SORTED && stat[1]) return;
+  const int lane = threadIdx.x & (kReplayLanes - 1), c = threadIdx.x / kReplayLanes;
+  const int e = blockIdx.x * kReplayCells + c;
+  if (e >= E) return;  // whole groups of eight lanes; nothing below waits for other groups
+  const int s0 = ptr[e], n = ptr[e + 1] - s0;
+  const unsigned long long o0 = off[e], o1 = off[e + 1];
+  const int a0 = (int)(unsigned)o0, na = (int)((unsigned)o1 - (unsigned)o0), q0 = (int)(o0 >> 32);
+  const int nr = cnt_r[e];
+  int* out = new_pid + q0;
+  if (lane == 0) {
+    new_ptr[e] = q0;
+    if (e == E - 1) new_ptr[E] = (int)(o1 >> 32);
+  }
+  if (na == 0 && nr == 0) {
+    for (int k = lane; k < n; k += kReplayLanes) out[k] = pid[s0 + k];
+    return;
+  }
+  unsigned* L = n + na <= kReplayList ? list[c] : (unsigned*)tmp + s0 + a0;
+  for (int k = lane; k < n; k += kReplayLanes) {
+    const int p = pid[s0 + k];
+    L[k] = (unsigned)p | (nr != 0 && new_owner[p] != e ? kGone : 0u);
+  }
+  __threadfence_block();
+  const int* A = add + a0;
+  auto group_min = [&](unsigned long long v) {
+    for (int s = 1; s < kReplayLanes; s <<= 1) {
+      const unsigned long long w = __shfl_xor(v, s, kReplayLanes);
+      v = w < v ? w : v;
+    }
+    return v;
+  };
+  int m = n, left_r = nr, left_a = na;
+  // (index, position) of the next removal; index of the next addition
+  auto next_removal = [&]() {
+    unsigned long long v = (unsigned long long)kNone << 32;
+    if (left_r > 0) {
+      for (int k = lane; k < m; k += kReplayLanes) {
+        const unsigned w = L[k];
+        if (w & kGone) {
+          const unsigned long long t = ((unsigned long long)(w & ~kGone) << 32) | (unsigned)k;
+          v = t < v ? t : v;
+        }
+      }
+      v = group_min(v);
+    }
+    return v;
+  };
+  auto next_addition = [&](long long last) {
+    if (left_a == 0) return kNone;
+    if (SORTED) return (unsigned)A[na - left_a];
+    unsigned long long v = kNone;
+    for (int k = lane; k < na; k += kReplayLanes) {
+      const unsigned a = (unsigned)A[k];
+      if ((long long)a > last && a < v) v = a;
+    }
+    return (unsigned)group_min(v);
+  };
+  unsigned long long r = next_removal();
+  unsigned a = next_addition(-1);
+  while (left_r > 0 || left_a > 0) {
+    if ((unsigned)(r >> 32) < a) {
+      const int k = (int)(unsigned)r;
+      m--;
+      left_r--;
+      const unsigned w = L[m];
+      if (lane == 0) L[k] = w;
+      __threadfence_block();
+      r = next_removal();
+    } else {
+      if (a == kNone) break;  // tables and owners disagree (never for tables this code keeps)
+      if (lane == 0) L[m] = a;
+      __threadfence_block();
+      m++;
+      left_a--;
+      a = next_addition((long long)a);
+    }
+  }
+  const int room = (int)(o1 >> 32) - q0;
+  for (int k = lane; k < m && k < room; k += kReplayLanes) out[k] = (int)(L[k] & ~kGone);
+}
+
+__global__ void k_iota_moved(long P, const int* __restrict__ oldo, const int* __restrict__ newo, int* __restrict__ ids,
+                             uint8_t* __restrict__ moved) {
+  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= P) return;
+  ids[p] = (int)p;
+  moved[p] = oldo[p] != newo[p];
+}
+__global__ void k_keys(int n, const int* __restrict__ mv, const int* __restrict__ newo, int* __restrict__ key) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) key[i] = newo[mv[i]];
+}
+
+// P: particles; cap: capacity of the swarm's particle arrays (the tables are exchanged with them)
+RelocWork* reloc_create(long P, long E, long cap) {
   RelocWork* w = new RelocWork();
   w->P = P;
   w->E = E;
-  long Pm = P > 0 ? P : 1;
-  UWG_HIP(hipMalloc(&w->new_owner, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->moved, Pm));
-  UWG_HIP(hipMalloc(&w->ids, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->mv, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->nmv, sizeof(int) * 2));
-  UWG_HIP(hipMalloc(&w->key_a, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->key_r, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->key_a_s, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->key_r_s, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->val_a_s, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->val_r_s, sizeof(int) * Pm));
-  for (int** a : {&w->cnt_a, &w->cnt_r, &w->off_a, &w->off_r, &w->new_cnt, &w->new_ptr, &w->tmp_ptr, &w->tmp_cnt})
-    UWG_HIP(hipMalloc(a, sizeof(int) * (E + 2)));
+  const long Pm = P > 0 ? P : 1;
+  if (cap < Pm) cap = Pm;
+  UWG_HIP(hipMalloc(&w->new_owner, sizeof(int) * cap));
+  UWG_HIP(hipMalloc(&w->pid, sizeof(int) * cap));
+  UWG_HIP(hipMalloc(&w->rank, sizeof(int) * Pm));
+  UWG_HIP(hipMalloc(&w->add, sizeof(int) * Pm));
   UWG_HIP(hipMalloc(&w->tmp, sizeof(int) * 2 * Pm));
-  UWG_HIP(hipMalloc(&w->new_pid, sizeof(int) * Pm));
-  UWG_HIP(hipMalloc(&w->outside, sizeof(int)));
-  hipLaunchKernelGGL(k_iota, nb(Pm, 256), 256, 0, 0, Pm, w->ids);
-  // temp storage: max over the primitives used
-  size_t b1 = 0, b2 = 0, b3 = 0;
-  hipcub::DeviceSelect::Flagged(nullptr, b1, w->ids, w->moved, w->mv, w->nmv, (int)Pm);
-  hipcub::DeviceRadixSort::SortPairs(nullptr, b2, w->key_a, w->key_a_s, w->mv, w->val_a_s, (int)Pm);
-  hipcub::DeviceScan::ExclusiveSum(nullptr, b3, w->cnt_a, w->off_a, (int)(E + 1));
-  w->cub_bytes = b1;
-  if (b2 > w->cub_bytes) w->cub_bytes = b2;
-  if (b3 > w->cub_bytes) w->cub_bytes = b3;
+  UWG_HIP(hipMalloc(&w->cnt, sizeof(int) * (2 * (E + 2) + 4)));
+  w->stat = w->cnt + 2 * (E + 2);
+  UWG_HIP(hipMalloc(&w->off, sizeof(unsigned long long) * (E + 2)));
+  UWG_HIP(hipMalloc(&w->ptr, sizeof(int) * (E + 1)));
+  const CellCounts f{w->ptr, w->cnt, w->cnt, (int)E};
+  hipcub::TransformInputIterator<unsigned long long, CellCounts, hipcub::CountingInputIterator<int>> in(
+      hipcub::CountingInputIterator<int>(0), f);
+  UWG_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, w->cub_bytes, in, w->off, (int)(E + 1)));
   UWG_HIP(hipMalloc(&w->cub_tmp, w->cub_bytes));
   return w;
 }
 
 void reloc_destroy(RelocWork* w) {
   if (!w) return;
-  for (void* p : {(void*)w->new_owner, (void*)w->moved, (void*)w->ids, (void*)w->mv, (void*)w->nmv, (void*)w->key_a,
-                  (void*)w->key_r, (void*)w->key_a_s, (void*)w->key_r_s, (void*)w->val_a_s, (void*)w->val_r_s,
-                  (void*)w->cnt_a, (void*)w->cnt_r, (void*)w->off_a, (void*)w->off_r, (void*)w->new_cnt,
-                  (void*)w->new_ptr, (void*)w->tmp_ptr, (void*)w->tmp_cnt, (void*)w->tmp, (void*)w->new_pid,
-                  (void*)w->outside, w->cub_tmp})
+  for (void* p : {(void*)w->new_owner, (void*)w->pid, (void*)w->rank, (void*)w->add, (void*)w->tmp, (void*)w->cnt,
+                  (void*)w->off, (void*)w->ptr, (void*)w->ids, (void*)w->mv, (void*)w->key, (void*)w->key_s,
+                  (void*)w->moved, w->cub_tmp})
     (void)hipFree(p);
   delete w;
 }
 
-long relocate(const Geom& g, long P, const double* coords, int* owner, int* cell_ptr, int* cell_pid, RelocWork* w,
-              hipStream_t s) {
-  const long E = g.E;
-  if (P == 0) return 0;
-  launch_cell_of(g, P, coords, w->new_owner, s);
-  hipLaunchKernelGGL(k_moved, nb(P, 256), 256, 0, s, P, owner, w->new_owner, w->moved);
-  size_t bytes = w->cub_bytes;
-  UWG_HIP(hipcub::DeviceSelect::Flagged(w->cub_tmp, bytes, w->ids, w->moved, w->mv, w->nmv, (int)P, s));
-  int nmv = 0;
-  UWG_HIP(hipMemcpyAsync(&nmv, w->nmv, sizeof(int), hipMemcpyDeviceToHost, s));
-  UWG_HIP(hipStreamSynchronize(s));
-  UWG_HIP(hipMemsetAsync(w->cnt_a, 0, sizeof(int) * (E + 2), s));
-  UWG_HIP(hipMemsetAsync(w->cnt_r, 0, sizeof(int) * (E + 2), s));
-  int bits = 1;
-  while ((1L << bits) <= E) bits++;
-  if (nmv > 0) {
-    hipLaunchKernelGGL(k_keys, nb(nmv, 256), 256, 0, s, w->nmv, w->mv, owner, w->new_owner, w->key_a, w->key_r);
-    bytes = w->cub_bytes;
-    UWG_HIP(hipcub::DeviceRadixSort::SortPairs(w->cub_tmp, bytes, w->key_a, w->key_a_s, w->mv, w->val_a_s, nmv, 0,
-                                               bits, s));
-    bytes = w->cub_bytes;
-    UWG_HIP(hipcub::DeviceRadixSort::SortPairs(w->cub_tmp, bytes, w->key_r, w->key_r_s, w->mv, w->val_r_s, nmv, 0,
-                                               bits, s));
-    hipLaunchKernelGGL(k_hist, nb(nmv, 256), 256, 0, s, w->nmv, w->key_a, w->cnt_a);
-    hipLaunchKernelGGL(k_hist, nb(nmv, 256), 256, 0, s, w->nmv, w->key_r, w->cnt_r);
+// additions of every cell in index order: the movers, stably sorted by new cell
+static void sort_movers(RelocWork* w, const int* owner, hipStream_t s) {
+  const long P = w->P;
+  if (!w->ids) {
+    for (int** a : {&w->ids, &w->mv, &w->key, &w->key_s}) UWG_HIP(hipMalloc(a, sizeof(int) * P));
+    UWG_HIP(hipMalloc(&w->moved, P));
+    size_t b1 = 0, b2 = 0;
+    UWG_HIP(hipcub::DeviceSelect::Flagged(nullptr, b1, w->ids, w->moved, w->mv, w->stat, (int)P));
+    UWG_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, b2, w->key, w->key_s, w->mv, w->add, (int)P));
+    const size_t need = std::max(b1, b2);
+    if (need > w->cub_bytes) {
+      UWG_HIP(hipFree(w->cub_tmp));
+      w->cub_tmp = nullptr;
+      UWG_HIP(hipMalloc(&w->cub_tmp, need));
+      w->cub_bytes = need;
+    }
   }
-  bytes = w->cub_bytes;
-  UWG_HIP(hipcub::DeviceScan::ExclusiveSum(w->cub_tmp, bytes, w->cnt_a, w->off_a, (int)(E + 1), s));
-  bytes = w->cub_bytes;
-  UWG_HIP(hipcub::DeviceScan::ExclusiveSum(w->cub_tmp, bytes, w->cnt_r, w->off_r, (int)(E + 1), s));
-  hipLaunchKernelGGL(k_newcnt, nb(E, 256), 256, 0, s, E, cell_ptr, w->cnt_a, w->cnt_r, w->new_cnt, w->tmp_cnt);
-  UWG_HIP(hipMemsetAsync(w->new_cnt + E, 0, sizeof(int), s));
-  UWG_HIP(hipMemsetAsync(w->tmp_cnt + E, 0, sizeof(int), s));
-  bytes = w->cub_bytes;
-  UWG_HIP(hipcub::DeviceScan::ExclusiveSum(w->cub_tmp, bytes, w->new_cnt, w->new_ptr, (int)(E + 1), s));
-  bytes = w->cub_bytes;
-  UWG_HIP(hipcub::DeviceScan::ExclusiveSum(w->cub_tmp, bytes, w->tmp_cnt, w->tmp_ptr, (int)(E + 1), s));
-  hipLaunchKernelGGL(k_replay, nb(E * kReplayLanes, kReplayBlock), kReplayBlock, 0, s, E, cell_ptr, cell_pid, w->off_a,
-                     w->cnt_a, w->val_a_s, w->off_r,
-                     w->cnt_r, w->val_r_s, w->tmp_ptr, w->tmp, w->new_ptr, w->new_pid);
-  UWG_HIP(hipGetLastError());
-  UWG_HIP(hipMemcpyAsync(cell_ptr, w->new_ptr, sizeof(int) * (E + 1), hipMemcpyDeviceToDevice, s));
-  UWG_HIP(hipMemcpyAsync(cell_pid, w->new_pid, sizeof(int) * P, hipMemcpyDeviceToDevice, s));
-  UWG_HIP(hipMemcpyAsync(owner, w->new_owner, sizeof(int) * P, hipMemcpyDeviceToDevice, s));
-  UWG_HIP(hipMemsetAsync(w->outside, 0, sizeof(int), s));
-  hipLaunchKernelGGL(k_count_outside, nb(P, 256), 256, 0, s, P, owner, E, w->outside);
-  int outside = 0;
-  UWG_HIP(hipMemcpyAsync(&outside, w->outside, sizeof(int), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_iota_moved, nb(P, 256), 256, 0, s, P, owner, w->new_owner, w->ids, w->moved);
+  size_t bytes = w->cub_bytes;
+  int* nmv = w->stat + 1;  // the flag has been read
+  UWG_HIP(hipcub::DeviceSelect::Flagged(w->cub_tmp, bytes, w->ids, w->moved, w->mv, nmv, (int)P, s));
+  int n = 0;
+  UWG_HIP(hipMemcpyAsync(&n, nmv, sizeof(int), hipMemcpyDeviceToHost, s));
   UWG_HIP(hipStreamSynchronize(s));
-  return outside;
+  if (n == 0) return;
+  int bits = 1;
+  while ((1L << bits) <= w->E) bits++;
+  hipLaunchKernelGGL(k_keys, nb(n, 256), 256, 0, s, n, w->mv, w->new_owner, w->key);
+  bytes = w->cub_bytes;
+  UWG_HIP(hipcub::DeviceRadixSort::SortPairs(w->cub_tmp, bytes, w->key, w->key_s, w->mv, w->add, n, 0, bits, s));
+}
+
+void reloc_begin(RelocWork* w, hipStream_t s) {
+  UWG_HIP(hipMemsetAsync(w->cnt, 0, sizeof(int) * (2 * (w->E + 2) + 4), s));
+}
+int* reloc_counters(RelocWork* w) { return w->stat + 2; }
+
+// The new tables are built beside the old ones and exchanged with them at the end; they are not
+// when counters[0] (particles the caller could not move) is non-zero.
+long relocate(const Geom& g, long P, const double* coords, int*& owner, int*& cell_ptr, int*& cell_pid, RelocWork* w,
+              hipStream_t s, int* counters) {
+  const int E = (int)g.E;
+  if (P == 0) return 0;
+  if (!counters) reloc_begin(w, s);
+  CellGrid cg;
+  for (int d = 0; d < 3; d++) {
+    cg.res[d] = g.res[d];
+    cg.lo[d] = g.lo[d];
+    cg.hi[d] = g.hi[d];
+  }
+  cg.E = g.E;
+  int *ca = w->cnt, *cr = w->cnt + E + 2;
+  if (g.dim == 3)
+    hipLaunchKernelGGL(k_moves<3>, nb(P, 256), 256, 0, s, cg, P, coords, owner, w->new_owner, w->rank, ca, cr, w->stat);
+  else
+    hipLaunchKernelGGL(k_moves<2>, nb(P, 256), 256, 0, s, cg, P, coords, owner, w->new_owner, w->rank, ca, cr, w->stat);
+  const CellCounts f{cell_ptr, ca, cr, E};
+  hipcub::TransformInputIterator<unsigned long long, CellCounts, hipcub::CountingInputIterator<int>> in(
+      hipcub::CountingInputIterator<int>(0), f);
+  size_t bytes = w->cub_bytes;
+  UWG_HIP(hipcub::DeviceScan::ExclusiveSum(w->cub_tmp, bytes, in, w->off, E + 1, s));
+  hipLaunchKernelGGL(k_group, nb(P, 256), 256, 0, s, P, E, owner, w->new_owner, w->rank, w->off, w->add);
+  hipLaunchKernelGGL(k_replay<false>, nb(E, kReplayCells), kReplayBlock, 0, s, E, cell_ptr, cell_pid, w->new_owner,
+                     w->off, cr, w->add, w->tmp, w->ptr, w->pid, w->stat);
+  UWG_HIP(hipGetLastError());
+  int h[4];
+  UWG_HIP(hipMemcpyAsync(h, w->stat, sizeof(h), hipMemcpyDeviceToHost, s));
+  UWG_HIP(hipStreamSynchronize(s));
+  if (counters) {
+    counters[0] = h[2];
+    counters[1] = h[3];
+    if (h[2] > 0) return 0;
+  }
+  if (h[1]) {
+    sort_movers(w, owner, s);
+    hipLaunchKernelGGL(k_replay<true>, nb(E, kReplayCells), kReplayBlock, 0, s, E, cell_ptr, cell_pid, w->new_owner,
+                       w->off, cr, w->add, w->tmp, w->ptr, w->pid, w->stat);
+    UWG_HIP(hipGetLastError());
+  }
+  std::swap(owner, w->new_owner);
+  std::swap(cell_ptr, w->ptr);
+  std::swap(cell_pid, w->pid);
+  return h[0];
 }
 
 // Exclusive prefix sum of 0/1 flags into 64-bit counts (the particle layout's skip counts).

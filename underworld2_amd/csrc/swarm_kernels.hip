@@ -181,27 +181,6 @@ void launch_mesh_coords(const Geom& g, double* out, hipStream_t s) {
   UWG_HIP(hipGetLastError());
 }
 
-// ---------------------------------------------------------------------------------------
-// A17 cell search for every particle (owner = E when outside the domain)
-// ---------------------------------------------------------------------------------------
-template <int DIM>
-__global__ void k_cell_of(GeomArgs g, long P, const double* coords, int* owner) {
-  long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= P) return;
-  double x[3];
-  for (int d = 0; d < DIM; d++) x[d] = coords[p * DIM + d];
-  owner[p] = (int)cell_of<DIM>(g.res, g.lo, g.hi, x, g.E);
-}
-
-void launch_cell_of(const Geom& g, long P, const double* coords, int* owner, hipStream_t s) {
-  if (P == 0) return;
-  if (g.dim == 3)
-    hipLaunchKernelGGL(k_cell_of<3>, nblocks(P, 256), 256, 0, s, pack(g), P, coords, owner);
-  else
-    hipLaunchKernelGGL(k_cell_of<2>, nblocks(P, 256), 256, 0, s, pack(g), P, coords, owner);
-  UWG_HIP(hipGetLastError());
-}
-
 // slot -> owning cell, from the CSR cell pointer
 __global__ void k_slot_cell(long E, const int* cell_ptr, int* slot_cell) {
   long e = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -458,7 +458,7 @@ extern "C" int uwg_swarm_destroy(uwg_swarm* s) {
 static void ensure_reloc(uwg_swarm* s) {
   if (!s->reloc || s->reloc_P != s->P) {
     reloc_destroy(s->reloc);
-    s->reloc = reloc_create(s->P, s->mesh->g.E);
+    s->reloc = reloc_create(s->P, s->mesh->g.E, s->cap);
     s->reloc_P = s->P;
   }
 }
@@ -576,10 +576,8 @@ extern "C" int uwg_swarm_set_material(uwg_swarm* s, const int* mat) {
   return 0;
   API_END
 }
-extern "C" int uwg_swarm_update_owners(uwg_swarm* s, long* outside) {
-  API_BEGIN
-  ensure_reloc(s);
-  long o = relocate(s->mesh->g, s->P, s->coords, s->owner, s->cell_ptr, s->cell_pid, s->reloc, 0);
+// bookkeeping after a relocation that left `o` particles outside the mesh
+static int owners_updated(uwg_swarm* s, long o, long* outside) {
   if (outside) *outside = o;
   s->state++;
   s->geom_state++;
@@ -588,6 +586,13 @@ extern "C" int uwg_swarm_update_owners(uwg_swarm* s, long* outside) {
     return UWG_ERR_DOMAIN;
   }
   return 0;
+}
+
+extern "C" int uwg_swarm_update_owners(uwg_swarm* s, long* outside) {
+  API_BEGIN
+  ensure_reloc(s);
+  return owners_updated(s, relocate(s->mesh->g, s->P, s->coords, s->owner, s->cell_ptr, s->cell_pid, s->reloc, 0),
+                        outside);
   API_END
 }
 
@@ -729,12 +734,15 @@ extern "C" int uwg_advect_rk2(uwg_swarm* s, uwg_field* vel, double dt, int updat
   if (vel->mesh != s->mesh || vel->on_elements || vel->ncomp != s->mesh->g.dim)
     return arg_error("velocity field must be a nodal vector field on the swarm's mesh");
   API_BEGIN
-  int* cnt = dalloc<int>(2);
-  UWG_HIP(hipMemset(cnt, 0, sizeof(int) * 2));
-  launch_advect_rk2(s->mesh->g, s->P, vel->d, s->coords, dt, cnt, 0, vel->mesh->order);
-  int h[2];
-  UWG_HIP(hipMemcpy(h, cnt, sizeof(int) * 2, hipMemcpyDeviceToHost));
-  dfree(cnt);
+  ensure_reloc(s);
+  reloc_begin(s->reloc, 0);
+  launch_advect_rk2(s->mesh->g, s->P, vel->d, s->coords, dt, reloc_counters(s->reloc), 0, vel->mesh->order);
+  int h[2] = {0, 0};  // particles without a velocity, first-order fallbacks
+  long o = 0;
+  if (update_owners)
+    o = relocate(s->mesh->g, s->P, s->coords, s->owner, s->cell_ptr, s->cell_pid, s->reloc, 0, h);
+  else
+    UWG_HIP(hipMemcpy(h, reloc_counters(s->reloc), sizeof(h), hipMemcpyDeviceToHost));
   s->state++;
   s->geom_state++;
   if (h[0] > 0) {
@@ -742,8 +750,7 @@ extern "C" int uwg_advect_rk2(uwg_swarm* s, uwg_field* vel, double dt, int updat
               " particle(s): coordinate outside the global domain");
     return UWG_ERR_DOMAIN;
   }
-  if (update_owners) return uwg_swarm_update_owners(s, outside);
-  return 0;
+  return update_owners ? owners_updated(s, o, outside) : 0;
   API_END
 }
 

@@ -66,7 +66,6 @@ void launch_layout_sobol(const Geom& g, int ppc, long seed, double* coords, hipS
 // out[i] = sum of flags[0..i-1] (relocate.hip, hipcub)
 void scan_exclusive_flags(const int* flags, long long* out, long n, hipStream_t s);
 void launch_mesh_coords(const Geom& g, double* out, hipStream_t s);
-void launch_cell_of(const Geom& g, long P, const double* coords, int* owner, hipStream_t s);
 void launch_coincident_map(const Geom& g, long P, const int* slot_cell, const int* cell_pid,
                            const double* coords, double* xi_slot, hipStream_t s);
 void launch_slot_cell(long E, const int* cell_ptr, int* slot_cell, hipStream_t s);
@@ -139,10 +138,14 @@ void launch_dvc_list(int dim, int num, long E0, long nE, const int* elist, const
 // relocation (relocate.hip): rebuild per-cell tables after owners change; returns the number
 // of particles outside the domain
 struct RelocWork;
-RelocWork* reloc_create(long P, long E);
+RelocWork* reloc_create(long P, long E, long cap);
 void reloc_destroy(RelocWork* w);
-long relocate(const Geom& g, long P, const double* coords, int* owner, int* cell_ptr, int* cell_pid,
-              RelocWork* w, hipStream_t s);
+// clears the counts; reloc_counters: two device counters a caller's kernel may use between
+// reloc_begin and relocate (which then reads them back into counters[2])
+void reloc_begin(RelocWork* w, hipStream_t s);
+int* reloc_counters(RelocWork* w);
+long relocate(const Geom& g, long P, const double* coords, int*& owner, int*& cell_ptr, int*& cell_pid,
+              RelocWork* w, hipStream_t s, int* counters = nullptr);
 void launch_bc_mask_from_walls(const Geom& g, uint8_t* bc, int wallbits, hipStream_t s);
 void launch_inject_bc(const Geom& f, const Geom& c, const uint8_t* fbc, uint8_t* cbc, hipStream_t s);
 void launch_fill_hash(long n, double* x, hipStream_t s);
