@@ -1,0 +1,79 @@
+"""K applies of small grids against the streaming element kernels (selected with an explicit
+chunk, themselves checked against the oracle in test_gpu_parity3d.py).
+
+3D: the kernel that evaluates a chunk's element levels side by side shares the element arithmetic
+and the order of the node sums, so every value is equal; grids at the tile edges (7 columns), the
+level counts 2, 3 and 4 of its dispatch and one element.
+2D: the assembled stencil sums the same terms in another order: per row 36 products and sums of
+rounding u each, so |dy| <= 40 u sum|K||x| (u = 2^-53, 2^-24); FP32 entries add u.  Irregular
+Dirichlet masks reach every form of the row-sum block."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _system(res, hi, seed, mask=None):
+    import underworld2_amd as uw
+    from underworld2_amd import _lib as L
+    d = len(res)
+    rng = np.random.default_rng(seed)
+    mesh = uw.mesh.FeMesh_Cartesian("Q1/dQ0", res, (0.0,) * d, hi)
+    v, p = uw.mesh.MeshVariable(mesh, d), uw.mesh.MeshVariable(mesh.subMesh, 1)
+    sets = mesh.specialSets
+    if mask is None:
+        walls = tuple(sets[f"Min{a}_VertexSet"] + sets[f"Max{a}_VertexSet"] for a in "IJK"[:d])
+    else:
+        walls = tuple(uw.mesh.IndexSet(np.flatnonzero(rng.random(mesh.nodesGlobal) < mask), mesh.nodesGlobal)
+                      for _ in range(d))
+    st = uw.systems.Stokes(v, p, fn_viscosity=1.0, fn_bodyforce=(0.0,) * d,
+                           conditions=[uw.conditions.DirichletCondition(v, walls)])
+    eta = np.exp(2.0 * rng.standard_normal((mesh.elementsGlobal, 3 ** d)))
+    L.check(L.lib().uwg_stokes_assemble_fields(st._h, L.dptr(eta), None))
+    return mesh, v, p, st, rng.standard_normal(mesh.nodesGlobal * d)
+
+
+def _apply(st, which, x):
+    from underworld2_amd import _lib as L
+    y = np.zeros_like(x)
+    L.check(L.lib().uwg_stokes_apply(st._h, which, 0, L.dptr(x), L.dptr(y)))
+    return y
+
+
+@pytest.mark.parametrize("res", [(1, 1, 1), (6, 7, 2), (7, 6, 13), (8, 15, 3), (22, 13, 9), (26, 28, 30), (36, 41, 40)])
+def test_3d_levels_side_by_side_equal_streaming(res):
+    from underworld2_amd import _lib as L
+    *keep, st, x = _system(res, (1.0, 0.9, 1.3), 3)
+    got = [_apply(st, w, x) for w in (0, 4, 5, 6, 7)]
+    try:
+        L.lib().uwg_set_apply_chunk(2, 0)
+        ref = [_apply(st, w, x) for w in (0, 4, 5, 6, 7)]
+    finally:
+        L.lib().uwg_set_apply_chunk(-1, 0)
+    for a, b in zip(got, ref):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("res,mask", [((1, 1), None), ((3, 2), 0.3), ((31, 29), 0.1), ((64, 5), None), ((130, 61), 0.02)])
+def test_2d_stencil_against_element_kernel(res, mask):
+    from underworld2_amd import _lib as L
+    *keep, st, x = _system(res, (1.0, 1.3), 4, mask)
+    got = [_apply(st, w, x) for w in (0, 4, 6, 7)]
+    try:
+        L.lib().uwg_set_apply_chunk(0, 1)
+        ref = [_apply(st, w, x) for w in (0, 4, 6, 7)]
+        # sum |K| |x| row by row is bounded by the largest row sum times max |x|; the row sum of
+        # |K| is at most 18 times its largest entry, itself at most the largest diagonal entry
+        n = x.size
+        diag = np.zeros(n)
+        for c in range(18):  # the diagonal by colouring: unit vectors three nodes apart
+            e = np.zeros((res[1] + 1, res[0] + 1, 2))
+            e[(c // 2) // 3::3, (c // 2) % 3::3, c % 2] = 1.0
+            e = e.ravel()
+            diag += e * _apply(st, 0, e)
+    finally:
+        L.lib().uwg_set_apply_chunk(0, 32)
+    bound = 40 * 18 * diag.max() * np.abs(x).max()
+    for a, b, u in zip(got, ref, (2.0 ** -53, 2.0 ** -24, 2.0 ** -53, 2.0 ** -24)):
+        assert np.abs(a - b).max() <= u * bound
+        assert np.linalg.norm(a - b) <= 20 * u * np.linalg.norm(b)

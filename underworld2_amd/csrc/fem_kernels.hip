@@ -500,6 +500,9 @@ struct KArgs {
   int ntx, nty;      // 3D: tiles of 16 x 16 element columns (overlapping by one)
 };
 
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 template <typename T, typename WF>
 __device__ __forceinline__ void elem3(WF wq, const T (&u)[8][3], T (&r)[8][3], T sx, T sy, T sz) {
   const T q8 = (T)0.125;
@@ -535,8 +538,13 @@ __device__ __forceinline__ void elem3(WF wq, const T (&u)[8][3], T (&r)[8][3], T
 #pragma unroll
       for (int k = 0; k < 3; k++) {
         const T K = (T)gpt(k);  // Y for x-lines, X for y-lines
-        GX[i][k] = sx * (cX[i] + cXY[i] * K + cXZ[i] * Z + cXYZ[i] * (K * Z));
-        GY[i][k] = sy * (cY[i] + cXY[i] * K + cYZ[i] * Z + cXYZ[i] * (K * Z));
+        // du_i/dx along x-lines, du_i/dy along y-lines; those that enter the sums only through a
+        // shear stress are kept without their factor, which the fused multiply-add there applies
+        // (spelled out, as below, so that every kernel rounds the element alike)
+        const T gx = cX[i] + cXY[i] * K + cXZ[i] * Z + cXYZ[i] * (K * Z);
+        const T gy = cY[i] + cXY[i] * K + cYZ[i] * Z + cXYZ[i] * (K * Z);
+        GX[i][k] = i == 0 ? sx * gx : gx;
+        GY[i][k] = i == 2 ? gy : sy * gy;
         PX[i][k] = (T)0;
         PY[i][k] = (T)0;
       }
@@ -547,12 +555,12 @@ __device__ __forceinline__ void elem3(WF wq, const T (&u)[8][3], T (&r)[8][3], T
         const T X = (T)gpt(gx), Y = (T)gpt(gy);
         const T w = wq(gx + 3 * gy + 9 * gz);
         const T w2 = w + w;
-        const T G00 = GX[0][gy], G10 = GX[1][gy], G20 = GX[2][gy];
-        const T G01 = GY[0][gx], G11 = GY[1][gx], G21 = GY[2][gx];
+        const T G00 = GX[0][gy], G11 = GY[1][gx];
         T G2[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) G2[i] = sz * (cZ[i] + cXZ[i] * X + cYZ[i] * Y + cXYZ[i] * (X * Y));
-        const T S01 = w * (G01 + G10), S02 = w * (G2[0] + G20), S12 = w * (G2[1] + G21);
+        const T S01 = w * fma_t(sx, GX[1][gy], GY[0][gx]), S02 = w * fma_t(sx, GX[2][gy], G2[0]),
+                S12 = w * fma_t(sy, GY[2][gx], G2[1]);
         PX[0][gy] += w2 * G00;
         PX[1][gy] += S01;
         PX[2][gy] += S02;
@@ -563,9 +571,9 @@ __device__ __forceinline__ void elem3(WF wq, const T (&u)[8][3], T (&r)[8][3], T
 #pragma unroll
         for (int i = 0; i < 3; i++) {
           dZ[i] += pz[i];
-          dXZ[i] += pz[i] * X;
-          dYZ[i] += pz[i] * Y;
-          dXYZ[i] += pz[i] * (X * Y);
+          dXZ[i] = fma_t(pz[i], X, dXZ[i]);
+          dYZ[i] = fma_t(pz[i], Y, dYZ[i]);
+          dXYZ[i] = fma_t(pz[i], X * Y, dXYZ[i]);
         }
       }
     // fold the x- and y-lines of this plane into the dual coefficients
@@ -576,13 +584,13 @@ __device__ __forceinline__ void elem3(WF wq, const T (&u)[8][3], T (&r)[8][3], T
         const T K = (T)gpt(k);
         const T px = PX[i][k] * sx, py = PY[i][k] * sy;
         dX[i] += px;
-        dXY[i] += px * K;
-        dXZ[i] += px * Z;
-        dXYZ[i] += px * (K * Z);
+        dXY[i] = fma_t(px, K, dXY[i]);
+        dXZ[i] = fma_t(px, Z, dXZ[i]);
+        dXYZ[i] = fma_t(px, K * Z, dXYZ[i]);
         dY[i] += py;
-        dXY[i] += py * K;
-        dYZ[i] += py * Z;
-        dXYZ[i] += py * (K * Z);
+        dXY[i] = fma_t(py, K, dXY[i]);
+        dYZ[i] = fma_t(py, Z, dYZ[i]);
+        dXYZ[i] = fma_t(py, K * Z, dXYZ[i]);
       }
   }
 #pragma unroll
@@ -743,10 +751,11 @@ __device__ __forceinline__ void elem3_lines(WF wq, const T (&u)[8][3], T (&r)[8]
     const T eZ = q0[0] + q0[1] + q0[2], eYZz = q0[2] - q0[0];
     const T eXZz = q1[0] + q1[1] + q1[2], eXYZz = q1[2] - q1[0];
     const T dX = hx * eX[i], dY = hy * eY[i], dZ = hz * eZ;
-    const T dXY = g * (hx * eXYx[i] + hy * eXYy[i]);
-    const T dXZ = g * (hx * eXZx[i] + hz * eXZz);
-    const T dYZ = g * (hy * eYZy[i] + hz * eYZz);
-    const T dXYZ = g2 * (hx * eXYZx[i] + hy * eXYZy[i] + hz * eXYZz);
+    // sums of two products, the fused one spelled out so that every kernel rounds them alike
+    const T dXY = g * fma_t(hx, eXYx[i], hy * eXYy[i]);
+    const T dXZ = g * fma_t(hz, eXZz, hx * eXZx[i]);
+    const T dYZ = g * fma_t(hz, eYZz, hy * eYZy[i]);
+    const T dXYZ = g2 * fma_t(hz, eXYZz, fma_t(hx, eXYZx[i], hy * eXYZy[i]));
     // r_a = s dX + t dY + r dZ + st dXY + sr dXZ + tr dYZ + str dXYZ, a = (s, t, r) bits
     const T pp = dX + dXY, pm = dX - dXY;  // s-coefficient of F for t = +1 / -1
     const T F0 = -pm - dY, F1 = pm - dY, F2 = dY - pp, F3 = pp + dY;  // F(s,t), a = s + 2t bits
@@ -1060,6 +1069,79 @@ __global__ __launch_bounds__(256, 2) void k_apply3f(KArgs<float> A, const void* 
   });
 }
 
+// The same applies for small grids.  Streaming up z makes a launch take KZ + 1 dependent element
+// evaluations (4-6 us each at one wave per SIMD) however few elements there are.  Here the KL
+// element levels of a chunk are evaluated side by side, one wave per level of an 8 x 8 column
+// tile, and meet in LDS: one evaluation deep, at the price of evaluating (8/7)^2 KL/(KL-1) times
+// the elements.  Same element kernels and the same order of the node sums as k_apply3 /
+// k_apply3f, so the results are theirs bit for bit.
+template <typename T, int MODE, bool BF, int KL>
+__global__ __launch_bounds__(64 * KL) void k_apply3s(KArgs<T> A, const void* __restrict__ W,
+                                                       const T* __restrict__ x, T* __restrict__ y,
+                                                       const uint8_t* __restrict__ bc, SmoothArgs<T> S) {
+  __shared__ T sb[KL][12][64];
+  __shared__ T st[KL][12][64];
+  const int tid = threadIdx.x & 63, lx = tid & 7, ly = tid >> 3;
+  const int lz = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = xcd_logical_id();
+  const int bx = t % A.ntx, by = (t / A.ntx) % A.nty, k0 = (t / (A.ntx * A.nty)) * (KL - 1);
+  const int ei = bx * 7 - 1 + lx, ej = by * 7 - 1 + ly, ek = k0 - 1 + lz;
+  const bool elem = ei >= 0 && ei < A.rx && ej >= 0 && ej < A.ry && ek >= 0 && ek < A.rz;
+  // the wave's element level also owns the node level below it (the first wave is the halo)
+  const bool node = lz >= 1 && lx >= 1 && ly >= 1 && ei <= A.rx && ej <= A.ry && ek <= A.rz;
+  const uint32_t nN = node ? (uint32_t)(ei + A.nx * ej + A.nxy * ek) : 0u;
+  const uint32_t eo = elem ? (uint32_t)(ei + A.rx * (ej + A.ry * ek)) * (uint32_t)sizeof(T) : 0u;
+  LevelLoad<T> lo, hi;
+  lo.issue(A, x, bc, ei, ej, ek);
+  hi.issue(A, x, bc, ei, ej, ek + 1);
+  NodeOperands<T, MODE> nd;
+  nd.load(S, x, bc, nN);
+  T u[8][3], r[8][3];
+  uint32_t wn[sizeof(T) == 4 ? (BF ? 14 : 27) : 1];
+  if constexpr (sizeof(T) == 4) {
+    constexpr int NW = BF ? 14 : 27;
+    const __amdgpu_buffer_rsrc_t wr = weight_rsrc((const float*)W, (uint32_t)(NW * A.Ws * 4));
+#pragma unroll
+    for (int q = 0; q < NW; q++) wn[q] = ld_buf_u32(wr, eo, q * (uint32_t)(A.Ws * 4));
+  }
+  lo.finish(u, 0);
+  hi.finish(u, 4);
+  if (elem) {
+    if constexpr (sizeof(T) == 4)
+      elem3_lines<float>(
+          [&](int q) {
+            if constexpr (BF)
+              return __uint_as_float((q & 1) ? (wn[q >> 1] & 0xffff0000u) : (wn[q >> 1] << 16));
+            else
+              return __uint_as_float(wn[q]);
+          },
+          u, r, A.sx, A.sy, A.sz);
+    else
+      elem3<T>([&](int q) { return ld_off((const T*)W + (long)q * A.Ws, eo); }, u, r, A.sx, A.sy, A.sz);
+  } else {
+#pragma unroll
+    for (int a = 0; a < 8; a++)
+#pragma unroll
+      for (int i = 0; i < 3; i++) r[a][i] = (T)0;
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      sb[lz][c * 3 + i][tid] = r[c][i];
+      st[lz][c * 3 + i][tid] = r[4 + c][i];
+    }
+  __syncthreads();
+  if (!node) return;
+  const T(*pb)[64] = sb[lz];
+  const T(*pt)[64] = st[lz - 1];
+#pragma unroll
+  for (int i = 0; i < 3; i++)
+    nd.store(S, y, nN, i,
+             pt[9 + i][tid - 9] + pt[6 + i][tid - 8] + pt[3 + i][tid - 1] + pt[i][tid] + pb[9 + i][tid - 9] +
+                 pb[6 + i][tid - 8] + pb[3 + i][tid - 1] + pb[i][tid]);
+}
+
 // bfloat16 rounding (round to nearest, ties to even) of a finite float
 __device__ __forceinline__ uint32_t bf16_rne(float f) {
   const uint32_t u = __float_as_uint(f);
@@ -1197,11 +1279,201 @@ __global__ __launch_bounds__(64) void k_apply2(KArgs<T> A, const T* __restrict__
   }
 }
 
-static int g_kz3 = 0, g_kz2 = 32;  // g_kz3 = 0: automatic 3D chunk
+// ---------------------------------------------------------------------------------------
+// K of a 2D level as an assembled stencil.  The streaming kernel above takes 40-60 us at any
+// size up to 512^2 with its 32 rows per block, 5 us with one row: a long dependent stream per
+// element on a mostly idle chip.  Stored as nine 2 x 2 blocks per node, the operator is a short
+// independent sum per row, one lane per row: 18 loads, all in flight at once.
+// S[(2 nb + c) n + row]: neighbour nb (x fastest), column component c, so consecutive lanes
+// read consecutive entries.
+//   (K x)_n = sum_{nb != n} K_nb (x_nb - x_n) + R x_n,  R = sum_nb K_nb
+// Summed as differences because K annihilates translations: the plain sum would cancel large
+// entries on smooth vectors and lose what the element form (which takes differences first)
+// keeps (error against 64 bits, FP32: 8e-8 on smooth and 5e-8 on random vectors at 64^2, element
+// kernel 1.2e-7 and 7e-8).  R (in the place of the node's own block) is non-zero only next to
+// Dirichlet dofs, whose columns are zero and whose rows are identity rows.  Entries of
+// neighbours outside the grid are zero.
+// Measured per apply, stencil against the element kernel at its best chunk (us, FP64 / FP32):
+// 64^2 2.8 / 2.6 against 4.9 / 4.8, 256^2 3.9 / 2.8 against 6.3 / 4.6, 384^2 10.7 / 4.5 against
+// 11.0 / 5.2, 512^2 19.6 / 9.4 against 13.5 / 7.3.
+// ---------------------------------------------------------------------------------------
+// Block of node (i, j) and its neighbour at offset o, summed over the elements holding both
+// (fixed order) and their Gauss points, in FP64; the weights as the operator reads them (rounded
+// to FP32 for the FP32 cycle).  The neighbour lies inside the grid.
+template <bool F32>
+__device__ void stencil_block(const Geom& g, const double* __restrict__ W, const int* at, const int* o,
+                              double (&A)[2][2]) {
+  double sc[2];
+#pragma unroll
+  for (int d = 0; d < 2; d++) sc[d] = 2.0 / ((g.hi[d] - g.lo[d]) / g.res[d]);
+#pragma unroll
+  for (int r = 0; r < 2; r++)
+#pragma unroll
+    for (int c = 0; c < 2; c++) A[r][c] = 0.0;
+  for (int el = 0; el < 4; el++) {
+    // element whose corner `1 - bit` per axis is this node, and the neighbour's corner in it
+    int e2[2], cb[2];
+    bool has = true;
+#pragma unroll
+    for (int d = 0; d < 2; d++) {
+      const int bit = (el >> d) & 1;
+      e2[d] = at[d] - 1 + bit;
+      cb[d] = 1 - bit + o[d];
+      has = has && e2[d] >= 0 && e2[d] < g.res[d] && cb[d] >= 0 && cb[d] <= 1;
+    }
+    if (!has) continue;
+    const long e = e2[0] + (long)g.res[0] * e2[1];
+#pragma unroll
+    for (int q = 0; q < 9; q++) {
+      double ga[2], gb[2];
+#pragma unroll
+      for (int d = 0; d < 2; d++) {
+        const double X = gpt(d == 0 ? q / 3 : q % 3);  // the other axis' abscissa
+        const double sa = (el >> d) & 1 ? -1.0 : 1.0, sb = cb[d] ? 1.0 : -1.0;
+        const double ta = (el >> (1 - d)) & 1 ? -1.0 : 1.0, tb = cb[1 - d] ? 1.0 : -1.0;
+        ga[d] = 0.25 * sa * (1.0 + ta * X) * sc[d];
+        gb[d] = 0.25 * sb * (1.0 + tb * X) * sc[d];
+      }
+      const double dot = ga[0] * gb[0] + ga[1] * gb[1];
+      double w = W[(long)q * g.Es + e];
+      if (F32) w = (double)(float)w;
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) A[r][c] += w * ((r == c ? dot : 0.0) + ga[c] * gb[r]);
+    }
+  }
+}
+
+// One thread per (node, neighbour)
+template <typename T>
+__global__ __launch_bounds__(256) void k_stencil_build(Geom g, const double* __restrict__ W,
+                                                       const uint8_t* __restrict__ bc, T* __restrict__ S) {
+  constexpr bool F32 = sizeof(T) == 4;
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= g.N * 9) return;
+  const int nb = (int)(t / g.N);
+  const long n = t - nb * g.N;
+  const int nx = g.nn[0], ny = g.nn[1];
+  const int at[2] = {(int)(n % nx), (int)(n / nx)};
+  const uint8_t mr = bc[n];
+  const auto inside = [&](const int* o) {
+    return at[0] + o[0] >= 0 && at[0] + o[0] < nx && at[1] + o[1] >= 0 && at[1] + o[1] < ny;
+  };
+  double A[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+  if (nb != 4) {
+    const int o[2] = {nb % 3 - 1, nb / 3 - 1};
+    if (inside(o)) {
+      stencil_block<F32>(g, W, at, o, A);
+      const uint8_t mc = bc[n + o[0] + (long)nx * o[1]];
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+          if (((mr >> r) & 1) || ((mc >> c) & 1)) A[r][c] = 0.0;
+    }
+  } else {
+    // R: minus the sum of the Dirichlet columns' blocks
+    double R[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+    for (int m = 0; m < 9; m++) {
+      const int o[2] = {m % 3 - 1, m / 3 - 1};
+      if (!inside(o)) continue;
+      const uint8_t mc = bc[n + o[0] + (long)nx * o[1]];
+      if (!mc) continue;
+      stencil_block<F32>(g, W, at, o, A);
+#pragma unroll
+      for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+          if ((mc >> c) & 1) R[r][c] -= A[r][c];
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) A[r][c] = ((mr >> r) & 1) ? (r == c ? 1.0 : 0.0) : R[r][c];
+  }
+  const long nd = g.N * 2;
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+#pragma unroll
+    for (int r = 0; r < 2; r++) S[(long)(nb * 2 + c) * nd + n * 2 + r] = (T)A[r][c];
+}
+
+// Largest level held as a stencil: where its entries leave the caches and the element kernel,
+// which reads nine weights per element instead, passes it (figures above).  3D levels keep the
+// element kernels (the stencil has 243 entries per node against 27 weights per element; see
+// k_apply3s).
+bool stencil_level(const Geom& g) { return g.dim == 2 && g.N <= 150000; }
+long stencil_entries(const Geom& g) { return g.N * 36; }
+
+template <typename T>
+void launch_stencil_build(const Geom& g, const double* W, const uint8_t* bc, T* S, hipStream_t s) {
+  hipLaunchKernelGGL(k_stencil_build<T>, nblocks(g.N * 9, 256), 256, 0, s, g, W, bc, S);
+  UWG_HIP(hipGetLastError());
+}
+template void launch_stencil_build<double>(const Geom&, const double*, const uint8_t*, double*, hipStream_t);
+template void launch_stencil_build<float>(const Geom&, const double*, const uint8_t*, float*, hipStream_t);
+
+// y = K x with the epilogues of the element kernels.  A workgroup owns 64 consecutive nodes; the
+// three runs of 66 nodes around them are staged in LDS (zero outside the vector) while the
+// entries load into registers.
+template <typename T, int MODE>
+__global__ __launch_bounds__(128) void k_stencil(int nx, int nd, const T* __restrict__ S, const T* __restrict__ x,
+                                                 T* __restrict__ y, SmoothArgs<T> A) {
+  __shared__ T xs[3][132];
+  const int tid = threadIdx.x;
+  const int base = blockIdx.x * 128, row = base + tid;
+  const bool on = row < nd;
+  const int rr = on ? row : 0;
+  T c[18];
+#pragma unroll
+  for (int q = 0; q < 18; q++) c[q] = S[(size_t)q * nd + rr];
+  T b = 0, dinv = 0, d = 0;
+  if (MODE != APPLY_Y) b = A.b[rr];
+  if (MODE == APPLY_CHEB || MODE == APPLY_CHEB0) dinv = A.dinv[rr];
+  if (MODE == APPLY_CHEB) d = A.d[rr];
+#pragma unroll
+  for (int s = 0; s < 3; s++) {
+    const int first = base + ((s - 1) * nx - 1) * 2;
+    for (int q = tid; q < 132; q += 128) {
+      const int o = first + q;
+      const T v = x[min(max(o, 0), nd - 1)];
+      xs[s][q] = o >= 0 && o < nd ? v : (T)0;
+    }
+  }
+  __syncthreads();
+  if (!on) return;
+  const int l = tid & ~1;  // this node's run position of its x - 1 neighbour
+  T own[2], acc[3];
+#pragma unroll
+  for (int q = 0; q < 2; q++) own[q] = xs[1][l + 2 + q];
+  // one partial sum per run: less rounding than a single running sum
+#pragma unroll
+  for (int s = 0; s < 3; s++) {
+    acc[s] = 0;
+#pragma unroll
+    for (int q = 0; q < 6; q++) acc[s] += c[s * 6 + q] * (s * 3 + q / 2 == 4 ? own[q & 1] : xs[s][l + q] - own[q & 1]);
+  }
+  const T kx = (acc[0] + acc[1]) + acc[2], xn = xs[1][l + 2 + (tid & 1)];
+  if (MODE == APPLY_Y) {
+    y[row] = kx;
+    return;
+  }
+  const T r = b - kx;
+  if (MODE == APPLY_RESIDUAL) {
+    y[row] = r;
+    return;
+  }
+  const T v = MODE == APPLY_CHEB ? A.a * d + A.c * (dinv * r) : A.c * (dinv * r);
+  A.d[row] = v;
+  y[row] = xn + v;
+}
+
+static int g_kz3 = 0, g_kz2 = 0;  // 0: automatic
 void set_apply_chunk(int kz3, int kz2) {
   if (kz3 > 0) g_kz3 = kz3;
   if (kz3 < 0) g_kz3 = 0;
-  if (kz2 > 0) g_kz2 = kz2;
+  if (kz2 > 0) g_kz2 = kz2 == 32 ? 0 : kz2;
 }
 
 // compute units of the current device (cached per device)
@@ -1238,9 +1510,31 @@ static int auto_kz3(long tiles, int rz) {
   return best;
 }
 
+// Element levels evaluated side by side by k_apply3s, 0 for the streaming kernels.  More levels
+// per workgroup waste fewer halo evaluations, fewer give more workgroups; the lines lie where
+// the waves fill the SIMDs about once (KL 2 and 3) and, at KL 4, where the streaming kernel's
+// longer runs catch up.  Measured (us, bf16-weight FP32 / FP64; KL 2, 3, 4, streaming):
+// 16^3 4.9, 5.4, 5.8, 15.6 / 6.3, 6.8, 6.8, 26; 32^3 7.5, 6.9, 7.4, 11.2 / 10.8, 10.5, 10.6, 16.8;
+// 40^3 9.1, 8.2, 7.7, 12.3 / 19.7, 15.4, 11.7, 18.8; 48^3 13.9, 12.2, 12.5, 14.2 / 28, 24, 21, 29;
+// 64^3 31, 25, 23, 22 / 66, 58, 47, 47.
+static int small_levels(const Geom& g) {
+  const long tiles = (long)((g.res[0] + 7) / 7) * ((g.res[1] + 7) / 7), cus = device_cus();
+  const auto waves = [&](int kl) { return tiles * ((g.res[2] + kl - 1) / (kl - 1)) * kl; };
+  if (waves(2) <= 2 * cus) return 2;
+  if (waves(3) <= 6 * cus) return 3;
+  return waves(4) <= 16 * cus ? 4 : 0;
+}
+
 template <typename T, int MODE>
 static void launch_apply_mode(const Geom& g, const T* W, const T* x, T* y, const uint8_t* bc, const SmoothArgs<T>& S,
-                              hipStream_t s, const uint32_t* Wbf) {
+                              hipStream_t s, const uint32_t* Wbf, const T* St) {
+  // a chunk that was set explicitly addresses the element kernel
+  if (St && g_kz2 == 0) {
+    const int nd = (int)(g.N * 2);
+    hipLaunchKernelGGL((k_stencil<T, MODE>), nblocks(nd, 128), 128, 0, s, g.nn[0], nd, St, x, y, S);
+    UWG_HIP(hipGetLastError());
+    return;
+  }
   KArgs<T> A{};
   A.rx = g.res[0];
   A.ry = g.res[1];
@@ -1254,6 +1548,30 @@ static void launch_apply_mode(const Geom& g, const T* W, const T* x, T* y, const
   if (g.dim == 3) {
     if (27.0 * g.Es * sizeof(T) >= 4294967296.0 || 3.0 * g.N * sizeof(T) >= 4294967296.0)
       throw std::runtime_error("3D K apply: weight planes and node vectors must stay below 4 GiB");
+    const int kl = g_kz3 > 0 ? 0 : small_levels(g);
+    if (kl) {
+      A.ntx = (g.res[0] + 1 + 6) / 7;
+      A.nty = (g.res[1] + 1 + 6) / 7;
+      const unsigned nwg = (unsigned)(A.ntx * A.nty * ((g.res[2] + kl - 1) / (kl - 1)));
+      const auto go = [&](auto n) {
+        constexpr int KL = decltype(n)::value;
+        if constexpr (sizeof(T) == 4) {
+          if (Wbf)
+            hipLaunchKernelGGL((k_apply3s<T, MODE, true, KL>), nwg, 64 * KL, 0, s, A, (const void*)Wbf, x, y, bc, S);
+          else
+            hipLaunchKernelGGL((k_apply3s<T, MODE, false, KL>), nwg, 64 * KL, 0, s, A, (const void*)W, x, y, bc, S);
+        } else
+          hipLaunchKernelGGL((k_apply3s<T, MODE, false, KL>), nwg, 64 * KL, 0, s, A, (const void*)W, x, y, bc, S);
+      };
+      if (kl == 2)
+        go(std::integral_constant<int, 2>());
+      else if (kl == 3)
+        go(std::integral_constant<int, 3>());
+      else
+        go(std::integral_constant<int, 4>());
+      UWG_HIP(hipGetLastError());
+      return;
+    }
     A.ntx = (g.res[0] + 1 + 14) / 15;
     A.nty = (g.res[1] + 1 + 14) / 15;
     const long tiles = (long)A.ntx * A.nty;
@@ -1269,7 +1587,9 @@ static void launch_apply_mode(const Geom& g, const T* W, const T* x, T* y, const
   } else {
     if (2.0 * g.N * sizeof(T) >= 4294967296.0)
       throw std::runtime_error("2D K apply: node vectors must stay below 4 GiB");
-    A.KZ = g_kz2;
+    // a block streams KZ + 1 rows; as many blocks as fill the chip with a few waves per SIMD
+    const int cols = (g.res[0] + 1 + 62) / 63;
+    A.KZ = g_kz2 > 0 ? g_kz2 : std::max(1, std::min(32, (int)((long)cols * (g.res[1] + 1) / (16L * device_cus()))));
     dim3 grid((g.res[0] + 1 + 62) / 63, (g.res[1] + 1 + A.KZ - 1) / A.KZ);
     hipLaunchKernelGGL((k_apply2<T, MODE>), grid, 64, 0, s, A, W, x, y, bc, S);
   }
@@ -1278,31 +1598,31 @@ static void launch_apply_mode(const Geom& g, const T* W, const T* x, T* y, const
 
 template <typename T>
 void launch_apply_K(const Geom& g, const T* W, const T* x, T* y, const uint8_t* bc, hipStream_t s,
-                    const uint32_t* Wbf) {
-  launch_apply_mode<T, APPLY_Y>(g, W, x, y, bc, SmoothArgs<T>(), s, Wbf);
+                    const uint32_t* Wbf, const T* St) {
+  launch_apply_mode<T, APPLY_Y>(g, W, x, y, bc, SmoothArgs<T>(), s, Wbf, St);
 }
 template void launch_apply_K<double>(const Geom&, const double*, const double*, double*, const uint8_t*, hipStream_t,
-                                     const uint32_t*);
+                                     const uint32_t*, const double*);
 template void launch_apply_K<float>(const Geom&, const float*, const float*, float*, const uint8_t*, hipStream_t,
-                                    const uint32_t*);
+                                    const uint32_t*, const float*);
 
 // r = b - K x
 template <typename T>
 void launch_residual_K(const Geom& g, const T* W, const T* x, const T* b, T* r, const uint8_t* bc, hipStream_t s,
-                       const uint32_t* Wbf) {
+                       const uint32_t* Wbf, const T* St) {
   SmoothArgs<T> S;
   S.b = b;
-  launch_apply_mode<T, APPLY_RESIDUAL>(g, W, x, r, bc, S, s, Wbf);
+  launch_apply_mode<T, APPLY_RESIDUAL>(g, W, x, r, bc, S, s, Wbf, St);
 }
 template void launch_residual_K<double>(const Geom&, const double*, const double*, const double*, double*,
-                                        const uint8_t*, hipStream_t, const uint32_t*);
+                                        const uint8_t*, hipStream_t, const uint32_t*, const double*);
 template void launch_residual_K<float>(const Geom&, const float*, const float*, const float*, float*, const uint8_t*,
-                                       hipStream_t, const uint32_t*);
+                                       hipStream_t, const uint32_t*, const float*);
 
 // one Chebyshev step: r = b - K x; d = a d + c dinv r (a d dropped when first); xn = x + d
 template <typename T>
 void launch_cheb_step_K(const Geom& g, const T* W, const T* x, T* xn, const T* b, const T* dinv, T* d, T a, T c,
-                        bool first, const uint8_t* bc, hipStream_t s, const uint32_t* Wbf) {
+                        bool first, const uint8_t* bc, hipStream_t s, const uint32_t* Wbf, const T* St) {
   SmoothArgs<T> S;
   S.b = b;
   S.dinv = dinv;
@@ -1310,15 +1630,16 @@ void launch_cheb_step_K(const Geom& g, const T* W, const T* x, T* xn, const T* b
   S.a = a;
   S.c = c;
   if (first)
-    launch_apply_mode<T, APPLY_CHEB0>(g, W, x, xn, bc, S, s, Wbf);
+    launch_apply_mode<T, APPLY_CHEB0>(g, W, x, xn, bc, S, s, Wbf, St);
   else
-    launch_apply_mode<T, APPLY_CHEB>(g, W, x, xn, bc, S, s, Wbf);
+    launch_apply_mode<T, APPLY_CHEB>(g, W, x, xn, bc, S, s, Wbf, St);
 }
 template void launch_cheb_step_K<double>(const Geom&, const double*, const double*, double*, const double*,
                                          const double*, double*, double, double, bool, const uint8_t*, hipStream_t,
-                                         const uint32_t*);
+                                         const uint32_t*, const double*);
 template void launch_cheb_step_K<float>(const Geom&, const float*, const float*, float*, const float*, const float*,
-                                        float*, float, float, bool, const uint8_t*, hipStream_t, const uint32_t*);
+                                        float*, float, float, bool, const uint8_t*, hipStream_t, const uint32_t*,
+                                        const float*);
 
 // ---------------------------------------------------------------------------------------
 // G p (node gather) and G^T u (element gather); G_e constant on a regular mesh

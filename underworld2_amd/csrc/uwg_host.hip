@@ -105,6 +105,8 @@ struct Level {
   double* W = nullptr;
   float* W32 = nullptr;
   uint32_t* Wbf = nullptr;  // 3D FP32 cycle: the weights as bfloat16 pairs [14][Es] (when enabled)
+  double* S = nullptr;      // small 2D levels: K as an assembled stencil
+  float* S32 = nullptr;
   uint8_t* bc = nullptr;
   double* dinv = nullptr;
   float* dinv32 = nullptr;
@@ -885,7 +887,7 @@ static void build_levels(uwg_stokes* st, int levels_req) {
   double* W0 = st->L.empty() ? nullptr : st->L[0].W;
   for (size_t l = 0; l < st->L.size(); l++) {
     Level& A = st->L[l];
-    for (void* p : {(void*)A.W, (void*)A.W32, (void*)A.Wbf, (void*)A.bc, (void*)A.dinv, (void*)A.dinv32, (void*)A.x,
+    for (void* p : {(void*)A.W, (void*)A.W32, (void*)A.Wbf, (void*)A.S, (void*)A.S32, (void*)A.bc, (void*)A.dinv, (void*)A.dinv32, (void*)A.x,
                     (void*)A.b, (void*)A.r, (void*)A.d, (void*)A.x32, (void*)A.b32, (void*)A.r32, (void*)A.d32})
       if (p != (void*)st->bc0 && p != (void*)W0) dfree(p);
   }
@@ -922,6 +924,7 @@ static void build_levels(uwg_stokes* st, int levels_req) {
     A.r = dalloc<double>(A.n());
     A.d = dalloc<double>(A.n());
     A.bc = l > 0 ? dalloc<uint8_t>(A.g.N) : st->bc0;
+    if (stencil_level(A.g)) A.S = dalloc<double>(stencil_entries(A.g));
   }
   st->hierarchy_built = true;
   st->fp32_ready = false;
@@ -959,6 +962,10 @@ static void ensure_fp32(uwg_stokes* st) {
     } else if (A.Wbf) {
       dfree(A.Wbf);
       A.Wbf = nullptr;
+    }
+    if (A.S) {
+      if (!A.S32) A.S32 = dalloc<float>(stencil_entries(A.g));
+      launch_stencil_build<float>(A.g, A.W, A.bc, A.S32, 0);
     }
   }
   st->fp32_bf16 = g_cycle_bf16;
@@ -1102,7 +1109,7 @@ static void estimate_lmax(uwg_stokes* st, Level& A) {
   const double* ptr[1] = {A.d};
   UWG_HIP(hipMemcpy(st->dptrs, ptr, sizeof(double*), hipMemcpyHostToDevice));
   for (int it = 0; it < 12; it++) {
-    launch_apply_K<double>(A.g, A.W, A.x, A.r, A.bc, 0);
+    launch_apply_K<double>(A.g, A.W, A.x, A.r, A.bc, 0, nullptr, A.S);
     vk_xmy_scale<double>(n, A.dinv, A.r, A.d, 0);
     vk_multi_dot(n, 1, A.d, st->dptrs, st->red_partial, st->red_out, 0);
     if (it < 11) vk_scale_inv_sqrt(n, st->red_out, A.d, A.x, 0);
@@ -1162,7 +1169,10 @@ static void setup_hierarchy(uwg_stokes* st) {
   // coarse Dirichlet masks: a coarse dof is constrained when the coincident fine dof is
   // (nested walls); derived from level 0's mask by injection
   for (size_t l = 1; l < st->L.size(); l++) launch_inject_bc(st->L[l - 1].g, st->L[l].g, st->L[l - 1].bc, st->L[l].bc, 0);
-  for (auto& A : st->L) launch_diag(A.g, A.W, A.bc, A.dinv, 0);
+  for (auto& A : st->L) {
+    launch_diag(A.g, A.W, A.bc, A.dinv, 0);
+    if (A.S) launch_stencil_build<double>(A.g, A.W, A.bc, A.S, 0);
+  }
   for (auto& A : st->L) estimate_lmax(st, A);
   build_coarse(st);
   st->fp32_ready = false;
@@ -1182,6 +1192,7 @@ template <typename T> struct LV;
 template <> struct LV<double> {
   static double* W(Level& A) { return A.W; }
   static const uint32_t* Wbf(Level&) { return nullptr; }
+  static const double* S(Level& A) { return A.S; }
   static double* dinv(Level& A) { return A.dinv; }
   static double* x(Level& A) { return A.x; }
   static double* b(Level& A) { return A.b; }
@@ -1191,6 +1202,7 @@ template <> struct LV<double> {
 template <> struct LV<float> {
   static float* W(Level& A) { return A.W32; }
   static const uint32_t* Wbf(Level& A) { return A.Wbf; }
+  static const float* S(Level& A) { return A.S32; }
   static float* dinv(Level& A) { return A.dinv32; }
   static float* x(Level& A) { return A.x32; }
   static float* b(Level& A) { return A.b32; }
@@ -1227,11 +1239,11 @@ static void chebyshev(Level& A, const T* b, T* x, int degree, bool zero_guess) {
     T* nxt = (cur == x) ? tmp : x;
     if (!zero_guess && k == 0) {
       launch_cheb_step_K<T>(A.g, LV<T>::W(A), cur, nxt, b, dinv, d, (T)0, (T)(1.0 / theta), true, A.bc, 0,
-                            LV<T>::Wbf(A));
+                            LV<T>::Wbf(A), LV<T>::S(A));
     } else {
       const double rho_new = 1.0 / (2.0 * sigma - rho);
       launch_cheb_step_K<T>(A.g, LV<T>::W(A), cur, nxt, b, dinv, d, (T)(rho_new * rho), (T)(2.0 * rho_new / delta),
-                            false, A.bc, 0, LV<T>::Wbf(A));
+                            false, A.bc, 0, LV<T>::Wbf(A), LV<T>::S(A));
       rho = rho_new;
     }
     cur = nxt;
@@ -1278,7 +1290,7 @@ static void vcycle(uwg_stokes* st, int l, const T* b, T* x) {
   Level& C = st->L[l + 1];
   chebyshev<T>(A, b, x, g_smooth_degree, true);
   T* r = LV<T>::r(A);
-  launch_residual_K<T>(A.g, LV<T>::W(A), x, b, r, A.bc, 0, LV<T>::Wbf(A));
+  launch_residual_K<T>(A.g, LV<T>::W(A), x, b, r, A.bc, 0, LV<T>::Wbf(A), LV<T>::S(A));
   launch_restrict2<T>(A.g, C.g, r, LV<T>::b(C), C.bc, A.bc, 0);
   const bool capture = st->capture_level == l + 1 && st->captured < st->capture_max &&
                        (st->capture_seen++ % st->capture_every) == 0;
@@ -1299,7 +1311,7 @@ static void vcycle(uwg_stokes* st, int l, const T* b, T* x) {
     if (capture && st->capture_kind == 1) {
       // residual the coarse cycle leaves behind: its error K_C^{-1} r is what an additive
       // correction has to supply
-      launch_residual_K<T>(C.g, LV<T>::W(C), LV<T>::x(C), LV<T>::b(C), LV<T>::r(C), C.bc, 0, LV<T>::Wbf(C));
+      launch_residual_K<T>(C.g, LV<T>::W(C), LV<T>::x(C), LV<T>::b(C), LV<T>::r(C), C.bc, 0, LV<T>::Wbf(C), LV<T>::S(C));
       capture_vector<T>(st, C.n(), LV<T>::r(C));
     }
     if constexpr (std::is_same<T, float>::value) {
@@ -1344,13 +1356,19 @@ template <> struct Q2V<float> {
 };
 }  // namespace
 
+// the finest level's stencil where it was built with this mask
+template <typename T>
+static const T* top_stencil(uwg_stokes* st, const uint8_t* bc) {
+  return bc == st->L[0].bc ? LV<T>::S(st->L[0]) : nullptr;
+}
+
 // K on the finest level; bc selects the Dirichlet rows/columns (identity rows)
 template <typename T>
 static void top_K(uwg_stokes* st, const T* x, T* y, const uint8_t* bc) {
   if (st->q2)
     launch_q2_apply<T>(st->g, Q2V<T>::W(*st->q2), x, y, bc, 0, Q2V<T>::D(*st->q2));
   else
-    launch_apply_K<T>(st->g, LV<T>::W(st->L[0]), x, y, bc, 0);
+    launch_apply_K<T>(st->g, LV<T>::W(st->L[0]), x, y, bc, 0, nullptr, top_stencil<T>(st, bc));
 }
 template <typename T>
 static void top_G(uwg_stokes* st, const T* p, T* y, const uint8_t* bc) {
@@ -1699,7 +1717,7 @@ extern "C" int uwg_stokes_create(uwg_field* vel, uwg_field* p, const unsigned ch
 extern "C" int uwg_stokes_destroy(uwg_stokes* st) {
   if (!st) return 0;
   for (auto& A : st->L)
-    for (void* p : {(void*)A.W, (void*)A.W32, (void*)A.Wbf, (void*)A.bc, (void*)A.dinv, (void*)A.dinv32, (void*)A.x,
+    for (void* p : {(void*)A.W, (void*)A.W32, (void*)A.Wbf, (void*)A.S, (void*)A.S32, (void*)A.bc, (void*)A.dinv, (void*)A.dinv32, (void*)A.x,
                     (void*)A.b, (void*)A.r, (void*)A.d, (void*)A.x32, (void*)A.b32, (void*)A.r32, (void*)A.d32})
       if (p != (void*)st->bc0) dfree(p);
   dfree(st->bc0);
@@ -2486,7 +2504,7 @@ extern "C" int uwg_stokes_apply(uwg_stokes* st, int which, int level, const doub
   UWG_HIP(hipMemcpy(dx, x, sizeof(double) * nin, hipMemcpyHostToDevice));
   if (which == 6) {
     // the multigrid residual kernel (apply with the r = b - K x epilogue), b = x
-    launch_residual_K<double>(A.g, A.W, dx, dx, dy, A.bc, 0);
+    launch_residual_K<double>(A.g, A.W, dx, dx, dy, A.bc, 0, nullptr, A.S);
     UWG_HIP(hipMemcpy(y, dy, sizeof(double) * nout, hipMemcpyDeviceToHost));
     dfree(dx);
     dfree(dy);
@@ -2501,9 +2519,9 @@ extern "C" int uwg_stokes_apply(uwg_stokes* st, int which, int level, const doub
     float* fy = dalloc<float>(nout);
     vk_d2f(nin, 1.0, dx, fx, 0);
     if (which == 7)
-      launch_residual_K<float>(A.g, A.W32, fx, fx, fy, A.bc, 0, A.Wbf);
+      launch_residual_K<float>(A.g, A.W32, fx, fx, fy, A.bc, 0, A.Wbf, A.S32);
     else
-      launch_apply_K<float>(A.g, A.W32, fx, fy, A.bc, 0, which == 4 ? A.Wbf : nullptr);
+      launch_apply_K<float>(A.g, A.W32, fx, fy, A.bc, 0, which == 4 ? A.Wbf : nullptr, A.S32);
     vk_f2d(nout, 1.0, fy, dy, 0);
     UWG_HIP(hipMemcpy(y, dy, sizeof(double) * nout, hipMemcpyDeviceToHost));
     dfree(fx);
@@ -2513,7 +2531,7 @@ extern "C" int uwg_stokes_apply(uwg_stokes* st, int which, int level, const doub
     return 0;
   }
   if (which == 0)
-    launch_apply_K<double>(A.g, A.W, dx, dy, A.bc, 0);
+    launch_apply_K<double>(A.g, A.W, dx, dy, A.bc, 0, nullptr, A.S);
   else if (which == 1)
     launch_apply_G(st->g, st->Ge, dx, st->L[0].bc, dy, 0);
   else if (which == 2)
@@ -2679,14 +2697,14 @@ extern "C" int uwg_stokes_time_apply(uwg_stokes* st, int precision, int level, i
     // 1: the FP32 cycle's apply (bfloat16 weights when the cycle uses them), 2: FP32 weights
     ensure_fp32(st);
     const uint32_t* wb = precision == 1 ? A.Wbf : nullptr;
-    launch_apply_K<float>(A.g, A.W32, A.x32, A.r32, A.bc, 0, wb);
+    launch_apply_K<float>(A.g, A.W32, A.x32, A.r32, A.bc, 0, wb, A.S32);
     UWG_HIP(hipEventRecord(e0, 0));
-    for (int i = 0; i < reps; i++) launch_apply_K<float>(A.g, A.W32, A.x32, A.r32, A.bc, 0, wb);
+    for (int i = 0; i < reps; i++) launch_apply_K<float>(A.g, A.W32, A.x32, A.r32, A.bc, 0, wb, A.S32);
     UWG_HIP(hipEventRecord(e1, 0));
   } else {
-    launch_apply_K<double>(A.g, A.W, A.x, A.r, A.bc, 0);
+    launch_apply_K<double>(A.g, A.W, A.x, A.r, A.bc, 0, nullptr, A.S);
     UWG_HIP(hipEventRecord(e0, 0));
-    for (int i = 0; i < reps; i++) launch_apply_K<double>(A.g, A.W, A.x, A.r, A.bc, 0);
+    for (int i = 0; i < reps; i++) launch_apply_K<double>(A.g, A.W, A.x, A.r, A.bc, 0, nullptr, A.S);
     UWG_HIP(hipEventRecord(e1, 0));
   }
   UWG_HIP(hipEventSynchronize(e1));
@@ -2863,7 +2881,7 @@ extern "C" int uwg_stokes_level_solve(uwg_stokes* st, int level, const double* b
   double* wb = dalloc<double>(n);
   UWG_HIP(hipMemcpy(db, b, sizeof(double) * n, hipMemcpyHostToDevice));
   vk_fill<double>(n, 0.0, dx, 0);
-  OpFn Aop = [&](const double* xx, double* yy) { launch_apply_K<double>(A.g, A.W, xx, yy, A.bc, 0); };
+  OpFn Aop = [&](const double* xx, double* yy) { launch_apply_K<double>(A.g, A.W, xx, yy, A.bc, 0, nullptr, A.S); };
   OpFn Mop = [&](const double* rr, double* zz) {
     vk_copy<double>(n, rr, wb, 0);
     vcycle<double>(st, level, wb, zz);

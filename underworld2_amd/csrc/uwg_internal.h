@@ -96,17 +96,24 @@ void launch_gauss_assemble(const Geom& g, const double* eta_g, const double* for
                            double* approxS, const double* Ge, hipStream_t s);
 void launch_restrict_W(const Geom& fine, const Geom& coarse, const double* Wf, double* Wc, hipStream_t s);
 void launch_diag(const Geom& g, const double* W, const uint8_t* bc, double* dinv, hipStream_t s);
+// 2D levels small enough to hold K as an assembled stencil, and its entries (FP32: from the
+// weights rounded to FP32, as the FP32 applies read them)
+bool stencil_level(const Geom& g);
+long stencil_entries(const Geom& g);
+template <typename T>
+void launch_stencil_build(const Geom& g, const double* W, const uint8_t* bc, T* S, hipStream_t s);
 // K applies.  Wbf (FP32 instance, 3D only): the weights as bfloat16 pairs [14][Es] (see
-// launch_pack_w3_bf16); when given, the apply reads them instead of W.
+// launch_pack_w3_bf16); when given, the apply reads them instead of W.  St: the level's
+// stencil (built with the same bc), which replaces both.
 template <typename T>
 void launch_apply_K(const Geom& g, const T* W, const T* x, T* y, const uint8_t* bc, hipStream_t s,
-                    const uint32_t* Wbf = nullptr);
+                    const uint32_t* Wbf = nullptr, const T* St = nullptr);
 template <typename T>
 void launch_residual_K(const Geom& g, const T* W, const T* x, const T* b, T* r, const uint8_t* bc, hipStream_t s,
-                       const uint32_t* Wbf = nullptr);
+                       const uint32_t* Wbf = nullptr, const T* St = nullptr);
 template <typename T>
 void launch_cheb_step_K(const Geom& g, const T* W, const T* x, T* xn, const T* b, const T* dinv, T* d, T a, T c,
-                        bool first, const uint8_t* bc, hipStream_t s, const uint32_t* Wbf = nullptr);
+                        bool first, const uint8_t* bc, hipStream_t s, const uint32_t* Wbf = nullptr, const T* St = nullptr);
 // FP64 weights [27][Es] -> bfloat16 pairs [14][Es]: word p = bf16(W_2p) | bf16(W_2p+1) << 16
 void launch_pack_w3_bf16(long Es, const double* W, uint32_t* Wb, hipStream_t s);
 template <typename T>
