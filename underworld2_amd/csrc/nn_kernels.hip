@@ -16,6 +16,7 @@
 // x fastest).  Grids here are at most 33^3 nodes, where direct convolution with weights
 // broadcast from the scalar cache is latency-bound rather than FLOP-bound, so MFMA tiles
 // would not pay.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
@@ -78,7 +79,11 @@ __global__ void k_conv_fwd(int B, int Ci, int Co, Grid3 g, const float* __restri
 // values per input channel overflowed the scalar registers: about 4,400 instructions per
 // channel for 432 FMAs.  The FMA order (input channel, then taps) is unchanged, so the sums are
 // the same bit for bit.
-template <int COB>
+// BWD: the input gradient of the same convolution, din[ci][p] = sum_co sum_tap w[co][ci][tap]
+// dout[co][p - off(tap)]: in is dout (Ci = its channels), out is din (Co = its channels).  Its own
+// kernel with four channels per thread and scalar weight loads took 405 us for 16 x 16 channels at
+// 4 x 48^3, this 150 us.
+template <int COB, bool BWD = false>
 __global__ __launch_bounds__(256) void k_conv_fwd_blk(int B, int Ci, int Co, Grid3 g, const float* __restrict__ in,
                                                       const float* __restrict__ w, const float* __restrict__ bias,
                                                       float* __restrict__ out, int relu) {
@@ -93,13 +98,13 @@ __global__ __launch_bounds__(256) void k_conv_fwd_blk(int B, int Ci, int Co, Gri
   const int i = (int)(p % g.nx), j = (int)((p / g.nx) % g.ny), k = (int)(p / ((long)g.nx * g.ny));
   float acc[COB];
 #pragma unroll
-  for (int c = 0; c < COB; c++) acc[c] = bias[co0 + c];
+  for (int c = 0; c < COB; c++) acc[c] = BWD ? 0.0f : bias[co0 + c];
   const long cs = (long)Ci * 27;
   for (int ci = 0; ci < Ci; ci++) {
     __syncthreads();  // the previous channel's weights are no longer read
     for (int q = threadIdx.x; q < 27 * COB; q += blockDim.x) {
       const int c = q % COB, tap = q / COB;
-      ws[q] = w[(long)(co0 + c) * cs + ci * 27 + tap];
+      ws[q] = BWD ? w[((long)ci * Co + co0 + c) * 27 + tap] : w[(long)(co0 + c) * cs + ci * 27 + tap];
     }
     __syncthreads();
     if (!active) continue;
@@ -108,15 +113,15 @@ __global__ __launch_bounds__(256) void k_conv_fwd_blk(int B, int Ci, int Co, Gri
     // the kernel needs 496 registers per lane (one wave per SIMD)
 #pragma unroll 1
     for (int dz = -1; dz <= 1; dz++) {
-      const int kk = k + dz;
+      const int kk = BWD ? k - dz : k + dz;
       const bool okz = kk >= 0 && kk < g.nz;
 #pragma unroll 1
       for (int dy = -1; dy <= 1; dy++) {
-        const int jj = j + dy;
+        const int jj = BWD ? j - dy : j + dy;
         const bool oky = okz && jj >= 0 && jj < g.ny;
 #pragma unroll
         for (int dx = -1; dx <= 1; dx++) {
-          const int ii = i + dx;
+          const int ii = BWD ? i - dx : i + dx;
           const float v = (oky && ii >= 0 && ii < g.nx) ? src[ii + (long)g.nx * (jj + (long)g.ny * kk)] : 0.0f;
           const int tap = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
 #pragma unroll
@@ -195,47 +200,6 @@ __global__ __launch_bounds__(256) void k_conv_fwd_ks(int B, int Ci, int Co, Grid
   }
 }
 
-// Channel-blocked input gradient: each thread produces CIB input channels of one node.
-template <int CIB>
-__global__ __launch_bounds__(256) void k_conv_bwd_data_blk(int B, int Ci, int Co, Grid3 g,
-                                                           const float* __restrict__ dout,
-                                                           const float* __restrict__ w, float* __restrict__ din) {
-  const long N = g.N();
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int ci0 = blockIdx.y * CIB;
-  if (t >= (long)B * N) return;
-  const long p = t % N;
-  const int b = (int)(t / N);
-  const int i = (int)(p % g.nx), j = (int)((p / g.nx) % g.ny), k = (int)(p / ((long)g.nx * g.ny));
-  float acc[CIB];
-#pragma unroll
-  for (int c = 0; c < CIB; c++) acc[c] = 0.0f;
-  for (int co = 0; co < Co; co++) {
-    const float* src = dout + ((long)b * Co + co) * N;
-    const float* wc = w + ((long)co * Ci + ci0) * 27;
-#pragma unroll
-    for (int dz = -1; dz <= 1; dz++) {
-      const int kk = k - dz;
-      const bool okz = kk >= 0 && kk < g.nz;
-#pragma unroll
-      for (int dy = -1; dy <= 1; dy++) {
-        const int jj = j - dy;
-        const bool oky = okz && jj >= 0 && jj < g.ny;
-#pragma unroll
-        for (int dx = -1; dx <= 1; dx++) {
-          const int ii = i - dx;
-          const float v = (oky && ii >= 0 && ii < g.nx) ? src[ii + (long)g.nx * (jj + (long)g.ny * kk)] : 0.0f;
-          const int tap = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
-#pragma unroll
-          for (int c = 0; c < CIB; c++) acc[c] += wc[c * 27 + tap] * v;
-        }
-      }
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < CIB; c++) din[((long)b * Ci + ci0 + c) * N + p] = acc[c];
-}
-
 // din[b][ci][p] = sum_co sum_tap w[co][ci][tap] dout[b][co][p - off(tap)]
 __global__ void k_conv_bwd_data(int B, int Ci, int Co, Grid3 g, const float* __restrict__ dout,
                                 const float* __restrict__ w, float* __restrict__ din) {
@@ -270,65 +234,184 @@ __global__ void k_conv_bwd_data(int B, int Ci, int Co, Grid3 g, const float* __r
   din[t] = acc;
 }
 
-// dw[co][ci][tap] = sum_b sum_p dout[b][co][p] in[b][ci][p + off(tap)] ; one block per (co, ci)
-__global__ __launch_bounds__(256) void k_conv_bwd_w(int B, int Ci, int Co, Grid3 g, const float* __restrict__ dout,
-                                                    const float* __restrict__ in, float* __restrict__ dw) {
-  __shared__ float sm[27][256];
-  const int co = blockIdx.x / Ci, ci = blockIdx.x % Ci;
-  const long N = g.N();
-  float acc[27];
+// Sums of NV per-thread values over a workgroup of 256 into res, by halves (128, 64, ... 1): sixteen
+// values at a time cross the waves through LDS, then each wave finishes four of them.
+template <int NV>
+__device__ __forceinline__ void block_sums(const float (&v)[NV], float* res) {
+  __shared__ float sm[16][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-  for (int q = 0; q < 27; q++) acc[q] = 0.0f;
-  for (long t = threadIdx.x; t < (long)B * N; t += 256) {
-    const int b = (int)(t / N);
-    const long p = t % N;
-    const float go = dout[((long)b * Co + co) * N + p];
-    if (go == 0.0f) continue;
-    const float* src = in + ((long)b * Ci + ci) * N;
-    const int i = (int)(p % g.nx), j = (int)((p / g.nx) % g.ny), k = (int)(p / ((long)g.nx * g.ny));
+  for (int g = 0; g < NV; g += 16) {
 #pragma unroll
-    for (int dz = -1; dz <= 1; dz++) {
-      int kk = k + dz;
-      bool okz = kk >= 0 && kk < g.nz;
+    for (int q = 0; q < 16; q++)
+      if (g + q < NV) sm[q][threadIdx.x] = v[g + q];
+    __syncthreads();
+    for (int q = wave; q < 16 && g + q < NV; q += 4) {
+      float a = (sm[q][lane] + sm[q][lane + 128]) + (sm[q][lane + 64] + sm[q][lane + 192]);
 #pragma unroll
-      for (int dy = -1; dy <= 1; dy++) {
-        int jj = j + dy;
-        bool oky = okz && jj >= 0 && jj < g.ny;
-#pragma unroll
-        for (int dx = -1; dx <= 1; dx++) {
-          int ii = i + dx;
-          if (oky && ii >= 0 && ii < g.nx)
-            acc[(dz + 1) * 9 + (dy + 1) * 3 + (dx + 1)] += go * src[ii + (long)g.nx * (jj + (long)g.ny * kk)];
-        }
-      }
+      for (int s = 32; s > 0; s >>= 1) a += __shfl_xor(a, s);
+      if (lane == 0) res[g + q] = a;
     }
-  }
-#pragma unroll
-  for (int q = 0; q < 27; q++) sm[q][threadIdx.x] = acc[q];
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s)
-#pragma unroll
-      for (int q = 0; q < 27; q++) sm[q][threadIdx.x] += sm[q][threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x < 27) dw[((long)co * Ci + ci) * 27 + threadIdx.x] = sm[threadIdx.x][0];
 }
 
-// db[co] = sum_b sum_p dout[b][co][p]
-__global__ __launch_bounds__(256) void k_bias_grad(int B, int Co, long N, const float* __restrict__ dout,
-                                                   float* __restrict__ db) {
-  __shared__ float sm[256];
-  const int co = blockIdx.x;
-  float a = 0.0f;
-  for (long t = threadIdx.x; t < (long)B * N; t += 256) a += dout[((long)(t / N) * Co + co) * N + t % N];
-  sm[threadIdx.x] = a;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] += sm[threadIdx.x + s];
-    __syncthreads();
+// Weight and bias gradients of a 3x3x3 convolution,
+//   dw[co][ci][tap] = sum_b sum_p dout[b][co][p] in[b][ci][p + off(tap)],  db[co] = sum dout,
+// as partial sums part[chunk][Co Ci 27 + Co] of chunks of points, added up in FP64 by k_sum_parts
+// in chunk order (deterministic).  A thread holds COB x 27 sums, so each of the 27 neighbours it
+// loads serves COB products, and the points are split so that every size fills the chip: one
+// workgroup per (co, ci) pair over all points took 6.0 ms for 16 x 16 channels at 4 x 48^3, this
+// 0.2 ms (bound by the loads of the neighbours, which hit the caches).
+template <int COB>
+__global__ __launch_bounds__(256) void k_wgrad3(int B, int Ci, int Co, Grid3 g, const float* __restrict__ dout,
+                                                const float* __restrict__ in, int per, float* __restrict__ part) {
+  constexpr int NV = COB * 28;  // the last of 28: the bias
+  __shared__ float sum[NV];
+  const int ci = blockIdx.y, co0 = blockIdx.z * COB;
+  const int N = (int)g.N(), nx = g.nx, ny = g.ny, nz = g.nz, nxy = nx * ny;
+  const int T = B * N, t0 = blockIdx.x * per, t1 = min(t0 + per, T);
+  float acc[NV];
+#pragma unroll
+  for (int q = 0; q < NV; q++) acc[q] = 0.0f;
+  for (int t = t0 + (int)threadIdx.x; t < t1; t += 256) {
+    const int b = t / N, p = t - b * N, k = p / nxy, r = p - k * nxy, j = r / nx, i = r - j * nx;
+    float go[COB];
+#pragma unroll
+    for (int c = 0; c < COB; c++) go[c] = dout[(size_t)(b * Co + min(co0 + c, Co - 1)) * N + p];
+    const float* src = in + (size_t)(b * Ci + ci) * N;
+    const int im = max(i - 1, 0), ip = min(i + 1, nx - 1);
+#pragma unroll
+    for (int s = 0; s < 9; s++) {
+      const int jj = j + s % 3 - 1, kk = k + s / 3 - 1;
+      const bool row = jj >= 0 && jj < ny && kk >= 0 && kk < nz;
+      const float* line = src + (row ? nx * jj + nxy * kk : 0);
+      const float x0 = line[im], x1 = line[i], x2 = line[ip];
+      const float v[3] = {row && i > 0 ? x0 : 0.0f, row ? x1 : 0.0f, row && i < nx - 1 ? x2 : 0.0f};
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int c = 0; c < COB; c++) acc[c * 28 + s * 3 + d] += go[c] * v[d];
+    }
+#pragma unroll
+    for (int c = 0; c < COB; c++) acc[c * 28 + 27] += go[c];
   }
-  if (threadIdx.x == 0) db[co] = sm[0];
+  block_sums<NV>(acc, sum);
+  const long nw = (long)Co * Ci * 27;
+  float* out = part + (long)blockIdx.x * (nw + Co);
+  for (int q = threadIdx.x; q < NV; q += 256) {
+    const int co = co0 + q / 28, tap = q % 28;
+    const float v = sum[q];
+    if (co >= Co) continue;
+    if (tap < 27)
+      out[((long)co * Ci + ci) * 27 + tap] = v;
+    else if (ci == 0)
+      out[nw + co] = v;
+  }
+}
+
+// The same for a 1x1x1 convolution with 27 outputs: part[chunk][27 Ci + 27], 9 outputs x CB inputs
+// per thread
+template <int CB>
+__global__ __launch_bounds__(256) void k_wgrad1(int B, int Ci, long N, const float* __restrict__ gout,
+                                                const float* __restrict__ in, int per, float* __restrict__ part) {
+  constexpr int NV = 9 * (CB + 1);
+  __shared__ float sum[NV];
+  const int c0 = blockIdx.y * CB, o0 = blockIdx.z * 9;
+  const int n = (int)N, T = B * n, t0 = blockIdx.x * per, t1 = min(t0 + per, T);
+  float acc[NV];
+#pragma unroll
+  for (int q = 0; q < NV; q++) acc[q] = 0.0f;
+  for (int t = t0 + (int)threadIdx.x; t < t1; t += 256) {
+    const int b = t / n, p = t - b * n;
+    float x[CB];
+#pragma unroll
+    for (int c = 0; c < CB; c++) x[c] = in[(size_t)(b * Ci + min(c0 + c, Ci - 1)) * n + p];
+#pragma unroll
+    for (int o = 0; o < 9; o++) {
+      const float go = gout[(size_t)(b * 27 + o0 + o) * n + p];
+#pragma unroll
+      for (int c = 0; c < CB; c++) acc[o * (CB + 1) + c] += go * x[c];
+      acc[o * (CB + 1) + CB] += go;
+    }
+  }
+  block_sums<NV>(acc, sum);
+  float* out = part + (long)blockIdx.x * (27L * Ci + 27);
+  for (int q = threadIdx.x; q < NV; q += 256) {
+    const int o = o0 + q / (CB + 1), c = q % (CB + 1);
+    const float v = sum[q];
+    if (c < CB && c0 + c < Ci)
+      out[(long)o * Ci + c0 + c] = v;
+    else if (c == CB && c0 == 0)
+      out[27L * Ci + o] = v;
+  }
+}
+
+__global__ void k_sum_parts(long n, int nchunk, const float* __restrict__ part, float* __restrict__ out) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  double a = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < nchunk; c++) a += (double)part[c * n + t];
+  out[t] = (float)a;
+}
+
+// Chunks of T points for `pairs` workgroups per chunk: about 2,048 workgroups (eight per CU), each
+// thread with at least eight points so that the closing sums stay a small part.  Up to kWgradOne
+// points (32 per thread) one workgroup per output pair is as fast, without partial sums.
+constexpr long kWgradOne = 8192;
+constexpr int kWgradCo = 4, kWgradC = 4;
+static int wgrad_chunks(long T, long pairs) {
+  if (T <= kWgradOne) return 1;
+  const long c = std::min((2048 + pairs - 1) / pairs, (T + 2047) / 2048);
+  return (int)std::max(1L, c);
+}
+static int wgrad3_chunks(long T, int ci, int co) { return wgrad_chunks(T, (long)ci * ((co + kWgradCo - 1) / kWgradCo)); }
+static int wgrad1_chunks(long T, int ci) { return wgrad_chunks(T, 3L * ((ci + kWgradC - 1) / kWgradC)); }
+static long wgrad3_part(long T, int ci, int co) { return wgrad3_chunks(T, ci, co) * ((long)co * ci * 27 + co); }
+static long wgrad1_part(long T, int ci) { return wgrad1_chunks(T, ci) * (27L * ci + 27); }
+
+// grads: dw[co][ci][27] followed by db[co]; part: wgrad3_part floats
+static void wgrad3(int B, int ci, int co, Grid3 g, const float* dout, const float* in, float* part, float* grads,
+                   hipStream_t s) {
+  const long T = (long)B * g.N(), n = (long)co * ci * 27 + co;
+  if (T >= 2147483647L) throw std::runtime_error("convolution gradient: batch too large");
+  const int nc = wgrad3_chunks(T, ci, co), per = (int)((T + nc - 1) / nc);
+  if (T <= kWgradOne) {
+    hipLaunchKernelGGL(k_wgrad3<1>, dim3(1, ci, co), 256, 0, s, B, ci, co, g, dout, in, per, grads);
+    return;
+  }
+  hipLaunchKernelGGL(k_wgrad3<kWgradCo>, dim3(nc, ci, (co + kWgradCo - 1) / kWgradCo), 256, 0, s, B, ci, co, g, dout,
+                     in, per, part);
+  hipLaunchKernelGGL(k_sum_parts, (unsigned)((n + 255) / 256), 256, 0, s, n, nc, part, grads);
+}
+// 27 outputs; grads: dw[27][ci] followed by db[27]
+static void wgrad1(int B, int ci, long N, const float* gout, const float* in, float* part, float* grads,
+                   hipStream_t s) {
+  const long T = (long)B * N, n = 27L * ci + 27;
+  if (T >= 2147483647L) throw std::runtime_error("convolution gradient: batch too large");
+  const int nc = wgrad1_chunks(T, ci), per = (int)((T + nc - 1) / nc);
+  if (T <= kWgradOne) {
+    hipLaunchKernelGGL(k_wgrad1<1>, dim3(1, ci, 3), 256, 0, s, B, ci, N, gout, in, per, grads);
+    return;
+  }
+  hipLaunchKernelGGL(k_wgrad1<kWgradC>, dim3(nc, (ci + kWgradC - 1) / kWgradC, 3), 256, 0, s, B, ci, N, gout, in, per,
+                     part);
+  hipLaunchKernelGGL(k_sum_parts, (unsigned)((n + 255) / 256), 256, 0, s, n, nc, part, grads);
+}
+
+// input gradient of a 3x3x3 convolution with ci input and co output channels
+static void conv3_bwd_data(int B, int ci, int co, Grid3 g, const float* dout, const float* w, float* din,
+                           hipStream_t s) {
+  const long nb = (long)B * g.N();
+  const unsigned nblk = (unsigned)((nb + 255) / 256);
+  const float* none = nullptr;
+  if (ci % 16 == 0 && nb > 65536)
+    hipLaunchKernelGGL((k_conv_fwd_blk<16, true>), dim3(nblk, ci / 16), 256, 0, s, B, co, ci, g, dout, w, none, din, 0);
+  else if (ci % 4 == 0)  // small grids: more workgroups
+    hipLaunchKernelGGL((k_conv_fwd_blk<4, true>), dim3(nblk, ci / 4), 256, 0, s, B, co, ci, g, dout, w, none, din, 0);
+  else
+    hipLaunchKernelGGL(k_conv_bwd_data, (unsigned)((nb * ci + 255) / 256), 256, 0, s, B, ci, co, g, dout, w, din);
 }
 
 // dy *= (y > 0)
@@ -495,6 +578,7 @@ struct NNModel {
   std::vector<float*> pool, gpool;  // per level (l >= 1): R(e_{l-1})/8
   std::vector<float*> sum, gsum;    // per level (l <= D-2): P(up) + e_l
   float *xin = nullptr, *y = nullptr, *gy = nullptr, *lossb = nullptr;
+  float* wpart = nullptr;           // partial weight gradients
   float *scale = nullptr, *feat = nullptr;
   int cd(int l) const { return 2 * depth + (depth - 2 - l); }
   int head() const { return 3 * depth - 1; }
@@ -535,8 +619,9 @@ static void free_batch(NNModel* m) {
   for (auto v : {&m->act, &m->gact, &m->pool, &m->gpool, &m->sum, &m->gsum})
     for (auto p : *v) (void)hipFree(p);
   for (auto v : {&m->act, &m->gact, &m->pool, &m->gpool, &m->sum, &m->gsum}) v->clear();
-  for (void* p : {(void*)m->xin, (void*)m->y, (void*)m->gy, (void*)m->lossb}) (void)hipFree(p);
-  m->xin = m->y = m->gy = m->lossb = nullptr;
+  for (void* p : {(void*)m->xin, (void*)m->y, (void*)m->gy, (void*)m->lossb, (void*)m->wpart})
+    (void)hipFree(p);
+  m->xin = m->y = m->gy = m->lossb = m->wpart = nullptr;
   m->bmax = 0;
 }
 
@@ -560,6 +645,11 @@ static void ensure_batch(NNModel* m, int B) {
   m->y = nalloc<float>((long)B * m->cout * m->grid[0].N());
   m->gy = nalloc<float>((long)B * m->cout * m->grid[0].N());
   m->lossb = nalloc<float>(B);
+  // the chunk count does not fall with the batch, so the largest batch's partial sums serve all
+  long part = 0;
+  for (size_t c = 0; c < m->conv.size(); c++)
+    part = std::max(part, wgrad3_part((long)B * m->grid[m->level_of((int)c)].N(), m->conv[c].ci, m->conv[c].co));
+  m->wpart = nalloc<float>(part);
   m->bmax = B;
 }
 
@@ -622,17 +712,8 @@ static void conv_bwd(NNModel* m, int c, int B, const float* in, float* gout, flo
     long n = (long)B * cs.co * g.N();
     hipLaunchKernelGGL(k_relu_bwd, nbk(n, 256), 256, 0, s, n, outact, gout);
   }
-  hipLaunchKernelGGL(k_conv_bwd_w, cs.co * cs.ci, 256, 0, s, B, cs.ci, cs.co, g, gout, in, m->grads + cs.woff);
-  hipLaunchKernelGGL(k_bias_grad, cs.co, 256, 0, s, B, cs.co, g.N(), gout, m->grads + cs.boff);
-  if (gin) {
-    const long nb = (long)B * g.N();
-    if (cs.ci % 4 == 0)
-      hipLaunchKernelGGL(k_conv_bwd_data_blk<4>, dim3(nbk(nb, 256), cs.ci / 4), 256, 0, s, B, cs.ci, cs.co, g, gout,
-                         m->params + cs.woff, gin);
-    else
-      hipLaunchKernelGGL(k_conv_bwd_data, nbk(nb * cs.ci, 256), 256, 0, s, B, cs.ci, cs.co, g, gout,
-                         m->params + cs.woff, gin);
-  }
+  wgrad3(B, cs.ci, cs.co, g, gout, in, m->wpart, m->grads + cs.woff, s);
+  if (gin) conv3_bwd_data(B, cs.ci, cs.co, g, gout, m->params + cs.woff, gin, s);
 }
 
 // backward from m->gy (dL/dy); parameter gradients written into m->grads
@@ -833,38 +914,26 @@ __global__ __launch_bounds__(256) void k_conv1_fwd(int B, int Ci, int Co, long N
   for (int c = 0; c < COB; c++) out[((long)b * Co + co0 + c) * N + p] = acc[c];
 }
 
-// gin[b][ci][p] = sum_co w[co][ci] gout[b][co][p]
-__global__ void k_conv1_bwd_data(int B, int Ci, int Co, long N, const float* __restrict__ gout,
-                                 const float* __restrict__ w, float* __restrict__ gin) {
+// gin[b][ci][p] = sum_co w[co][ci] gout[b][co][p]; CIB input channels per thread, so that gout is
+// read Ci / CIB times instead of Ci times
+template <int CIB>
+__global__ __launch_bounds__(256) void k_conv1_bwd_data(int B, int Ci, int Co, long N, const float* __restrict__ gout,
+                                                        const float* __restrict__ w, float* __restrict__ gin) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const int c0 = blockIdx.y * CIB;
   if (t >= (long)B * N) return;
   const long p = t % N;
   const int b = (int)(t / N);
-  for (int ci = 0; ci < Ci; ci++) {
-    float a = 0.0f;
-    for (int co = 0; co < Co; co++) a += w[(long)co * Ci + ci] * gout[((long)b * Co + co) * N + p];
-    gin[((long)b * Ci + ci) * N + p] = a;
+  float acc[CIB];
+#pragma unroll
+  for (int c = 0; c < CIB; c++) acc[c] = 0.0f;
+  for (int co = 0; co < Co; co++) {
+    const float v = gout[((long)b * Co + co) * N + p];
+#pragma unroll
+    for (int c = 0; c < CIB; c++) acc[c] += w[(long)co * Ci + c0 + c] * v;
   }
-}
-
-// dw[co][ci] = sum_b sum_p gout[b][co][p] in[b][ci][p]; one block per (co, ci)
-__global__ __launch_bounds__(256) void k_conv1_bwd_w(int B, int Ci, int Co, long N, const float* __restrict__ gout,
-                                                     const float* __restrict__ in, float* __restrict__ dw) {
-  __shared__ float sm[256];
-  const int co = blockIdx.x / Ci, ci = blockIdx.x % Ci;
-  float a = 0.0f;
-  for (long t = threadIdx.x; t < (long)B * N; t += 256) {
-    const int b = (int)(t / N);
-    const long p = t % N;
-    a += gout[((long)b * Co + co) * N + p] * in[((long)b * Ci + ci) * N + p];
-  }
-  sm[threadIdx.x] = a;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] += sm[threadIdx.x + s];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) dw[(long)co * Ci + ci] = sm[0];
+#pragma unroll
+  for (int c = 0; c < CIB; c++) gin[((long)b * Ci + c0 + c) * N + p] = acc[c];
 }
 
 // out[b][e] = sum_s (delta_s,13 + y[b][s][e]) r[b][e + off(s)]  (0 outside the grid);
@@ -1025,6 +1094,7 @@ struct SchurNet {
   int bmax = 0;
   std::vector<float*> act, gact;
   float *xin = nullptr, *y = nullptr, *gy = nullptr, *diff = nullptr, *lossb = nullptr, *gscale = nullptr;
+  float* wpart = nullptr;  // partial weight gradients
   double* part = nullptr;
   // training set (all samples on one grid)
   Grid3 dg{0, 0, 0};
@@ -1056,9 +1126,9 @@ static void snn_free_batch(SchurNet* m) {
   m->act.clear();
   m->gact.clear();
   for (void* p : {(void*)m->xin, (void*)m->y, (void*)m->gy, (void*)m->diff, (void*)m->lossb, (void*)m->gscale,
-                  (void*)m->part})
+                  (void*)m->part, (void*)m->wpart})
     (void)hipFree(p);
-  m->xin = m->y = m->gy = m->diff = m->lossb = m->gscale = nullptr;
+  m->xin = m->y = m->gy = m->diff = m->lossb = m->gscale = m->wpart = nullptr;
   m->part = nullptr;
   m->bmax = 0;
   m->ncap = 0;
@@ -1078,6 +1148,8 @@ static void snn_ensure(SchurNet* m, int B, long N, bool train) {
     m->gy = nalloc<float>(n * 27);
     m->diff = nalloc<float>(n);
     m->part = nalloc<double>((long)B * nbk(N, 256) * 2);
+    // the chunk count does not fall with the points, so the largest batch's partial sums serve all
+    m->wpart = nalloc<float>(std::max({wgrad3_part(n, kSnnFeat, m->C), wgrad3_part(n, m->C, m->C), wgrad1_part(n, m->C)}));
   }
   m->lossb = nalloc<float>(B);
   m->gscale = nalloc<float>(B);
@@ -1129,24 +1201,15 @@ static void snn_loss_backward(SchurNet* m, int B, Grid3 g, const float* r, const
   hipLaunchKernelGGL(k_snn_stencil_grad, nbk(nb, 256), 256, 0, s, B, g, m->diff, r, m->gscale, m->gy);
   // head (1x1x1)
   const int L = m->L, C = m->C;
-  hipLaunchKernelGGL(k_conv1_bwd_w, 27 * C, 256, 0, s, B, C, 27, N, m->gy, m->act[L - 1], m->grads + m->woff[L]);
-  hipLaunchKernelGGL(k_bias_grad, 27, 256, 0, s, B, 27, N, m->gy, m->grads + m->boff[L]);
-  hipLaunchKernelGGL(k_conv1_bwd_data, nbk(nb, 256), 256, 0, s, B, C, 27, N, m->gy, m->params + m->woff[L],
+  wgrad1(B, C, N, m->gy, m->act[L - 1], m->wpart, m->grads + m->woff[L], s);
+  hipLaunchKernelGGL(k_conv1_bwd_data<8>, dim3(nbk(nb, 256), C / 8), 256, 0, s, B, C, 27, N, m->gy, m->params + m->woff[L],
                      m->gact[L - 1]);
   for (int l = L - 1; l >= 0; l--) {
     const int ci = l == 0 ? kSnnFeat : C;
     hipLaunchKernelGGL(k_relu_bwd, nbk(nb * C, 256), 256, 0, s, nb * C, m->act[l], m->gact[l]);
     const float* in = l == 0 ? m->xin : m->act[l - 1];
-    hipLaunchKernelGGL(k_conv_bwd_w, C * ci, 256, 0, s, B, ci, C, g, m->gact[l], in, m->grads + m->woff[l]);
-    hipLaunchKernelGGL(k_bias_grad, C, 256, 0, s, B, C, N, m->gact[l], m->grads + m->boff[l]);
-    if (l > 0) {
-      if (ci % 4 == 0)
-        hipLaunchKernelGGL(k_conv_bwd_data_blk<4>, dim3(nbk(nb, 256), ci / 4), 256, 0, s, B, ci, C, g, m->gact[l],
-                           m->params + m->woff[l], m->gact[l - 1]);
-      else
-        hipLaunchKernelGGL(k_conv_bwd_data, nbk(nb * ci, 256), 256, 0, s, B, ci, C, g, m->gact[l],
-                           m->params + m->woff[l], m->gact[l - 1]);
-    }
+    wgrad3(B, ci, C, g, m->gact[l], in, m->wpart, m->grads + m->woff[l], s);
+    if (l > 0) conv3_bwd_data(B, ci, C, g, m->gact[l], m->params + m->woff[l], m->gact[l - 1], s);
   }
   UWG_HIP(hipGetLastError());
 }
