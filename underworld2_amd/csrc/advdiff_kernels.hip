@@ -4,7 +4,7 @@
 // AD/ = LU/Underworld/Utils/AdvectionDiffusion/src/.
 //  * k_supg_elem: the element residual of AD/Residual.cpp:223-343 with the per-element upwind
 //    diffusivity of AD/Residual.cpp:430-513 -- one thread per element, the 3^dim Gauss points
-//    of the Q1 mesh, written to [E][2^dim] (no atomics).
+//    of the Q1 mesh, written to [2^dim][E] (no atomics).
 //  * k_supg_correct: vertex gather of the element residuals in a fixed element order, then the
 //    explicit corrector of AD/Multicorrector.c:206-260: dphidot = R / M (lumped mass),
 //    phi += dt gamma dphidot, phidot += dphidot on free dofs, nodal fields refreshed.
@@ -91,13 +91,71 @@ __device__ __forceinline__ void ad_shape(const double* X, double* N, double (*dN
   }
 }
 
+// Shape functions, their local derivatives and the weight at every Gauss point, evaluated at
+// compile time with the expressions of ad_gauss / ad_shape.
 template <int DIM>
-__global__ void k_supg_elem(ADGeom G, const double* __restrict__ phi, const double* __restrict__ phidot,
-                            const double* __restrict__ vel, const double* __restrict__ kap,
-                            const double* __restrict__ src, int upwind, double* __restrict__ res_e) {
+struct SupgRule {
+  static constexpr int NN = DIM == 3 ? 8 : 4, Q = DIM == 3 ? 27 : 9;
+  double N[Q][NN] = {}, dN[Q][DIM][NN] = {}, w[Q] = {};
+  constexpr SupgRule() {
+    const double ga = 0.77459666924148337704;
+    const double x1[3] = {-ga, 0.0, ga}, w1[3] = {5.0 / 9.0, 8.0 / 9.0, 5.0 / 9.0};
+    for (int q = 0; q < Q; q++) {
+      const double X[3] = {x1[q % 3], x1[(q / 3) % 3], DIM == 3 ? x1[q / 9] : 0.0};
+      w[q] = w1[q % 3] * w1[(q / 3) % 3] * (DIM == 3 ? w1[q / 9] : 1.0);
+      for (int a = 0; a < NN; a++) {
+        double s[3] = {}, f[3] = {};
+        for (int d = 0; d < DIM; d++) {
+          s[d] = ((a >> d) & 1) ? 1.0 : -1.0;
+          f[d] = 0.5 * (1.0 + s[d] * X[d]);
+        }
+        N[q][a] = f[0] * f[1] * (DIM == 3 ? f[2] : 1.0);
+        for (int k = 0; k < DIM; k++) {
+          double v = 0.5 * s[k];
+          for (int d = 0; d < DIM; d++)
+            if (d != k) v *= f[d];
+          dN[q][k][a] = v;
+        }
+      }
+    }
+  }
+};
+__constant__ const SupgRule<2> kSupgRule2 = SupgRule<2>();
+__constant__ const SupgRule<3> kSupgRule3 = SupgRule<3>();
+template <int DIM>
+__device__ __forceinline__ const SupgRule<DIM>& supg_rule() {
+  if constexpr (DIM == 3)
+    return kSupgRule3;
+  else
+    return kSupgRule2;
+}
+
+// FP64 arithmetic bound (about 9,000 operations per 3D element: multiplies and adds stay separate,
+// see the build flags).  The rule's tables are wave-uniform and come through scalar registers; the
+// diffusivities, 27 consecutive values per element, are staged in LDS by coalesced loads.  Forming
+// the shape functions per thread with indices the compiler kept in scratch, and reading the
+// diffusivities with a 216-byte stride, took 470 us for 64^3 elements; this takes
+// 108 us.
+constexpr int kSupgBlock = 128;
+template <int DIM>
+__global__ __launch_bounds__(kSupgBlock, 2) void k_supg_elem(ADGeom G, const double* __restrict__ phi,
+                                                             const double* __restrict__ phidot,
+                                                             const double* __restrict__ vel,
+                                                             const double* __restrict__ kap,
+                                                             const double* __restrict__ src, int upwind,
+                                                             double* __restrict__ res_e) {
   constexpr int NN = DIM == 3 ? 8 : 4, Q = DIM == 3 ? 27 : 9;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ double ks[kSupgBlock * Q];
+  const long e0 = (long)blockIdx.x * kSupgBlock, e = e0 + threadIdx.x;
+  {
+    const double* kb = kap + e0 * Q;
+    const int n = (int)min((long)kSupgBlock, G.E - e0) * Q;
+    for (int q = threadIdx.x; q < n; q += kSupgBlock) ks[q] = kb[q];
+  }
+  __syncthreads();
   if (e >= G.E) return;
+  const double* kq_ = ks + threadIdx.x * Q;
+  const SupgRule<DIM>& R = supg_rule<DIM>();
   double V[24];
   element_verts<DIM>(G.res, G.lo, G.hi, e, V);
   double h[3] = {1.0, 1.0, 1.0}, detJ = 1.0;
@@ -108,69 +166,77 @@ __global__ void k_supg_elem(ADGeom G, const double* __restrict__ phi, const doub
   const long nx = G.res[0] + 1, ny = G.res[1] + 1;
   const long i = e % G.res[0], j = (e / G.res[0]) % G.res[1], k = DIM == 3 ? e / ((long)G.res[0] * G.res[1]) : 0;
   const long base = i + nx * (j + ny * k);
-  long nodes[8];
   double ph[8], pd[8], vv[8][3];
+#pragma unroll
   for (int a = 0; a < NN; a++) {
-    nodes[a] = base + (a & 1) + ((a >> 1) & 1) * nx + (DIM == 3 ? ((a >> 2) & 1) * nx * ny : 0);
-    ph[a] = phi[nodes[a]];
-    pd[a] = phidot[nodes[a]];
-    for (int d = 0; d < DIM; d++) vv[a][d] = vel[nodes[a] * DIM + d];
+    const long n = base + (a & 1) + ((a >> 1) & 1) * nx + (DIM == 3 ? ((a >> 2) & 1) * nx * ny : 0);
+    ph[a] = phi[n];
+    pd[a] = phidot[n];
+#pragma unroll
+    for (int d = 0; d < DIM; d++) vv[a][d] = vel[n * DIM + d];
   }
   // upwind diffusivity (element mean diffusivity, velocity at the centre)
   double avg = 0.0;
-  for (int q = 0; q < Q; q++) avg += kap[e * Q + q];
+  for (int q = 0; q < Q; q++) avg += kq_[q];
   avg /= (double)Q;
   if (avg < AD_MIN_DIFFUSIVITY) avg = AD_MIN_DIFFUSIVITY;
   double vc[3] = {0.0, 0.0, 0.0};
-  {
-    const double Xc[3] = {0.0, 0.0, 0.0};
-    double Nc[8], dNc[3][8];
-    ad_shape<DIM>(Xc, Nc, dNc);
-    for (int a = 0; a < NN; a++)
-      for (int d = 0; d < DIM; d++) vc[d] += vv[a][d] * Nc[a];
-  }
+#pragma unroll
+  for (int a = 0; a < NN; a++)
+#pragma unroll
+    for (int d = 0; d < DIM; d++) vc[d] += vv[a][d] * (DIM == 3 ? 0.125 : 0.25);
   double up = 0.0;
   for (int d = 0; d < DIM; d++) {
     const double pe = vc[d] * h[d] / (2.0 * avg);
     up += ad_upwind(pe, upwind) * vc[d] * h[d];
   }
   up *= AD_ISQRT15;
+  const bool plain = fabs(up) < AD_MIN_DIFFUSIVITY;
+  double sc[3];
+#pragma unroll
+  for (int d = 0; d < DIM; d++) sc[d] = 2.0 / h[d];
   double r[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 1
   for (int q = 0; q < Q; q++) {
-    double X[3], w, N[8], dN[3][8];
-    ad_gauss<DIM>(q, X, &w);
-    ad_shape<DIM>(X, N, dN);
+    double dN[3][8];
+#pragma unroll
     for (int d = 0; d < DIM; d++)
-      for (int a = 0; a < NN; a++) dN[d][a] *= 2.0 / h[d];
+#pragma unroll
+      for (int a = 0; a < NN; a++) dN[d][a] = R.dN[q][d][a] * sc[d];
     double v[3] = {0.0, 0.0, 0.0}, gphi[3] = {0.0, 0.0, 0.0}, pdot = 0.0;
+#pragma unroll
     for (int a = 0; a < NN; a++) {
+#pragma unroll
       for (int d = 0; d < DIM; d++) {
-        v[d] += vv[a][d] * N[a];
+        v[d] += vv[a][d] * R.N[q][a];
         gphi[d] += ph[a] * dN[d][a];
       }
-      pdot += pd[a] * N[a];
+      pdot += pd[a] * R.N[q][a];
     }
     double udotu = 0.0, vg = 0.0;
+#pragma unroll
     for (int d = 0; d < DIM; d++) {
       udotu += v[d] * v[d];
       vg += v[d] * gphi[d];
     }
-    const double fac = w * detJ;
-    const double kq = kap[e * Q + q];
+    const double fac = R.w[q] * detJ;
+    const double kq = kq_[q];
     const double total = pdot + vg - (src ? src[e * Q + q] : 0.0);
-    const bool plain = fabs(up) < AD_MIN_DIFFUSIVITY;
     const double supgf = plain ? 0.0 : up / udotu;
+#pragma unroll
     for (int a = 0; a < NN; a++) {
       double pert = 0.0, dif = 0.0;
+#pragma unroll
       for (int d = 0; d < DIM; d++) {
         pert += v[d] * dN[d][a];
         dif += dN[d][a] * gphi[d];
       }
-      const double sn = plain ? N[a] : N[a] + supgf * pert;
+      const double sn = plain ? R.N[q][a] : R.N[q][a] + supgf * pert;
       r[a] -= fac * (sn * total + kq * dif);
     }
   }
-  for (int a = 0; a < NN; a++) res_e[e * NN + a] = r[a];
+#pragma unroll
+  for (int a = 0; a < NN; a++) res_e[a * G.E + e] = r[a];
 }
 
 template <int DIM>
@@ -191,13 +257,12 @@ __global__ void k_supg_mass(ADGeom G, double* __restrict__ me) {
     for (int a = 0; a < NN; a++)
       for (int b = 0; b < NN; b++) m[a] += N[a] * N[b] * fac;
   }
-  for (int a = 0; a < NN; a++) me[e * NN + a] = m[a];
+  for (int a = 0; a < NN; a++) me[a * G.E + e] = m[a];
 }
 
 // sum of the element entries around vertex n (fixed order: lower elements first)
 template <int DIM>
 __device__ __forceinline__ double ad_gather(const ADGeom& G, const double* __restrict__ ve, long n) {
-  constexpr int NN = DIM == 3 ? 8 : 4;
   const long nx = G.res[0] + 1, ny = G.res[1] + 1;
   const int I = (int)(n % nx), J = (int)((n / nx) % ny), K = DIM == 3 ? (int)(n / (nx * ny)) : 0;
   double acc = 0.0;
@@ -208,7 +273,7 @@ __device__ __forceinline__ double ad_gather(const ADGeom& G, const double* __res
         if (ei < 0 || ei >= G.res[0] || ej < 0 || ej >= G.res[1] || ek < 0 || ek >= G.res[2]) continue;
         const long e = ei + (long)G.res[0] * (ej + (long)G.res[1] * ek);
         const int a = (1 - ox) + 2 * (1 - oy) + (DIM == 3 ? 4 * (1 - oz) : 0);
-        acc += ve[e * NN + a];
+        acc += ve[a * G.E + e];
       }
   return acc;
 }
@@ -275,9 +340,9 @@ void launch_supg_elem(const Geom& g, const double* phi, const double* phidot, co
                       const double* src, int upwind, double* res_e, hipStream_t s) {
   const ADGeom G = ad_pack(g);
   if (g.dim == 3)
-    hipLaunchKernelGGL(k_supg_elem<3>, ad_blocks(g.E, 128), 128, 0, s, G, phi, phidot, vel, kap, src, upwind, res_e);
+    hipLaunchKernelGGL(k_supg_elem<3>, ad_blocks(g.E, kSupgBlock), kSupgBlock, 0, s, G, phi, phidot, vel, kap, src, upwind, res_e);
   else
-    hipLaunchKernelGGL(k_supg_elem<2>, ad_blocks(g.E, 128), 128, 0, s, G, phi, phidot, vel, kap, src, upwind, res_e);
+    hipLaunchKernelGGL(k_supg_elem<2>, ad_blocks(g.E, kSupgBlock), kSupgBlock, 0, s, G, phi, phidot, vel, kap, src, upwind, res_e);
   UWG_HIP(hipGetLastError());
 }
 
