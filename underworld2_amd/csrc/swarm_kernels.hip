@@ -2,6 +2,8 @@
 // discrete-Voronoi weights, RK2 advection and interpolation.
 // Compiled with -ffp-contract=off: every floating-point expression keeps the reference's
 // operation order (citations in uwg_geom.h and below; LU/ = src/underworld/libUnderworld/).
+#include <algorithm>
+
 #include "uwg_internal.h"
 #include "uwg_geom.h"
 
@@ -379,6 +381,346 @@ __global__ void k_dvc(int num, long E0, long nE, const int* elist, const int* ce
   flag[t] = 0;
 }
 
+// ---------------------------------------------------------------------------------------
+// The same claims a round at a time (default grid of 15 cells per axis, at most 64 particles).
+// A particle's chain is fixed when its step begins: it is the set of neighbours of the cells it
+// claimed in the round before.  So a round is known cell by cell: the particles examining cell c
+// are those that claimed one of its neighbours in the last round, and taking them in particle
+// order against the cell's owner gives the claims, and the owner, of the sequential algorithm.
+// Cells are independent within a round, so all of a round's cells are processed at once: about 14
+// rounds instead of 300 dependent particle steps per element.
+//
+// Left out are examinations by a particle that owned the cell at its step: it either still owns it
+// or has lost it to a strictly closer one, so it cannot claim it.  That argument, and the
+// single-precision test below, need the comparisons to be those of real numbers; a comparison
+// within kDvcTie of a tie (symmetric layouts have exact ones) sends the element to the
+// sequential kernel, as do more than 64 particles and more active cells than the lists hold.
+//
+// Layout: cell (i, j, k) at i + 16 j + 256 k with blocked cells at i = 15, j = 15 and around the
+// grid, so that neighbours need neither divisions nor bounds tests.  Per cell one owner byte and
+// one mask of examining particles; the cells with a mask are listed.  A round is two passes: the
+// listed cells are examined and their claims listed (cell, claiming particles), then the claims
+// are spread to the masks of the neighbours.  LDS: 30 KB with 32-bit masks (five workgroups per
+// CU), 54 KB with 64-bit ones (three).  Bound by instruction issue and LDS latency (25,000 vector
+// instructions per element, in about 170 examining and 70 spreading wave passes and the centroids).
+// Measured: 48 x 40 x 56 elements of 25 particles 27.5 -> 6.6 ms against k_dvc_wave, 64 x 64 of
+// 20 particles 234 -> 36 us.
+// ---------------------------------------------------------------------------------------
+constexpr int kDvcNum = 15, kDvcFree = 0xFF, kDvcWall = 0xFE;
+constexpr double kDvcTie = 1e-12;  // rounding of the test: 3 terms of at most 8 x 4 roundings, 2e-14
+constexpr float kDvcNear = 2e-5f;  // single precision, coordinates up to 1.2: error below 1e-5
+
+template <int DIM, typename MT>
+struct DvcRound {
+  static constexpr int CELLS = DIM == 3 ? kDvcNum * 256 : 256, GUARD = DIM == 3 ? 256 : 16;
+  // listed cells and claims per round; the largest seen in 300 random cells of 32 / 60 particles
+  // are 1,400 / 1,770 and 910 / 1,100
+  static constexpr int CAP = DIM == 3 ? (sizeof(MT) == 8 ? 1920 : 1536) : 256;
+  static constexpr int CLAIMS = DIM == 3 ? (sizeof(MT) == 8 ? 1280 : 1024) : 256;
+  static constexpr int BS = DIM == 3 ? 256 : 64;  // a round lists about 470 (3D) / 55 (2D) cells
+  static constexpr int BATCHES = CELLS / BS;      // of 64 cells per wave
+  static constexpr int WAVES = sizeof(MT) == 8 ? 3 : 5;  // per SIMD, as many as LDS allows in 3D
+};
+
+template <int DIM, typename MT>
+__global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)) void k_dvc_rounds(long E, const int* __restrict__ cell_ptr,
+                                                                        double* __restrict__ xi_slot,
+                                                                        double* __restrict__ w_slot,
+                                                                        int* __restrict__ wide,
+                                                                        int* __restrict__ retry,
+                                                                        int* __restrict__ counts) {
+  using D = DvcRound<DIM, MT>;
+  constexpr int BS = D::BS, NPM = 8 * (int)sizeof(MT), NB = 2 * DIM;
+  constexpr bool WIDE = sizeof(MT) == 8;
+  __shared__ MT mask[D::CELLS];
+  __shared__ __align__(16) unsigned char own_[D::CELLS + 2 * D::GUARD];
+  // the claims' particles and cells and the listed cells; after the rounds the cells by owner
+  __shared__ __align__(16) unsigned char lists[D::CLAIMS * (sizeof(MT) + 2) + D::CAP * 2];
+  static_assert(sizeof(lists) >= 2 * ((DIM == 3 ? 3375 : 225) + 3 * NPM + 3), "cells by owner");
+  MT* cl_mask = reinterpret_cast<MT*>(lists);
+  unsigned short* cl_cell = reinterpret_cast<unsigned short*>(lists + D::CLAIMS * sizeof(MT));
+  unsigned short* list = cl_cell + D::CLAIMS;
+  unsigned short* order = reinterpret_cast<unsigned short*>(lists);
+  __shared__ float4 pos[NPM];  // -2 x, -2 y, -2 z, |x|^2
+  __shared__ unsigned short count[BS / 64][NPM], first[NPM], cells[NPM];
+  __shared__ double cen[kDvcNum + 1];
+  // counts of the listed cells and claims (alternating, so that one is cleared while the other is
+  // in use), failures noticed while examining and while spreading
+  __shared__ int n_cell[2], n_claim[2], bad_exam, bad_spread;
+  unsigned char* own = own_ + D::GUARD;
+  const int tid = threadIdx.x, lane = tid & 63, wave0 = tid & ~63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const double dx = (1.0 - -1.0) / kDvcNum, dy = dx, dz = dx;
+  const long n_el = WIDE ? (long)counts[0] : E;
+  if (blockIdx.x >= n_el) return;
+  if (tid == 0) {
+    // cell centres: X = X + dx accumulation per axis (_DVCWeights_ConstructGrid :527-544)
+    double X = -1.0 - dx / 2.0;
+    for (int i = 0; i < kDvcNum; i++) { X = X + dx; cen[i] = X; }
+    cen[kDvcNum] = 0.0;
+  }
+  for (int q = tid; q < D::CELLS; q += BS) mask[q] = 0;
+  for (long it = blockIdx.x; it < n_el; it += gridDim.x) {
+    const long e = WIDE ? (long)wide[it] : it;
+    const int s0 = cell_ptr[e], np = cell_ptr[e + 1] - s0;
+    if (np <= 0 || np > NPM) {
+      if (tid == 0) {
+        if (np <= 0)
+          atomicMin(&counts[2], (int)e);
+        else if (!WIDE && np <= 64)
+          wide[atomicAdd(&counts[0], 1)] = (int)e;
+        else
+          retry[atomicAdd(&counts[1], 1)] = (int)e;
+      }
+      continue;
+    }
+    __syncthreads();
+    {
+      unsigned* o32 = reinterpret_cast<unsigned*>(own_);
+      for (int q = tid; q < (D::CELLS + 2 * D::GUARD) / 4; q += BS) {
+        const int c = q * 4 - D::GUARD;  // first of four cells
+        const bool wall = c < 0 || c >= D::CELLS || (c & 0xF0) == 0xF0;
+        o32[q] = wall ? 0xFEFEFEFEu : ((c & 0xC) == 0xC ? 0xFEFFFFFFu : 0xFFFFFFFFu);
+      }
+      if (tid == 0) n_cell[0] = n_cell[1] = n_claim[0] = n_claim[1] = bad_exam = bad_spread = 0;
+    }
+    __syncthreads();
+    // the wave's lanes with claims append them to the list
+    auto list_claim = [&](int c, MT claim, int* count) {
+      const unsigned long long b = __ballot(claim != 0);
+      if (b == 0) return;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(count, __popcll(b));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (base + __popcll(b) > D::CLAIMS) {
+        if (lane == 0) bad_exam = 1;
+        return;
+      }
+      if (claim) {
+        const int at = base + __popcll(b & below);
+        cl_cell[at] = (unsigned short)c;
+        cl_mask[at] = claim;
+      }
+    };
+    // seeds (_DVCWeights_CreateVoronoi3D :676-721): of several in one cell the last owns it
+    int seed = 0;
+    if (tid < np) {
+      const double* x = xi_slot + (long)(s0 + tid) * DIM;
+      int k = (int)((x[0] - -1.0) / dx);
+      int j = (int)((x[1] - -1.0) / dy);
+      int l = DIM == 3 ? (int)((x[2] - -1.0) / dz) : 0;
+      if (k == kDvcNum) k--;
+      if (j == kDvcNum) j--;
+      if (DIM == 3 && l == kDvcNum) l--;
+      k = k < 0 ? 0 : (k > kDvcNum - 1 ? kDvcNum - 1 : k);
+      j = j < 0 ? 0 : (j > kDvcNum - 1 ? kDvcNum - 1 : j);
+      l = l < 0 ? 0 : (l > kDvcNum - 1 ? kDvcNum - 1 : l);
+      seed = k + 16 * j + 256 * l;
+      atomicOr(&mask[seed], (MT)1 << tid);
+      for (int d = 0; d < DIM; d++)
+        if (!(fabs(x[d]) <= 1.2)) bad_exam = 1;  // outside what kDvcNear allows for
+      const float fx = (float)x[0], fy = (float)x[1], fz = DIM == 3 ? (float)x[2] : 0.0f;
+      pos[tid] = make_float4(-2.0f * fx, -2.0f * fy, -2.0f * fz, fx * fx + fy * fy + fz * fz);
+    }
+    __syncthreads();
+    MT claim = 0;
+    if (tid < np) {
+      const MT m = mask[seed];
+      const int last = WIDE ? 63 - __clzll((long long)m) : 31 - __clz((int)m);
+      if (last == tid) {
+        own[seed] = (unsigned char)tid;
+        claim = m;
+      }
+    }
+    __syncthreads();
+    if (claim) mask[seed] = 0;
+    if (tid < 64) list_claim(seed, claim, &n_claim[0]);  // np <= 64
+    __syncthreads();
+    // rounds (_DVCWeights_UpdateBchain :388-438, _DVCWeights_ClaimCells :256-311).  bad_exam is
+    // written only while examining and read only after the barrier that follows, bad_spread
+    // likewise while spreading, so all waves leave the loop at the same place.
+    int cu = 0;
+    bool fail = false;
+    while (true) {
+      const int ncl = n_claim[cu];
+      fail = bad_exam != 0;
+      if (fail || ncl == 0) break;
+      if (tid == 0) n_cell[cu ^ 1] = 0;
+      // neighbours of the claimed cells, but for claimants that own them already
+      for (int q = tid; q - lane < ncl; q += BS) {
+        const int off[6] = {-16, 16, 1, -1, 256, -256};
+        const bool on = q < ncl;
+        const int c = on ? cl_cell[q] : 0;
+        const MT cl = on ? cl_mask[q] : (MT)0;
+        unsigned o[NB];
+#pragma unroll
+        for (int k = 0; k < NB; k++) o[k] = own[c + off[k]];
+        bool fresh[NB];
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          const MT self = (MT)(o[k] < (unsigned)NPM) << (o[k] & (NPM - 1));
+          const MT m = o[k] == (unsigned)kDvcWall ? (MT)0 : cl & ~self;
+          MT old = 1;
+          if (m) old = atomicOr(&mask[c + off[k]], m);
+          fresh[k] = old == 0;
+        }
+        int at[NB], total = 0;
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+          const unsigned long long b = __ballot(fresh[k]);
+          at[k] = total + __popcll(b & below);
+          total += __popcll(b);
+        }
+        if (total == 0) continue;
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&n_cell[cu], total);
+        base = __builtin_amdgcn_readfirstlane(base);
+        if (base + total > D::CAP) {
+          if (lane == 0) bad_spread = 1;
+          continue;
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++)
+          if (fresh[k]) list[base + at[k]] = (unsigned short)(c + off[k]);
+      }
+      __syncthreads();
+      const int n = n_cell[cu];
+      fail = bad_spread != 0;
+      if (fail) break;
+      if (tid == 0) n_claim[cu] = 0;
+      for (int q = tid; q - lane < n; q += BS) {
+        int c = 0;
+        claim = 0;
+        if (q < n) {
+          c = list[q];
+          MT ex = mask[c];
+          mask[c] = 0;
+          int o = own[c];
+          const int ci = c & 15, cj = (c >> 4) & 15, ck = DIM == 3 ? c >> 8 : 0;
+          const float step = 2.0f / kDvcNum, half = 1.0f / kDvcNum - 1.0f;
+          const float fx = __builtin_fmaf(step, (float)ci, half), fy = __builtin_fmaf(step, (float)cj, half),
+                      fz = __builtin_fmaf(step, (float)ck, half);
+          auto dist = [&](int p) {  // squared distance less |cell|^2
+            const float4 a = pos[p];
+            const float v = __builtin_fmaf(a.x, fx, __builtin_fmaf(a.y, fy, a.w));
+            return DIM == 3 ? __builtin_fmaf(a.z, fz, v) : v;
+          };
+          float best = o == kDvcFree ? 3e38f : dist(o);
+          do {
+            const int p = WIDE ? __ffsll((long long)ex) - 1 : __ffs((int)ex) - 1;
+            ex &= ex - 1;
+            const float dp = dist(p), diff = dp - best;
+            bool take = o == kDvcFree || diff < 0.0f;
+            if (fabsf(diff) < kDvcNear && p != o) {
+              // DistanceTest in the reference's operation order
+              const double x0 = cen[ci], y0 = cen[cj], z0 = cen[ck];
+              const double* p1 = xi_slot + (long)(s0 + o) * DIM;
+              const double* p2 = xi_slot + (long)(s0 + p) * DIM;
+              double r = (p1[0] + p2[0] - x0 - x0) * (p1[0] - p2[0]) + (p1[1] + p2[1] - y0 - y0) * (p1[1] - p2[1]);
+              if (DIM == 3) r = r + (p1[2] + p2[2] - z0 - z0) * (p1[2] - p2[2]);
+              take = r > 0.0;
+              if (!(fabs(r) > kDvcTie)) bad_exam = 1;
+            }
+            if (take && p != o) {
+              o = p;
+              best = dp;
+              claim |= (MT)1 << p;
+            }
+          } while (ex);
+          if (claim) own[c] = (unsigned char)o;
+        }
+        list_claim(c, claim, &n_claim[cu ^ 1]);
+      }
+      __syncthreads();
+      cu ^= 1;
+    }
+    if (fail) {
+      __syncthreads();
+      for (int q = tid; q < D::CELLS; q += BS) mask[q] = 0;
+      if (tid == 0) retry[atomicAdd(&counts[1], 1)] = (int)e;
+      continue;
+    }
+    // centroids and weights in grid order (_DVCWeights_GetCentroids3D :198-226): the cells are
+    // sorted by owner, stably, so that one lane per particle and component adds up a contiguous
+    // list.  (A lane that walked the grid's rows for its particle's cells took 8.7 ms of a 14.5 ms
+    // pass at 48 x 40 x 56: neighbouring lanes' particles have their rows at different places, so
+    // a wave stepped through nearly all of them.)
+    unsigned rank[D::BATCHES];
+    {
+      unsigned short* cnt = count[tid >> 6];
+      if (lane < NPM) cnt[lane] = 0;
+#pragma unroll
+      for (int b = 0; b < D::BATCHES; b++) {
+        const unsigned o = own[(tid >> 6) * (64 * D::BATCHES) + 64 * b + lane];
+        const bool on = o < (unsigned)NPM;
+        unsigned long long peers = __ballot(on);
+#pragma unroll
+        for (int k = 0; k < (WIDE ? 6 : 5); k++) {
+          const unsigned long long m = __ballot((o >> k) & 1);
+          peers &= (o >> k) & 1 ? m : ~m;
+        }
+        __builtin_amdgcn_wave_barrier();
+        const int had = on ? cnt[o] : 0;
+        const int r = __popcll(peers & below);
+        __builtin_amdgcn_wave_barrier();
+        if (on && r == 0) cnt[o] = (unsigned short)(had + __popcll(peers));
+        rank[b] = (unsigned)(had + r) << 8 | o;
+      }
+    }
+    __syncthreads();
+    if (tid < 64) {
+      int n = 0;
+      if (lane < NPM)
+        for (int w = 0; w < BS / 64; w++) {
+          const int m = count[w][lane];
+          count[w][lane] = (unsigned short)n;
+          n += m;
+        }
+      int end = (n + 3) & ~3;  // lists start at multiples of four entries
+      for (int k = 1; k < 64; k <<= 1) {
+        const int v = __shfl_up(end, k);
+        if (lane >= k) end += v;
+      }
+      const int start = end - ((n + 3) & ~3);
+      if (lane < NPM) {
+        for (int w = 0; w < BS / 64; w++) count[w][lane] += (unsigned short)start;
+        for (int k = start + n; k < end; k++) order[k] = 0xFFFF;  // cen[15] = 0
+        first[lane] = (unsigned short)start;
+        cells[lane] = (unsigned short)n;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < D::BATCHES; b++) {
+      const unsigned o = rank[b] & 0xFF;
+      const int c = (tid >> 6) * (64 * D::BATCHES) + 64 * b + lane;
+      if (o < (unsigned)NPM) order[count[tid >> 6][o] + (rank[b] >> 8)] = (unsigned short)(c << 3);
+    }
+    __syncthreads();
+    const double da = DIM == 3 ? dx * dy * dz : dx * dy;
+    for (int t = tid; t < np * DIM; t += BS) {
+      const int p = t / DIM, d = t - p * DIM, n = cells[p];
+      const char* table = reinterpret_cast<const char*>(cen);
+      const uint2* at = reinterpret_cast<const uint2*>(order + first[p]);
+      double s = 0.0;
+      for (int k = 0; k < n; k += 4) {
+        const uint2 c = *at++;
+        const unsigned lo = c.x >> (4 * d), hi = c.y >> (4 * d);
+        const double v0 = *reinterpret_cast<const double*>(table + (lo & 0x78)),
+                     v1 = *reinterpret_cast<const double*>(table + (lo >> 16 & 0x78)),
+                     v2 = *reinterpret_cast<const double*>(table + (hi & 0x78)),
+                     v3 = *reinterpret_cast<const double*>(table + (hi >> 16 & 0x78));
+        s += v0;
+        s += v1;
+        s += v2;
+        s += v3;
+      }
+      xi_slot[(long)(s0 + p) * DIM + d] = n != 0 ? s / n : 0.0;
+      if (d == 0) w_slot[s0 + p] = n * da;
+    }
+  }
+}
+
 // One wavefront per element, grid-stride over elements.  The claim grid, a one-bit-per-cell
 // mark and the particles' local coordinates live in LDS (about 8 KB, so many elements are in
 // flight per CU); each particle's boundary chain lives in a per-workgroup global buffer
@@ -396,8 +738,8 @@ __global__ void k_dvc(int num, long E0, long nE, const int* elist, const int* ce
 #define DVCW_MAXNC 4096
 #define DVCW_MAXNP 128
 template <int DIM, int NUM>
-__global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long E, const int* __restrict__ cell_ptr,
-                                                 double* __restrict__ xi_slot, double* __restrict__ w_slot,
+__global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long nE, const int* __restrict__ elist,
+                                                 const int* __restrict__ cell_ptr, double* __restrict__ xi_slot, double* __restrict__ w_slot,
                                                  short* __restrict__ gbound, int cap, int* __restrict__ flag) {
   const int num = NUM > 0 ? NUM : num_rt;  // compile-time grid size for the default resolution
   constexpr int NC = NUM > 0 ? (DIM == 3 ? NUM * NUM * NUM : NUM * NUM) : DVCW_MAXNC;  // claim grid cells
@@ -437,11 +779,12 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long E, const int* 
                                      : (k == 2 ? i < nx - 1 : (k == 3 ? i > 0 : (k == 4 ? kk < nz - 1 : kk > 0))));
     return ok ? c + off : -2;
   };
-  for (long e = blockIdx.x; e < E; e += gridDim.x) {
+  for (long it = blockIdx.x; it < nE; it += gridDim.x) {
+    const long e = elist ? (long)elist[it] : it;
     const int s0 = cell_ptr[e];
     const int np = cell_ptr[e + 1] - s0;
     if (np <= 0 || np > DVCW_MAXNP) {
-      if (lane == 0) flag[e] = np <= 0 ? 2 : 1;
+      if (lane == 0) flag[it] = np <= 0 ? 2 : 1;
       continue;
     }
     for (int c = lane; c < ncell; c += 64) own[c] = 0xFF;
@@ -550,7 +893,7 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long E, const int* 
     if (overflow) {
       // leave LDS marks clean for the next element
       for (int q = lane; q < NCW; q += 64) mark[q] = 0u;
-      if (lane == 0) flag[e] = 1;
+      if (lane == 0) flag[it] = 1;
       __syncthreads();
       continue;
     }
@@ -618,7 +961,7 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long E, const int* 
         if (DIM == 3) out[2] = 0.0;
       }
     }
-    if (lane == 0) flag[e] = 0;
+    if (lane == 0) flag[it] = 0;
     __syncthreads();
   }
 }
@@ -628,18 +971,49 @@ bool dvc_wave_supported(int dim, int num) {
   return nc <= DVCW_MAXNC && num <= 32;
 }
 
-void launch_dvc_wave(int dim, int num, long E, const int* cell_ptr, double* xi_slot, double* w_slot, short* gbound,
-                     int nblk, int cap, int* flag, hipStream_t s) {
-  if (E == 0) return;
+// elements elist[0 .. nE) (all elements where it is null)
+void launch_dvc_wave(int dim, int num, long nE, const int* elist, const int* cell_ptr, double* xi_slot, double* w_slot,
+                     short* gbound, int nblk, int cap, int* flag, hipStream_t s) {
+  if (nE == 0) return;
+  const auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, nblk, 64, 0, s, num, nE, elist, cell_ptr, xi_slot, w_slot, gbound, cap, flag);
+  };
   if (dim == 3 && num == 15)
-    hipLaunchKernelGGL((k_dvc_wave<3, 15>), nblk, 64, 0, s, num, E, cell_ptr, xi_slot, w_slot, gbound, cap, flag);
+    go(k_dvc_wave<3, 15>);
   else if (dim == 3)
-    hipLaunchKernelGGL((k_dvc_wave<3, 0>), nblk, 64, 0, s, num, E, cell_ptr, xi_slot, w_slot, gbound, cap, flag);
+    go(k_dvc_wave<3, 0>);
   else if (num == 15)
-    hipLaunchKernelGGL((k_dvc_wave<2, 15>), nblk, 64, 0, s, num, E, cell_ptr, xi_slot, w_slot, gbound, cap, flag);
+    go(k_dvc_wave<2, 15>);
   else
-    hipLaunchKernelGGL((k_dvc_wave<2, 0>), nblk, 64, 0, s, num, E, cell_ptr, xi_slot, w_slot, gbound, cap, flag);
+    go(k_dvc_wave<2, 0>);
   UWG_HIP(hipGetLastError());
+}
+
+__global__ void k_dvc_reset(int* counts) {
+  if (threadIdx.x < 2) counts[threadIdx.x] = 0;
+  if (threadIdx.x == 2) counts[2] = 0x7fffffff;
+}
+
+// DVC of all elements at the default resolution.  work [2 E + 4]: elements with 33-64 particles,
+// elements left to k_dvc_wave, then the counts of both and the first element without particles
+// (0x7fffffff: none).  Returns the counts' address.
+bool dvc_rounds_supported(int num) { return num == kDvcNum; }
+int* launch_dvc_rounds(int dim, long E, const int* cell_ptr, double* xi_slot, double* w_slot, int cus, int* work,
+                       hipStream_t s) {
+  int *wide = work, *retry = work + E, *counts = work + 2 * E;
+  hipLaunchKernelGGL(k_dvc_reset, 1, 64, 0, s, counts);
+  const auto go = [&](auto k32, auto k64, int bs, int per32, int per64) {
+    hipLaunchKernelGGL(k32, (unsigned)std::min(E, (long)cus * per32), bs, 0, s, E, cell_ptr, xi_slot, w_slot, wide,
+                       retry, counts);
+    hipLaunchKernelGGL(k64, (unsigned)std::min(E, (long)cus * per64), bs, 0, s, E, cell_ptr, xi_slot, w_slot, wide,
+                       retry, counts);
+  };
+  if (dim == 3)
+    go(k_dvc_rounds<3, unsigned>, k_dvc_rounds<3, unsigned long long>, DvcRound<3, unsigned>::BS, 20, 12);
+  else
+    go(k_dvc_rounds<2, unsigned>, k_dvc_rounds<2, unsigned long long>, DvcRound<2, unsigned>::BS, 64, 48);
+  UWG_HIP(hipGetLastError());
+  return counts;
 }
 
 long dvc_wave_bound_shorts(int cap) { return 2L * DVCW_MAXNP * cap; }

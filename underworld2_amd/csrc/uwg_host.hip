@@ -82,6 +82,7 @@ struct uwg_swarm {
   double* xi_slot = nullptr;  // [cap][dim]
   double* w_slot = nullptr;   // [cap]
   int* slot_cell = nullptr;   // [cap]
+  int* dvc_work = nullptr;    // element lists of the DVC, [2 E + 4]
   bool has_mat = false;
   bool has_integration = false;
   long state = 0;             // bumps whenever particles or their materials change (assembly cache)
@@ -449,7 +450,7 @@ extern "C" int uwg_swarm_create(uwg_mesh* m, uwg_swarm** out) {
 extern "C" int uwg_swarm_destroy(uwg_swarm* s) {
   if (!s) return 0;
   for (void* p : {(void*)s->coords, (void*)s->owner, (void*)s->cell_ptr, (void*)s->cell_pid, (void*)s->mat,
-                  (void*)s->xi_slot, (void*)s->w_slot, (void*)s->slot_cell})
+                  (void*)s->xi_slot, (void*)s->w_slot, (void*)s->slot_cell, (void*)s->dvc_work})
     dfree(p);
   reloc_destroy(s->reloc);
   for (int v = 0; v < 8; v++) dfree(s->var[v]);
@@ -601,38 +602,51 @@ extern "C" int uwg_swarm_update_owners(uwg_swarm* s, long* outside) {
 static int run_dvc(uwg_swarm* s, int dvc_res) {
   const Geom& g = s->mesh->g;
   const long E = g.E;
+  const auto underresolved = [](long e) {
+    set_error("Problem has an under resolved cell (Cell Id = " + std::to_string(e) +
+              "), add more particles to your model");
+    return UWG_ERR_UNDERRESOLVED;
+  };
+  int dev = 0, cus = 0;
+  UWG_HIP(hipGetDevice(&dev));
+  UWG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  long todo = E;               // elements for the kernels below
+  const int* elist = nullptr;  // their indices (null: all)
+  if (dvc_rounds_supported(dvc_res)) {
+    if (!s->dvc_work) s->dvc_work = dalloc<int>(2 * E + 4);
+    const int* counts = launch_dvc_rounds(g.dim, E, s->cell_ptr, s->xi_slot, s->w_slot, cus, s->dvc_work, 0);
+    int h[3];
+    UWG_HIP(hipMemcpy(h, counts, sizeof(h), hipMemcpyDeviceToHost));
+    if (h[2] != 0x7fffffff) return underresolved(h[2]);
+    if (h[1] == 0) return 0;
+    todo = h[1];
+    elist = s->dvc_work + E;
+  }
   // per-cell counts for capacity planning
   std::vector<int> ptr(E + 1);
   UWG_HIP(hipMemcpy(ptr.data(), s->cell_ptr, sizeof(int) * (E + 1), hipMemcpyDeviceToHost));
   int maxc = 0;
   for (long e = 0; e < E; e++) {
     int c = ptr[e + 1] - ptr[e];
-    if (c == 0) {
-      set_error("Problem has an under resolved cell (Cell Id = " + std::to_string(e) +
-                "), add more particles to your model");
-      return UWG_ERR_UNDERRESOLVED;
-    }
+    if (c == 0) return underresolved(e);
     maxc = std::max(maxc, c);
   }
   const int ncell = dvc_res * dvc_res * (g.dim == 3 ? dvc_res : 1);
   std::vector<int> retry;
   if (dvc_wave_supported(g.dim, dvc_res)) {
     // one wavefront per element; elements it cannot hold are flagged for the per-thread kernel
-    hipDeviceProp_t prop;
-    int dev = 0;
-    UWG_HIP(hipGetDevice(&dev));
-    UWG_HIP(hipGetDeviceProperties(&prop, dev));
     const int cap = std::min(512, ncell);
     // 16 workgroups per CU (19 fit in LDS; measured per pass at 128^3: 12 -> 659 ms, 16 -> 559 ms,
     // 19 -> 684 ms)
-    const int nblk = (int)std::min<long>(E, (long)prop.multiProcessorCount * 16);
+    const int nblk = (int)std::min<long>(todo, (long)cus * 16);
     short* gb = dalloc<short>(dvc_wave_bound_shorts(cap) * nblk);
-    int* flag = dalloc<int>(E);
-    launch_dvc_wave(g.dim, dvc_res, E, s->cell_ptr, s->xi_slot, s->w_slot, gb, nblk, cap, flag, 0);
-    std::vector<int> hflag(E);
-    UWG_HIP(hipMemcpy(hflag.data(), flag, sizeof(int) * E, hipMemcpyDeviceToHost));
-    for (long e = 0; e < E; e++)
-      if (hflag[e]) retry.push_back((int)e);
+    int* flag = dalloc<int>(todo);
+    launch_dvc_wave(g.dim, dvc_res, todo, elist, s->cell_ptr, s->xi_slot, s->w_slot, gb, nblk, cap, flag, 0);
+    std::vector<int> hflag(todo), el(elist ? todo : 0);
+    UWG_HIP(hipMemcpy(hflag.data(), flag, sizeof(int) * todo, hipMemcpyDeviceToHost));
+    if (elist) UWG_HIP(hipMemcpy(el.data(), elist, sizeof(int) * todo, hipMemcpyDeviceToHost));
+    for (long t = 0; t < todo; t++)
+      if (hflag[t]) retry.push_back(elist ? el[t] : (int)t);
     dfree(gb);
     dfree(flag);
   } else {

@@ -137,8 +137,11 @@ void launch_fn_eval(const Geom& g, long P, const double* coords, const int* mat,
                     double* force, int* err, hipStream_t s);
 void launch_field_interpolate(const Geom& g, long P, const double* f, int nc, const double* x, double* v, int* ok,
                               hipStream_t s);
-void launch_dvc_wave(int dim, int num, long E, const int* cell_ptr, double* xi_slot, double* w_slot, short* gbound,
-                     int nblk, int cap, int* flag, hipStream_t s);
+void launch_dvc_wave(int dim, int num, long nE, const int* elist, const int* cell_ptr, double* xi_slot, double* w_slot,
+                     short* gbound, int nblk, int cap, int* flag, hipStream_t s);
+bool dvc_rounds_supported(int num);
+int* launch_dvc_rounds(int dim, long E, const int* cell_ptr, double* xi_slot, double* w_slot, int cus, int* work,
+                       hipStream_t s);
 void launch_dvc_list(int dim, int num, long E0, long nE, const int* elist, const int* cell_ptr,
                      double* xi_slot, double* w_slot, void* scratch, int max_np, int cap, int* d_flag,
                      hipStream_t s);
