@@ -19,7 +19,8 @@
 // 125 (3D) or 5 x 25 (2D) quadrature points for the gradient/stress pass and to the 81 (3D)
 // or 5 x 18 (2D) element dofs for the transposed pass; elements of one parity class
 // ("colour") share no vertex, so 2^dim launches accumulate into y without atomics and in a
-// fixed order (deterministic).
+// fixed order (deterministic).  The default 3D kernels instead write element results and sum
+// them per vertex, in the same order.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -408,6 +409,11 @@ void q2_mfma_matrix(const Geom& g, std::vector<double>& D) {
   }
 }
 
+// 3D apply kernel: 2 sum-factorised (default), 1 matrix cores, 0 dense vector kernel
+static int g_q2_kernel = 2;
+void set_q2_mfma(int on) { g_q2_kernel = on ? 1 : 0; }
+void set_q2_apply_kernel(int kind) { g_q2_kernel = kind; }
+
 // ---------------------------------------------------------------------------------------
 // Sum-factorised 3D apply.  On the tensor 3 x 3 x 3 element and the 5 x 5 x 5 Gauss rule every
 // shape-function derivative factorises into 1D tables, B[m][a] = phi_a(g_m) and
@@ -415,160 +421,327 @@ void q2_mfma_matrix(const Geom& g, std::vector<double>& D) {
 // passes of 1D contractions (x, then y, then z; 2,070 multiply-adds per velocity component
 // instead of 27 x 125 x 3) and the transposed contraction the same passes in reverse: 12,420
 // multiply-adds, about 27 kflop per element with the pointwise stress, against 121.5 kflop for
-// the dense contraction.  Five elements per 128-lane workgroup; the x and y passes and their
-// transposes are spread over the lanes through LDS, each lane (element, qx, qy) runs the
-// z pass, the stress at its five points and the transposed z pass in registers.  Elements of
-// one parity class share no vertex, so the colour launches add into y without atomics.
+// the dense contraction.
+//
+// k_q2_elem writes each element's 81 results to `ye`; k_q2_nodes adds those of a vertex's
+// elements up and finishes the row (Dirichlet rows, residual, smoother step).  Elements of one
+// parity class share no vertex and could add into y directly, eight launches one after the
+// other; but a class of 24^3 elements is 346 workgroups of mostly latency: 20.7 us each, 186 us
+// with the clearing of y, the residual and the smoother step, against 14.5 + 7.7 us for the two
+// kernels here (48^3 in double precision: 51 + 12 us).  The sum over a vertex's elements keeps the
+// order of the classes.
+//
+// Half a wave per element and no barriers: 27 lanes run the x lines and their transposes, 25
+// lanes the (qx, qy) columns - y pass, z pass, stress at the five points, transposed z pass in
+// registers - and 45 tasks in two passes the transposed y lines; the passes exchange through the
+// half wave's own 676 words of LDS.  Bound by instruction issue, about 450 vector instructions
+// per element.
 // ---------------------------------------------------------------------------------------
-constexpr int Q2S_E = 5;
-
 template <typename T>
-__global__ __launch_bounds__(128) void k_q2_apply_sf(Q2G G, int cx, int cy, int cz, int ncx, int ncy, long nce,
-                                                     const T* __restrict__ W, const T* __restrict__ x,
-                                                     T* __restrict__ y, const uint8_t* __restrict__ bc) {
-  __shared__ T xs[Q2S_E][81];        // u[(ax + 3 ay + 9 az) * 3 + i]
-  __shared__ T U[Q2S_E][2][5][27];   // x pass [B|D][qx][(ay + 3 az) * 3 + i]; reused for the y^T pass
-  __shared__ T A[Q2S_E][25][27];     // after the z^T pass, per (qx, qy): [path * 9 + az * 3 + i]
-  __shared__ T tb[3][5][3];          // B, D * (2/h_x), D * (2/h_y); D * (2/h_z) is formed in the z pass
-  const int t = threadIdx.x;
-  const long ce0 = (long)blockIdx.x * Q2S_E;
-  auto elem_of = [&](long ce) -> long {
-    const int i = cx + 2 * (int)(ce % ncx), j = cy + 2 * (int)((ce / ncx) % ncy);
-    const int k = cz + 2 * (int)(ce / ((long)ncx * ncy));
-    return i + (long)G.rx * (j + (long)G.ry * k);
-  };
-  if (t < 15) {
-    const int m = t / 3, a = t % 3;
-    tb[0][m][a] = (T)ph(a, g5(m));
-    tb[1][m][a] = (T)dph(a, g5(m)) * (T)G.s[0];
-    tb[2][m][a] = (T)dph(a, g5(m)) * (T)G.s[1];
-  }
-  // 1. element dofs (Dirichlet dofs read as zero)
-  for (int idx = t; idx < Q2S_E * 81; idx += 128) {
-    const int le = idx / 81, r = idx % 81;
-    T v = (T)0;
-    if (ce0 + le < nce) {
-      const long n = q2_vertex<3>(G, elem_of(ce0 + le), r / 3);
-      const int i = r % 3;
-      const uint8_t m = bc[n];
-      const T xv = x[n * 3 + i];  // loaded unconditionally: the mask does not gate the load
-      v = ((m >> i) & 1) ? (T)0 : xv;
+struct Q2Tab {
+  T B[5][3], D[3][5][3];  // D scaled by 2/h of its axis
+};
+template <typename T>
+static Q2Tab<T> q2_tables(const Q2G& G) {
+  Q2Tab<T> t;
+  for (int m = 0; m < 5; m++)
+    for (int a = 0; a < 3; a++) {
+      t.B[m][a] = (T)ph(a, g5(m));
+      for (int d = 0; d < 3; d++) t.D[d][m][a] = (T)dph(a, g5(m)) * (T)G.s[d];
     }
-    xs[le][r] = v;
+  return t;
+}
+
+// n / d for 0 <= n < 2^31 as (n m) >> s: m = ceil(2^s / d) exceeds 2^s / d by less than
+// 2^(s - 31) / d with s = 31 + ceil(log2 d)
+struct Q2Div {
+  unsigned m;
+  int s, d;
+  explicit Q2Div(int den) : d(den) {
+    s = 31;
+    while ((1L << (s - 31)) < den) s++;
+    m = (unsigned)(((1ull << s) + den - 1) / den);
   }
-  __syncthreads();
-  // 2. x pass: U[v][qx][L*3+i] = sum_ax (B|D)[qx][ax] u[(ax + 3 L) * 3 + i], L = ay + 3 az
-  for (int idx = t; idx < Q2S_E * 270; idx += 128) {
-    const int le = idx / 270, r = idx % 270, v = r / 135, qx = (r % 135) / 27, ln = r % 27;
-    const int L = ln / 3, i = ln % 3;
-    T acc = (T)0;
-#pragma unroll
-    for (int ax = 0; ax < 3; ax++) acc += tb[v][qx][ax] * xs[le][(ax + 3 * L) * 3 + i];
-    U[le][v][qx][ln] = acc;
-  }
-  __syncthreads();
-  // 3. per (element, qx, qy): y pass, z pass, stress at the five points, z^T pass
+  __device__ __forceinline__ int div(int n) const { return (int)(((unsigned long long)(unsigned)n * m) >> s); }
+};
+
+constexpr int Q2S_WORDS = 676;    // exchange area of one element: 25 x 27, to 16 bytes
+constexpr int Q2S_PITCH = 28;     // 27 lanes' results of the x pass, to 16 bytes
+
+// between two passes through a wave's own LDS area: LDS operations of a wave complete in order,
+// the compiler must keep that order
+__device__ __forceinline__ void q2_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// elements of the layers [k0, k0 + nk); layer k is kept in slot k % slots of ye
+template <typename T>
+__global__ __launch_bounds__(256) void k_q2_elem(Q2G G, Q2Tab<T> tab, Q2Div by_rx, Q2Div by_ry, int k0, int nk,
+                                                 int slots, const T* __restrict__ W, const T* __restrict__ x,
+                                                 const uint8_t* __restrict__ bc, T* __restrict__ ye) {
+  __shared__ __align__(16) T lds[8][Q2S_WORDS];
+  const int l = threadIdx.x & 31, layer = G.rx * G.ry, ne = layer * nk;
+  int e = (int)blockIdx.x * 8 + (threadIdx.x >> 5);
+  const bool on = e < ne;
+  if (!on) e = ne - 1;  // same work, no result
+  const int row = by_rx.div(e), ei = e - row * G.rx, ek = by_ry.div(row), ej = row - ek * G.ry;
+  T* X = lds[threadIdx.x >> 5];
+  // the weights of this lane's column
+  const int qq = l < 25 ? l : 24, qx = qq % 5, qy = qq / 5;
+  T w[5];
   {
-    const int le = t / 25, qq = t % 25, qx = qq % 5, qy = qq / 5;
-    if (t < 125 && ce0 + le < nce) {
-      const long e = elem_of(ce0 + le);
-      T Vbb[3][3], Vdb[3][3], Vbd[3][3];  // [az][i]: z-derivative, x-derivative, y-derivative paths
+    const T* Wp = W + ((long)layer * (k0 + ek) + (long)ej * G.rx + ei) * 125 + qq;
 #pragma unroll
-      for (int az = 0; az < 3; az++)
+    for (int qz = 0; qz < 5; qz++) w[qz] = Wp[25 * qz];
+  }
+  // x pass, lane (L = ay + 3 az, component i): B and D of the three dofs of the line
+  {
+    const int ln = l < 27 ? l : 26, L = ln / 3, i = ln % 3;
+    const long n = 2 * ei + (long)G.nx * (2 * ej + L % 3 + (long)G.ny * (2 * (k0 + ek) + L / 3));
+    T u[3];
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-          T bb = (T)0, db = (T)0, bd = (T)0;
+    for (int ax = 0; ax < 3; ax++) {
+      const uint8_t m = bc[n + ax];
+      const T v = x[(n + ax) * 3 + i];  // loaded unconditionally: the mask does not gate the load
+      u[ax] = ((m >> i) & 1) ? (T)0 : v;
+    }
+    if (l < 27) {
 #pragma unroll
-          for (int ay = 0; ay < 3; ay++) {
-            const int ln = (ay + 3 * az) * 3 + i;
-            bb += tb[0][qy][ay] * U[le][0][qx][ln];
-            db += tb[0][qy][ay] * U[le][1][qx][ln];
-            bd += tb[2][qy][ay] * U[le][0][qx][ln];
-          }
-          Vbb[az][i] = bb;
-          Vdb[az][i] = db;
-          Vbd[az][i] = bd;
-        }
-      T A1[3][3], A2[3][3], A3[3][3];
+      for (int q = 0; q < 5; q++) {
+        X[q * Q2S_PITCH + l] = tab.B[q][0] * u[0] + tab.B[q][1] * u[1] + tab.B[q][2] * u[2];
+        X[(5 + q) * Q2S_PITCH + l] = tab.D[0][q][0] * u[0] + tab.D[0][q][1] * u[1] + tab.D[0][q][2] * u[2];
+      }
+    }
+  }
+  q2_wave_sync();
+  // column (qx, qy)
+  T A1[9], A2[9], A3[9];  // [az * 3 + i]
+  {
+    T Vbb[9], Vdb[9], Vbd[9];  // z-derivative, x-derivative, y-derivative paths
+    T by[3], dy[3];
 #pragma unroll
-      for (int az = 0; az < 3; az++)
+    for (int a = 0; a < 3; a++) {
+      by[a] = (T)ph(a, g5(qy));
+      dy[a] = (T)dph(a, g5(qy)) * (T)G.s[1];
+    }
+    T U[Q2S_PITCH];
+    struct __align__(16) Quad { T v[16 / sizeof(T)]; };
+    constexpr int PER = 16 / sizeof(T);
+    auto line = [&](int r) {
+      const Quad* p = reinterpret_cast<const Quad*>(X + r * Q2S_PITCH);
 #pragma unroll
-        for (int i = 0; i < 3; i++) A1[az][i] = A2[az][i] = A3[az][i] = (T)0;
+      for (int k = 0; k < Q2S_PITCH / PER; k++) {
+        const Quad c = p[k];
 #pragma unroll
-      for (int qz = 0; qz < 5; qz++) {
-        T bz[3], dz[3];
+        for (int j = 0; j < PER; j++) U[k * PER + j] = c.v[j];
+      }
+    };
+    line(qx);
 #pragma unroll
-        for (int az = 0; az < 3; az++) {
-          bz[az] = tb[0][qz][az];
-          dz[az] = (T)dph(az, g5(qz)) * (T)G.s[2];
-        }
-        T g[3][3];
+    for (int az = 0; az < 3; az++)
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-          g[i][0] = bz[0] * Vdb[0][i] + bz[1] * Vdb[1][i] + bz[2] * Vdb[2][i];
-          g[i][1] = bz[0] * Vbd[0][i] + bz[1] * Vbd[1][i] + bz[2] * Vbd[2][i];
-          g[i][2] = dz[0] * Vbb[0][i] + dz[1] * Vbb[1][i] + dz[2] * Vbb[2][i];
-        }
-        const T w = W[e * 125 + qx + 5 * qy + 25 * qz];
-        T tau[3][3];
+      for (int i = 0; i < 3; i++) {
+        const int r = 9 * az + i;
+        Vbb[az * 3 + i] = by[0] * U[r] + by[1] * U[r + 3] + by[2] * U[r + 6];
+        Vbd[az * 3 + i] = dy[0] * U[r] + dy[1] * U[r + 3] + dy[2] * U[r + 6];
+      }
+    line(5 + qx);
 #pragma unroll
-        for (int i = 0; i < 3; i++)
+    for (int az = 0; az < 3; az++)
 #pragma unroll
-          for (int j = 0; j < 3; j++) tau[i][j] = w * (g[i][j] + g[j][i]);
-#pragma unroll
-        for (int az = 0; az < 3; az++)
-#pragma unroll
-          for (int i = 0; i < 3; i++) {
-            A1[az][i] += bz[az] * tau[i][0];
-            A2[az][i] += bz[az] * tau[i][1];
-            A3[az][i] += dz[az] * tau[i][2];
-          }
+      for (int i = 0; i < 3; i++) {
+        const int r = 9 * az + i;
+        Vdb[az * 3 + i] = by[0] * U[r] + by[1] * U[r + 3] + by[2] * U[r + 6];
       }
 #pragma unroll
+    for (int k = 0; k < 9; k++) A1[k] = A2[k] = A3[k] = (T)0;
+#pragma unroll
+    for (int qz = 0; qz < 5; qz++) {
+      const T* bz = tab.B[qz];
+      const T* dz = tab.D[2][qz];
+      T g[3][3];
+#pragma unroll
+      for (int i = 0; i < 3; i++) {
+        g[i][0] = bz[0] * Vdb[i] + bz[1] * Vdb[3 + i] + bz[2] * Vdb[6 + i];
+        g[i][1] = bz[0] * Vbd[i] + bz[1] * Vbd[3 + i] + bz[2] * Vbd[6 + i];
+        g[i][2] = dz[0] * Vbb[i] + dz[1] * Vbb[3 + i] + dz[2] * Vbb[6 + i];
+      }
+      T tau[3][3];
+#pragma unroll
+      for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = i; j < 3; j++) tau[i][j] = tau[j][i] = w[qz] * (g[i][j] + g[j][i]);
+#pragma unroll
       for (int az = 0; az < 3; az++)
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-          A[le][qq][0 * 9 + az * 3 + i] = A1[az][i];
-          A[le][qq][1 * 9 + az * 3 + i] = A2[az][i];
-          A[le][qq][2 * 9 + az * 3 + i] = A3[az][i];
+          A1[az * 3 + i] += bz[az] * tau[i][0];
+          A2[az * 3 + i] += bz[az] * tau[i][1];
+          A3[az * 3 + i] += dz[az] * tau[i][2];
         }
     }
   }
-  __syncthreads();
-  // 4. y^T pass: C1[qx][L*3+i] = sum_qy B[qy][ay] A1, C2 = sum_qy (D[qy][ay] A2 + B[qy][ay] A3)
-  for (int idx = t; idx < Q2S_E * 270; idx += 128) {
-    const int le = idx / 270, r = idx % 270, v = r / 135, qx = (r % 135) / 27, ln = r % 27;
-    const int L = ln / 3, i = ln % 3, ay = L % 3, az = L / 3;
-    T acc = (T)0;
+  q2_wave_sync();
+  if (l < 25) {
 #pragma unroll
-    for (int qy = 0; qy < 5; qy++) {
-      const T* a = A[le][qx + 5 * qy];
-      if (v == 0)
-        acc += tb[0][qy][ay] * a[0 * 9 + az * 3 + i];
-      else
-        acc += tb[2][qy][ay] * a[1 * 9 + az * 3 + i] + tb[0][qy][ay] * a[2 * 9 + az * 3 + i];
+    for (int k = 0; k < 9; k++) {
+      X[l * 27 + k] = A1[k];
+      X[l * 27 + 9 + k] = A2[k];
+      X[l * 27 + 18 + k] = A3[k];
     }
-    U[le][v][qx][ln] = acc;
   }
-  __syncthreads();
-  // 5. x^T pass and scatter: y_ai += sum_qx D[qx][ax] C1 + B[qx][ax] C2
-  for (int idx = t; idx < Q2S_E * 81; idx += 128) {
-    const int le = idx / 81, r = idx % 81;
-    if (ce0 + le >= nce) continue;
-    const int a = r / 3, i = r % 3, ax = a % 3, L = a / 3;
-    T acc = (T)0;
+  q2_wave_sync();
+  // transposed y pass, task (qx, c = az * 3 + i): C1 = sum_qy B A1, C2 = sum_qy (D A2 + B A3)
+  T C1[2][3], C2[2][3];
 #pragma unroll
-    for (int qx = 0; qx < 5; qx++)
-      acc += tb[1][qx][ax] * U[le][0][qx][L * 3 + i] + tb[0][qx][ax] * U[le][1][qx][L * 3 + i];
-    const long n = q2_vertex<3>(G, elem_of(ce0 + le), a);
-    if (!((bc[n] >> i) & 1)) y[n * 3 + i] += acc;
+  for (int h = 0; h < 2; h++) {
+    const int task = l + 32 * h < 45 ? l + 32 * h : 44;
+    const T* p = X + (task % 5) * 27 + task / 5;
+#pragma unroll
+    for (int a = 0; a < 3; a++) C1[h][a] = C2[h][a] = (T)0;
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      const T a1 = p[q * 135], a2 = p[q * 135 + 9], a3 = p[q * 135 + 18];
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        C1[h][a] += tab.B[q][a] * a1;
+        C2[h][a] += tab.D[1][q][a] * a2 + tab.B[q][a] * a3;
+      }
+    }
+  }
+  q2_wave_sync();
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const int task = l + 32 * h, c = task / 5;
+    if (task < 45) {
+      T* p = X + (task % 5) * 27 + 9 * (c / 3) + c % 3;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        p[3 * a] = C1[h][a];
+        p[135 + 3 * a] = C2[h][a];
+      }
+    }
+  }
+  q2_wave_sync();
+  // transposed x pass, lane (L, i)
+  if (l < 27 && on) {
+    T s[3] = {(T)0, (T)0, (T)0};
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+      const T c1 = X[q * 27 + l], c2 = X[135 + q * 27 + l];
+#pragma unroll
+      for (int a = 0; a < 3; a++) s[a] += tab.D[0][q][a] * c1 + tab.B[q][a] * c2;
+    }
+    T* o = ye + ((long)layer * ((k0 + ek) % slots) + (long)ej * G.rx + ei) * 81 + 9 * (l / 3) + l % 3;
+#pragma unroll
+    for (int a = 0; a < 3; a++) o[3 * a] = s[a];
   }
 }
 
-// 3D apply kernel: 2 sum-factorised (default), 1 matrix cores, 0 dense vector kernel
-static int g_q2_kernel = 2;
-void set_q2_mfma(int on) { g_q2_kernel = on ? 1 : 0; }
-void set_q2_apply_kernel(int kind) { g_q2_kernel = kind; }
+// the vertices of planes [K0, K1): v = K x on a row (x on Dirichlet rows), then by Q2Op y = v,
+// y = b - v, or the smoother step with the residual r = b - v, d = ca d + cb (dinv r), xo += d
+template <typename T, Q2Op OP>
+__global__ __launch_bounds__(256) void k_q2_nodes(Q2G G, Q2Div by_nx, Q2Div by_ny, int K0, int K1, int slots,
+                                                  const T* __restrict__ ye, const T* x, const uint8_t* __restrict__ bc,
+                                                  Q2Out<T> out) {
+  const int idx = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (idx >= G.nx * G.ny * (K1 - K0)) return;
+  const int row = by_nx.div(idx), I = idx - row * G.nx, kk = by_ny.div(row), J = row - kk * G.ny, K = K0 + kk;
+  const long n = (long)G.nx * G.ny * K0 + idx;
+  // per axis the element of even and of odd index, or -1
+  auto pick = [](int I, int r, int* el) {
+    const int m = I >> 1, lo = (I & 1) ? -1 : m - 1, hi = m < r ? m : -1;
+    el[0] = (m & 1) ? lo : hi;
+    el[1] = (m & 1) ? hi : lo;
+  };
+  int ex[2], ey[2], ez[2];
+  pick(I, G.rx, ex);
+  pick(J, G.ry, ey);
+  pick(K, G.rz, ez);
+  T acc[3] = {(T)0, (T)0, (T)0};
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    if (ez[c] < 0) continue;
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+      if (ey[b] < 0) continue;
+      const long base = (long)G.rx * (ey[b] + (long)G.ry * (ez[c] % slots));
+      const int loc = 3 * (J - 2 * ey[b]) + 9 * (K - 2 * ez[c]);
+#pragma unroll
+      for (int a = 0; a < 2; a++) {
+        if (ex[a] < 0) continue;
+        const T* p = ye + (base + ex[a]) * 81 + (loc + I - 2 * ex[a]) * 3;
+#pragma unroll
+        for (int d = 0; d < 3; d++) acc[d] += p[d];
+      }
+    }
+  }
+  const uint8_t m = bc[n];
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const long i = n * 3 + d;
+    const T v = ((m >> d) & 1) ? x[i] : acc[d];
+    if constexpr (OP == Q2Op::apply) {
+      out.y[i] = v;
+    } else if constexpr (OP == Q2Op::residual) {
+      out.y[i] = out.b[i] - v;
+    } else {
+      const T r = out.b[i] - v;
+      const T dd = out.ca * out.d[i] + out.cb * (out.dinv[i] * r);
+      out.d[i] = dd;
+      out.x[i] += dd;
+    }
+  }
+}
+
+// Layers of element results kept at a time: all of them up to 32 MiB (47^3 elements in single
+// precision), else a ring of at least two.  A pass over the layers [k0, k1) finishes the vertex
+// planes below 2 k1 and leaves layer k1 - 1 in the ring for the plane shared with the next pass;
+// the layers after it read no plane that a smoother step has written yet.
+template <typename T>
+static int q2_slots(const Geom& g) {
+  const long layer = (long)g.res[0] * g.res[1] * 81 * (long)sizeof(T);
+  const long fit = (32L << 20) / layer;
+  return (int)std::min<long>(g.res[2], std::max<long>(2, fit));
+}
+bool q2_apply_fused(const Geom& g) {
+  return g.dim == 3 && g_q2_kernel == 2;
+}
+template <typename T>
+long q2_apply_scratch(const Geom& g) {
+  return (long)g.res[0] * g.res[1] * 81 * q2_slots<T>(g);
+}
+template long q2_apply_scratch<double>(const Geom&);
+template long q2_apply_scratch<float>(const Geom&);
+
+template <typename T>
+void launch_q2_apply_sf(const Geom& g, const T* W, const T* x, const uint8_t* bc, T* ye, Q2Op op, const Q2Out<T>& out,
+                        hipStream_t s) {
+  const Q2G G = q2_pack(g);
+  const Q2Tab<T> tab = q2_tables<T>(G);
+  const Q2Div rx(G.rx), ry(G.ry), nx(G.nx), ny(G.ny);
+  const int slots = q2_slots<T>(g), step = slots == G.rz ? G.rz : slots - 1;
+  for (int k0 = 0; k0 < G.rz; k0 += step) {
+    const int nk = std::min(step, G.rz - k0), K0 = 2 * k0, K1 = k0 + nk == G.rz ? G.nz : 2 * (k0 + nk);
+    hipLaunchKernelGGL((k_q2_elem<T>), q2_blocks((long)G.rx * G.ry * nk, 8), 256, 0, s, G, tab, rx, ry, k0, nk, slots, W,
+                       x, bc, ye);
+    UWG_HIP(hipGetLastError());
+    const unsigned nb = q2_blocks((long)G.nx * G.ny * (K1 - K0), 256);
+    if (op == Q2Op::apply)
+      hipLaunchKernelGGL((k_q2_nodes<T, Q2Op::apply>), nb, 256, 0, s, G, nx, ny, K0, K1, slots, ye, x, bc, out);
+    else if (op == Q2Op::residual)
+      hipLaunchKernelGGL((k_q2_nodes<T, Q2Op::residual>), nb, 256, 0, s, G, nx, ny, K0, K1, slots, ye, x, bc, out);
+    else
+      hipLaunchKernelGGL((k_q2_nodes<T, Q2Op::smooth>), nb, 256, 0, s, G, nx, ny, K0, K1, slots, ye, x, bc, out);
+    UWG_HIP(hipGetLastError());
+  }
+}
+template void launch_q2_apply_sf<double>(const Geom&, const double*, const double*, const uint8_t*, double*, Q2Op,
+                                         const Q2Out<double>&, hipStream_t);
+template void launch_q2_apply_sf<float>(const Geom&, const float*, const float*, const uint8_t*, float*, Q2Op,
+                                        const Q2Out<float>&, hipStream_t);
 
 // ---------------------------------------------------------------------------------------
 // matrix-free K apply
@@ -720,10 +893,7 @@ void launch_q2_apply(const Geom& g, const T* W, const T* x, T* y, const uint8_t*
     const int ncx = (G.rx - cx + 1) / 2, ncy = (G.ry - cy + 1) / 2, ncz = g.dim == 3 ? (G.rz - cz + 1) / 2 : 1;
     const long nce = (long)ncx * ncy * ncz;
     if (nce == 0) continue;
-    if (g.dim == 3 && g_q2_kernel == 2) {
-      hipLaunchKernelGGL((k_q2_apply_sf<T>), q2_blocks(nce, Q2S_E), 128, 0, s, G, cx, cy, cz, ncx, ncy, nce, W, x, y,
-                         bc);
-    } else if (g.dim == 3 && Dm && g_q2_kernel == 1) {
+    if (g.dim == 3 && Dm && g_q2_kernel == 1) {
       const long nbatch = (nce + Q2M_E - 1) / Q2M_E;
       if (sizeof(T) == 4 && nbatch >= 2L * 2048) {
         // persistent blocks (2+ batches each) keep their slice of D in registers
@@ -826,23 +996,36 @@ __global__ void k_q2_apply_G(Q2G G, const double* __restrict__ Gr, const T* __re
   for (int d = 0; d < DIM; d++) y[n * DIM + d] = ((m >> d) & 1) ? (T)0 : acc[d];
 }
 
+// One lane per vertex of an element (32 or 16 lanes per element), then the lanes' shares are
+// summed.  Bound by latency: one thread per element had 81 dependent multiply-adds on each of its
+// four sums and 108 workgroups at 24^3 elements, GT_MEASURED.
 template <typename T, int DIM>
-__global__ void k_q2_apply_GT(Q2G G, const double* __restrict__ Gr, const T* __restrict__ u,
-                              const uint8_t* __restrict__ bc, T* __restrict__ q) {
-  constexpr int NP = DIM + 1, NEN = DIM == 3 ? 27 : 9;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= G.E) return;
+__global__ __launch_bounds__(256) void k_q2_apply_GT(Q2G G, Q2Div by_rx, Q2Div by_ry, const double* __restrict__ Gr,
+                                                     const T* __restrict__ u, const uint8_t* __restrict__ bc,
+                                                     T* __restrict__ q) {
+  constexpr int NP = DIM + 1, NEN = DIM == 3 ? 27 : 9, LANES = DIM == 3 ? 32 : 16;
+  const long e0 = (long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+  const int e = (int)(e0 < G.E ? e0 : G.E - 1), l = threadIdx.x % LANES, a = l < NEN ? l : NEN - 1;
+  const int row = by_rx.div(e), i = e - row * G.rx, k = DIM == 3 ? by_ry.div(row) : 0, j = row - k * G.ry;
+  const long n = 2 * i + a % 3 + (long)G.nx * (2 * j + (a / 3) % 3 + (long)G.ny * (DIM == 3 ? 2 * k + a / 9 : 0));
+  const uint8_t m = bc[n];
   T acc[4] = {0, 0, 0, 0};
-  for (int a = 0; a < NEN; a++) {
-    const long n = q2_vertex<DIM>(G, e, a);
-    const uint8_t m = bc[n];
-    for (int d = 0; d < DIM; d++) {
-      if ((m >> d) & 1) continue;
-      const T v = u[n * DIM + d];
-      for (int r = 0; r < NP; r++) acc[r] += (T)Gr[(a * DIM + d) * NP + r] * v;
-    }
+#pragma unroll
+  for (int d = 0; d < DIM; d++) {
+    const T v = u[n * DIM + d];  // loaded unconditionally: the mask does not gate the load
+    const T f = l < NEN && !((m >> d) & 1) ? v : (T)0;
+#pragma unroll
+    for (int r = 0; r < NP; r++) acc[r] += (T)Gr[(a * DIM + d) * NP + r] * f;
   }
-  for (int r = 0; r < NP; r++) q[e * NP + r] = acc[r];
+  // lanes 4 k + c collect component c
+  const bool odd = l & 1, high = l & 2;
+  T p0 = odd ? acc[1] : acc[0], p1 = odd ? acc[3] : acc[2];
+  p0 += __shfl_xor(odd ? acc[0] : acc[1], 1);
+  p1 += __shfl_xor(odd ? acc[2] : acc[3], 1);
+  T s = (high ? p1 : p0) + __shfl_xor(high ? p0 : p1, 2);
+#pragma unroll
+  for (int o = 4; o < LANES; o <<= 1) s += __shfl_xor(s, o);
+  if (l < NP && e0 < G.E) q[(long)e * NP + l] = s;
 }
 
 template <typename T>
@@ -858,9 +1041,9 @@ template <typename T>
 void launch_q2_apply_GT(const Geom& g, const double* Gr, const T* u, const uint8_t* bc, T* q, hipStream_t s) {
   const Q2G G = q2_pack(g);
   if (g.dim == 3)
-    hipLaunchKernelGGL((k_q2_apply_GT<T, 3>), q2_blocks(G.E, 128), 128, 0, s, G, Gr, u, bc, q);
+    hipLaunchKernelGGL((k_q2_apply_GT<T, 3>), q2_blocks(G.E, 8), 256, 0, s, G, Q2Div(G.rx), Q2Div(G.ry), Gr, u, bc, q);
   else
-    hipLaunchKernelGGL((k_q2_apply_GT<T, 2>), q2_blocks(G.E, 128), 128, 0, s, G, Gr, u, bc, q);
+    hipLaunchKernelGGL((k_q2_apply_GT<T, 2>), q2_blocks(G.E, 16), 256, 0, s, G, Q2Div(G.rx), Q2Div(G.ry), Gr, u, bc, q);
   UWG_HIP(hipGetLastError());
 }
 template void launch_q2_apply_G<double>(const Geom&, const double*, const double*, const uint8_t*, double*, hipStream_t);

@@ -448,7 +448,7 @@ __global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)
   // in use), failures noticed while examining and while spreading
   __shared__ int n_cell[2], n_claim[2], bad_exam, bad_spread;
   unsigned char* own = own_ + D::GUARD;
-  const int tid = threadIdx.x, lane = tid & 63, wave0 = tid & ~63;
+  const int tid = threadIdx.x, lane = tid & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   const double dx = (1.0 - -1.0) / kDvcNum, dy = dx, dz = dx;
   const long n_el = WIDE ? (long)counts[0] : E;

@@ -42,7 +42,7 @@ enum WsSlot {
   WS_BLK_B, WS_BLK_X, WS_BLK_DS, WS_BLK_Q, WS_BLK_GP, WS_BLK_RP,
   WS_SCH_USTAR, WS_SCH_HHAT, WS_SCH_T, WS_SCH_Z, WS_SCH_DS,
   WS_MIX_B, WS_MIX_X, WS_MIX_R, WS_MIX_GP, WS_MIX_R32, WS_MIX_D32, WS_MIX_DS32, WS_MIX_Q32, WS_MIX_GP32,
-  WS_Q2_ETAG, WS_Q2_FORCEG, WS_Q2_BAD, WS_COARSE_WORK,
+  WS_Q2_ETAG, WS_Q2_FORCEG, WS_Q2_BAD, WS_Q2_ELEM, WS_COARSE_WORK,
   WS_COUNT
 };
 static double now() {
@@ -1376,11 +1376,26 @@ static const T* top_stencil(uwg_stokes* st, const uint8_t* bc) {
   return bc == st->L[0].bc ? LV<T>::S(st->L[0]) : nullptr;
 }
 
+// K on the Q2 level with the row operation `op`; out.y is written by kernels that have no fused
+// row operation also for the smoother step
+template <typename T>
+static void q2_K(uwg_stokes* st, const T* x, const uint8_t* bc, Q2Op op, const Q2Out<T>& out) {
+  Q2Level& A = *st->q2;
+  if (q2_apply_fused(st->g)) {
+    T* ye = wsbuf<T>(st, WS_Q2_ELEM, q2_apply_scratch<T>(st->g));
+    launch_q2_apply_sf<T>(st->g, Q2V<T>::W(A), x, bc, ye, op, out, 0);
+    return;
+  }
+  launch_q2_apply<T>(st->g, Q2V<T>::W(A), x, out.y, bc, 0, Q2V<T>::D(A));
+  if (op != Q2Op::apply) vk_residual<T>(A.n(), out.b, out.y, 0);
+  if (op == Q2Op::smooth) vk_cheb_update<T>(A.n(), out.ca, out.cb, out.dinv, out.y, out.d, out.x, 0);
+}
+
 // K on the finest level; bc selects the Dirichlet rows/columns (identity rows)
 template <typename T>
 static void top_K(uwg_stokes* st, const T* x, T* y, const uint8_t* bc) {
   if (st->q2)
-    launch_q2_apply<T>(st->g, Q2V<T>::W(*st->q2), x, y, bc, 0, Q2V<T>::D(*st->q2));
+    q2_K<T>(st, x, bc, Q2Op::apply, Q2Out<T>{y});
   else
     launch_apply_K<T>(st->g, LV<T>::W(st->L[0]), x, y, bc, 0, nullptr, top_stencil<T>(st, bc));
 }
@@ -1445,15 +1460,14 @@ static void q2_chebyshev(uwg_stokes* st, const T* b, T* x, int degree, bool zero
     k0 = 1;
   }
   for (int k = k0; k < degree; k++) {
-    top_K<T>(st, x, r, A.bc);
-    vk_residual<T>(n, b, r, 0);
-    if (!zero_guess && k == 0) {
-      vk_cheb_update<T>(n, (T)0, (T)(1.0 / theta), dinv, r, d, x, 0);
-    } else {
+    T ca = (T)0, cb = (T)(1.0 / theta);
+    if (zero_guess || k > 0) {
       const double rho_new = 1.0 / (2.0 * sigma - rho);
-      vk_cheb_update<T>(n, (T)(rho_new * rho), (T)(2.0 * rho_new / delta), dinv, r, d, x, 0);
+      ca = (T)(rho_new * rho);
+      cb = (T)(2.0 * rho_new / delta);
       rho = rho_new;
     }
+    q2_K<T>(st, x, A.bc, Q2Op::smooth, Q2Out<T>{r, b, dinv, d, x, ca, cb});
   }
 }
 
@@ -1466,8 +1480,7 @@ static void q2_vcycle(uwg_stokes* st, const T* b, T* x) {
   Level& C = st->L[0];
   q2_chebyshev<T>(st, b, x, g_smooth_degree, true);
   T* r = Q2V<T>::r(A);
-  top_K<T>(st, x, r, A.bc);
-  vk_residual<T>(A.n(), b, r, 0);
+  q2_K<T>(st, x, A.bc, Q2Op::residual, Q2Out<T>{r, b});
   launch_restrict2<T>(A.gn, C.g, r, LV<T>::b(C), C.bc, A.bc, 0);
   vcycle<T>(st, 0, LV<T>::b(C), LV<T>::x(C));
   launch_prolong_add<T>(A.gn, C.g, LV<T>::x(C), x, A.bc, 0);

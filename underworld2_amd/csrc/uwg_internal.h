@@ -173,6 +173,23 @@ void launch_q2_gather_f(const Geom& g, const double* fe, const uint8_t* bc, doub
 template <typename T>
 void launch_q2_apply(const Geom& g, const T* W, const T* x, T* y, const uint8_t* bc, hipStream_t s,
                      const T* Dm = nullptr);  // Dm: [32][384] derivative matrix -> matrix-core path (3D)
+// the sum-factorised 3D apply (the default kernel) with what is done with a row v = (K x)_i:
+// y = v, y = b - v, or the smoother step d = ca d + cb (dinv (b - v)), x += d (x may be the
+// vector applied to).  ye holds q2_apply_scratch elements.
+enum class Q2Op { apply, residual, smooth };
+template <typename T>
+struct Q2Out {
+  T* y;
+  const T *b, *dinv;
+  T *d, *x;
+  T ca, cb;
+};
+bool q2_apply_fused(const Geom& g);
+template <typename T>
+long q2_apply_scratch(const Geom& g);
+template <typename T>
+void launch_q2_apply_sf(const Geom& g, const T* W, const T* x, const uint8_t* bc, T* ye, Q2Op op, const Q2Out<T>& out,
+                        hipStream_t s);
 void q2_mfma_matrix(const Geom& g, std::vector<double>& D);
 void set_q2_mfma(int on);
 void set_q2_apply_kernel(int kind);
