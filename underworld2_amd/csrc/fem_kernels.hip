@@ -1650,7 +1650,9 @@ struct GeConst {
   double v[24];
 };
 
-template <typename T, int DIM>
+// y = G p, or with ADD y += G p (the pressure part of the coupled operator without a vector of its
+// own and a pass to add it)
+template <typename T, int DIM, bool ADD>
 __global__ void k_apply_G(int rx, int ry, int rz, long N, GeConst Ge, const T* __restrict__ p,
                           const uint8_t* __restrict__ bc, T* __restrict__ y) {
   long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1669,12 +1671,18 @@ __global__ void k_apply_G(int rx, int ry, int rz, long N, GeConst Ge, const T* _
         for (int d = 0; d < DIM; d++) acc[d] += (T)Ge.v[a * DIM + d] * pe;
       }
   uint8_t m = bc[n];
-  for (int d = 0; d < DIM; d++) y[n * DIM + d] = ((m >> d) & 1) ? (T)0 : acc[d];
+  for (int d = 0; d < DIM; d++) {
+    const T v = ((m >> d) & 1) ? (T)0 : acc[d];
+    y[n * DIM + d] = ADD ? y[n * DIM + d] + v : v;
+  }
 }
 
-template <typename T, int DIM>
+// q = G^T u; OP 1: q = r - G^T u; OP 2: q = s (r - G^T u), the diagonal Schur block.  One pass in
+// the place of up to four over the pressures; r may be narrower (an Arnoldi vector).
+template <typename T, int DIM, int OP, typename TR>
 __global__ void k_apply_GT(int rx, int ry, int rz, long E, GeConst Ge, const T* __restrict__ u,
-                           const uint8_t* __restrict__ bc, T* __restrict__ q) {
+                           const uint8_t* __restrict__ bc, const TR* __restrict__ r, const T* __restrict__ s,
+                           T* __restrict__ q) {
   long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= E) return;
   long nx = rx + 1, ny = ry + 1;
@@ -1699,131 +1707,176 @@ __global__ void k_apply_GT(int rx, int ry, int rz, long E, GeConst Ge, const T* 
       const T t = (T)Ge.v[a * DIM + d] * uv[a][d];
       acc = ((m[a] >> d) & 1) ? acc : acc + t;
     }
+  if constexpr (OP > 0) acc = (T)r[e] - acc;
+  if constexpr (OP > 1) acc = s[e] * acc;
   q[e] = acc;
 }
 
-template <typename T>
-void launch_apply_G(const Geom& g, const double* Ge, const T* p, const uint8_t* bc, T* y, hipStream_t s) {
+static GeConst ge_const(const Geom& g, const double* Ge) {
   GeConst G;
   for (int q = 0; q < 24; q++) G.v[q] = q < (1 << g.dim) * g.dim ? Ge[q] : 0.0;
-  if (g.dim == 3)
-    hipLaunchKernelGGL((k_apply_G<T, 3>), nblocks(g.N, 256), 256, 0, s, g.res[0], g.res[1], g.res[2], g.N, G, p, bc, y);
-  else
-    hipLaunchKernelGGL((k_apply_G<T, 2>), nblocks(g.N, 256), 256, 0, s, g.res[0], g.res[1], 1, g.N, G, p, bc, y);
-  UWG_HIP(hipGetLastError());
+  return G;
 }
 
 template <typename T>
-void launch_apply_GT(const Geom& g, const double* Ge, const T* u, const uint8_t* bc, T* q, hipStream_t s) {
-  GeConst G;
-  for (int k = 0; k < 24; k++) G.v[k] = k < (1 << g.dim) * g.dim ? Ge[k] : 0.0;
+void launch_apply_G(const Geom& g, const double* Ge, const T* p, const uint8_t* bc, T* y, bool add, hipStream_t s) {
+  const GeConst G = ge_const(g, Ge);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, nblocks(g.N, 256), 256, 0, s, g.res[0], g.res[1], g.dim == 3 ? g.res[2] : 1, g.N, G, p,
+                       bc, y);
+  };
   if (g.dim == 3)
-    hipLaunchKernelGGL((k_apply_GT<T, 3>), nblocks(g.E, 256), 256, 0, s, g.res[0], g.res[1], g.res[2], g.E, G, u, bc, q);
+    add ? go(k_apply_G<T, 3, true>) : go(k_apply_G<T, 3, false>);
   else
-    hipLaunchKernelGGL((k_apply_GT<T, 2>), nblocks(g.E, 256), 256, 0, s, g.res[0], g.res[1], 1, g.E, G, u, bc, q);
+    add ? go(k_apply_G<T, 2, true>) : go(k_apply_G<T, 2, false>);
   UWG_HIP(hipGetLastError());
 }
-template void launch_apply_G<double>(const Geom&, const double*, const double*, const uint8_t*, double*, hipStream_t);
-template void launch_apply_G<float>(const Geom&, const double*, const float*, const uint8_t*, float*, hipStream_t);
-template void launch_apply_GT<double>(const Geom&, const double*, const double*, const uint8_t*, double*, hipStream_t);
-template void launch_apply_GT<float>(const Geom&, const double*, const float*, const uint8_t*, float*, hipStream_t);
+
+template <typename T, typename TR>
+void launch_apply_GT(const Geom& g, const double* Ge, const T* u, const uint8_t* bc, T* q, hipStream_t s, const TR* r,
+                     const T* scale) {
+  const GeConst G = ge_const(g, Ge);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, nblocks(g.E, 256), 256, 0, s, g.res[0], g.res[1], g.dim == 3 ? g.res[2] : 1, g.E, G, u,
+                       bc, r, scale, q);
+  };
+  if (g.dim == 3)
+    !r ? go(k_apply_GT<T, 3, 0, TR>) : scale ? go(k_apply_GT<T, 3, 2, TR>) : go(k_apply_GT<T, 3, 1, TR>);
+  else
+    !r ? go(k_apply_GT<T, 2, 0, TR>) : scale ? go(k_apply_GT<T, 2, 2, TR>) : go(k_apply_GT<T, 2, 1, TR>);
+  UWG_HIP(hipGetLastError());
+}
+template void launch_apply_G<double>(const Geom&, const double*, const double*, const uint8_t*, double*, bool,
+                                     hipStream_t);
+template void launch_apply_G<float>(const Geom&, const double*, const float*, const uint8_t*, float*, bool,
+                                    hipStream_t);
+template void launch_apply_GT<double, double>(const Geom&, const double*, const double*, const uint8_t*, double*,
+                                              hipStream_t, const double*, const double*);
+template void launch_apply_GT<double, float>(const Geom&, const double*, const double*, const uint8_t*, double*,
+                                             hipStream_t, const float*, const double*);
+template void launch_apply_GT<float, float>(const Geom&, const double*, const float*, const uint8_t*, float*,
+                                            hipStream_t, const float*, const float*);
 
 // ---------------------------------------------------------------------------------------
 // Transfer operators: trilinear prolongation (a fine node averages its 1, 2, 4 or 8
 // coarse parents, SROpGenerator.c:748-1052) and its transpose.  Dirichlet dofs are
 // excluded on both levels.
 // ---------------------------------------------------------------------------------------
+// One thread per dof: on the small grids both kernels are bound by the latency of a few workgroups'
+// dependent loads, and a thread per vertex with three components made a third as many.  Restriction
+// to 17 x 13 x 21 vertices in double precision 13.7 -> 3.6 us including the first smoothing step
+// (a pass of 4.0 us before), to 17^3 in single 4.4 + 2.4 -> 3.6 us; 33^3 prolongation 3.9 -> 2.8 us.
 template <typename T, int DIM>
-__global__ void k_prolong_add(int fnx, int fny, int fnz, int cnx, int cny, long Nf, const T* __restrict__ xc,
-                              T* __restrict__ xf, const uint8_t* __restrict__ bcf) {
-  long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= Nf) return;
-  int I = (int)(n % fnx), J = (int)((n / fnx) % fny), K = (int)(n / ((long)fnx * fny));
-  T acc[3] = {0, 0, 0};
-  int ni = (I & 1) ? 2 : 1, nj = (J & 1) ? 2 : 1, nk = DIM == 3 ? ((K & 1) ? 2 : 1) : 1;
-  T wgt = (T)1;
-  if (I & 1) wgt *= (T)0.5;
-  if (J & 1) wgt *= (T)0.5;
-  if (DIM == 3 && (K & 1)) wgt *= (T)0.5;
-  for (int c = 0; c < nk; c++)
-    for (int b = 0; b < nj; b++)
-      for (int a = 0; a < ni; a++) {
-        int ci = (I >> 1) + a, cj = (J >> 1) + b, ck = DIM == 3 ? (K >> 1) + c : 0;
-        long cn = ci + (long)cnx * (cj + (long)cny * ck);
-        for (int d = 0; d < DIM; d++) acc[d] += xc[cn * DIM + d];
-      }
-  // the mask and the old values load independently of each other; a Dirichlet dof is
-  // rewritten with its own value
+__global__ __launch_bounds__(128) void k_prolong_add(int fnx, int fny, int cnx, int cny, unsigned nf,
+                                                     const T* __restrict__ xc, T* __restrict__ xf,
+                                                     const uint8_t* __restrict__ bcf) {
+  const long idx = (long)blockIdx.x * 128 + threadIdx.x;
+  if (idx >= (long)nf * DIM) return;
+  const unsigned n = (unsigned)(idx / DIM), row = n / fnx;
+  const int d = (int)(idx - (long)n * DIM), I = (int)(n % fnx), J = (int)(row % fny), K = (int)(row / fny);
+  // the mask and the old value load independently of the parents; a Dirichlet dof is rewritten
+  // with its own value
   const uint8_t m = bcf[n];
-  T old[3];
-  for (int d = 0; d < DIM; d++) old[d] = xf[n * DIM + d];
-  for (int d = 0; d < DIM; d++) xf[n * DIM + d] = ((m >> d) & 1) ? old[d] : old[d] + wgt * acc[d];
+  const T old = xf[idx];
+  // all parents load at once; on an even index both are the same one, which counts once
+  constexpr int NK = DIM == 3 ? 2 : 1;
+  const int odd[3] = {I & 1, J & 1, K & 1};
+  T v[4 * NK];
+#pragma unroll
+  for (int q = 0; q < 4 * NK; q++) {
+    const long ci = (I >> 1) + (q & odd[0]), cj = (J >> 1) + ((q >> 1) & odd[1]), ck = (K >> 1) + ((q >> 2) & odd[2]);
+    v[q] = xc[(ci + cnx * (cj + (DIM == 3 ? cny * ck : 0))) * DIM + d];
+  }
+  T acc = 0, wgt = (T)1;
+#pragma unroll
+  for (int q = 0; q < 4 * NK; q++)
+    acc = ((q & 1) > odd[0] || ((q >> 1) & 1) > odd[1] || (DIM == 3 && ((q >> 2) & 1) > odd[2])) ? acc : acc + v[q];
+  if (odd[0]) wgt *= (T)0.5;
+  if (odd[1]) wgt *= (T)0.5;
+  if (DIM == 3 && odd[2]) wgt *= (T)0.5;
+  xf[idx] = ((m >> d) & 1) ? old : old + wgt * acc;
 }
 
-template <typename T, int DIM>
-__global__ void k_restrict(int fnx, int fny, int fnz, int cnx, int cny, int cnz, long Nc, const T* __restrict__ rf,
-                           T* __restrict__ rc, const uint8_t* __restrict__ bcc, const uint8_t* __restrict__ bcf) {
-  long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= Nc) return;
-  int i = (int)(n % cnx), j = (int)((n / cnx) % cny), k = (int)(n / ((long)cnx * cny));
-  T acc[3] = {0, 0, 0};
-  // every fine value and mask is loaded unconditionally (out-of-grid neighbours read node 0
-  // and are skipped by the select), so no load waits on a mask byte
+// OP 1: also the first smoothing step on the coarse level, dd = x = c dinv b (k_cheb_first);
+// OP 2: also the value widened to `wide` (the coarsest level's solve)
+template <typename T, int DIM, int OP>
+__global__ __launch_bounds__(128) void k_restrict(int fnx, int fny, int fnz, int cnx, int cny, unsigned nc,
+                                                  const T* __restrict__ rf, T* __restrict__ rc,
+                                                  const uint8_t* __restrict__ bcc, const uint8_t* __restrict__ bcf,
+                                                  RestrictOut<T> out) {
+  const long idx = (long)blockIdx.x * 128 + threadIdx.x;
+  if (idx >= (long)nc * DIM) return;
+  const unsigned n = (unsigned)(idx / DIM), row = n / cnx;
+  const int d = (int)(idx - (long)n * DIM), i = (int)(n % cnx), j = (int)(row % cny), k = (int)(row / cny);
+  // every fine value and mask is loaded before the first is used (neighbours outside the grid load
+  // the vertex itself and are skipped by the select): the grids of the cycle are small, so the
+  // kernel is one round trip to memory instead of one per neighbour
+  constexpr int NZ = DIM == 3 ? 3 : 1, NQ = 9 * NZ;
+  const int I[3] = {i > 0 ? 2 * i - 1 : 0, 2 * i, 2 * i + 1 < fnx ? 2 * i + 1 : 2 * i};
+  const int J[3] = {j > 0 ? 2 * j - 1 : 0, 2 * j, 2 * j + 1 < fny ? 2 * j + 1 : 2 * j};
+  const int K[3] = {k > 0 ? 2 * k - 1 : 0, 2 * k, 2 * k + 1 < fnz ? 2 * k + 1 : 2 * k};
+  T v[NQ];
+  uint8_t mf[NQ];
 #pragma unroll
-  for (int oz = (DIM == 3 ? -1 : 0); oz <= (DIM == 3 ? 1 : 0); oz++) {
-    const int K = 2 * k + oz;
-#pragma unroll
-    for (int oy = -1; oy <= 1; oy++) {
-      const int J = 2 * j + oy;
-#pragma unroll
-      for (int ox = -1; ox <= 1; ox++) {
-        const int I = 2 * i + ox;
-        const bool in = K >= 0 && K < fnz && J >= 0 && J < fny && I >= 0 && I < fnx;
-        T w = (T)1;
-        if (ox) w *= (T)0.5;
-        if (oy) w *= (T)0.5;
-        if (oz) w *= (T)0.5;
-        const long fn = in ? I + (long)fnx * (J + (long)fny * K) : 0;
-        const uint8_t mf = bcf[fn];
-        T v[3];
-        for (int d = 0; d < DIM; d++) v[d] = rf[fn * DIM + d];
-        for (int d = 0; d < DIM; d++) acc[d] = (in && !((mf >> d) & 1)) ? acc[d] + w * v[d] : acc[d];
-      }
-    }
+  for (int q = 0; q < NQ; q++) {
+    const long fn = I[q % 3] + (long)fnx * (J[(q / 3) % 3] + (long)fny * (DIM == 3 ? K[q / 9] : 0));
+    mf[q] = bcf[fn];
+    v[q] = rf[fn * DIM + d];
   }
-  uint8_t m = bcc[n];
-  for (int d = 0; d < DIM; d++) rc[n * DIM + d] = ((m >> d) & 1) ? (T)0 : acc[d];
+  const uint8_t mc = bcc[n];
+  __builtin_amdgcn_sched_barrier(0);
+  const bool in[3][3] = {{i > 0, true, 2 * i + 1 < fnx}, {j > 0, true, 2 * j + 1 < fny}, {k > 0, true, 2 * k + 1 < fnz}};
+  T acc = 0;
+#pragma unroll
+  for (int q = 0; q < NQ; q++) {
+    const int ox = q % 3, oy = (q / 3) % 3, oz = DIM == 3 ? q / 9 : 1;
+    T w = (T)1;
+    if (ox != 1) w *= (T)0.5;
+    if (oy != 1) w *= (T)0.5;
+    if (oz != 1) w *= (T)0.5;
+    acc = (in[0][ox] && in[1][oy] && in[2][oz] && !((mf[q] >> d) & 1)) ? acc + w * v[q] : acc;
+  }
+  const T b = ((mc >> d) & 1) ? (T)0 : acc;
+  rc[idx] = b;
+  if constexpr (OP == 1) {
+    const T v = out.c * (out.dinv[idx] * b);
+    out.d[idx] = v;
+    out.x[idx] = v;
+  }
+  if constexpr (OP == 2) out.wide[idx] = 1.0 * (double)b;
 }
 
 template <typename T>
 void launch_prolong_add(const Geom& f, const Geom& c, const T* xc, T* xf, const uint8_t* bcf, hipStream_t s) {
   if (f.dim == 3)
-    hipLaunchKernelGGL((k_prolong_add<T, 3>), nblocks(f.N, 256), 256, 0, s, f.nn[0], f.nn[1], f.nn[2], c.nn[0], c.nn[1],
-                       f.N, xc, xf, bcf);
+    hipLaunchKernelGGL((k_prolong_add<T, 3>), nblocks(f.N * 3, 128), 128, 0, s, f.nn[0], f.nn[1], c.nn[0], c.nn[1],
+                       (unsigned)f.N, xc, xf, bcf);
   else
-    hipLaunchKernelGGL((k_prolong_add<T, 2>), nblocks(f.N, 256), 256, 0, s, f.nn[0], f.nn[1], 1, c.nn[0], c.nn[1], f.N,
-                       xc, xf, bcf);
+    hipLaunchKernelGGL((k_prolong_add<T, 2>), nblocks(f.N * 2, 128), 128, 0, s, f.nn[0], f.nn[1], c.nn[0], c.nn[1],
+                       (unsigned)f.N, xc, xf, bcf);
   UWG_HIP(hipGetLastError());
 }
 template void launch_prolong_add<double>(const Geom&, const Geom&, const double*, double*, const uint8_t*, hipStream_t);
 template void launch_prolong_add<float>(const Geom&, const Geom&, const float*, float*, const uint8_t*, hipStream_t);
 
-// restriction needs both masks; the fine mask is passed through a global set by the host
 template <typename T>
 void launch_restrict2(const Geom& f, const Geom& c, const T* rf, T* rc, const uint8_t* bcc, const uint8_t* bcf,
-                      hipStream_t s) {
+                      const RestrictOut<T>& out, hipStream_t s) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, nblocks(c.N * f.dim, 128), 128, 0, s, f.nn[0], f.nn[1], f.dim == 3 ? f.nn[2] : 1,
+                       c.nn[0], c.nn[1], (unsigned)c.N, rf, rc, bcc, bcf, out);
+  };
+  const int op = out.x ? 1 : (out.wide ? 2 : 0);
   if (f.dim == 3)
-    hipLaunchKernelGGL((k_restrict<T, 3>), nblocks(c.N, 256), 256, 0, s, f.nn[0], f.nn[1], f.nn[2], c.nn[0], c.nn[1],
-                       c.nn[2], c.N, rf, rc, bcc, bcf);
+    op == 0 ? go(k_restrict<T, 3, 0>) : op == 1 ? go(k_restrict<T, 3, 1>) : go(k_restrict<T, 3, 2>);
   else
-    hipLaunchKernelGGL((k_restrict<T, 2>), nblocks(c.N, 256), 256, 0, s, f.nn[0], f.nn[1], 1, c.nn[0], c.nn[1], 1, c.N,
-                       rf, rc, bcc, bcf);
+    op == 0 ? go(k_restrict<T, 2, 0>) : op == 1 ? go(k_restrict<T, 2, 1>) : go(k_restrict<T, 2, 2>);
   UWG_HIP(hipGetLastError());
 }
 template void launch_restrict2<double>(const Geom&, const Geom&, const double*, double*, const uint8_t*, const uint8_t*,
-                                       hipStream_t);
+                                       const RestrictOut<double>&, hipStream_t);
 template void launch_restrict2<float>(const Geom&, const Geom&, const float*, float*, const uint8_t*, const uint8_t*,
-                                      hipStream_t);
+                                      const RestrictOut<float>&, hipStream_t);
 
 // Dirichlet mask for walls: wallbits bit (2*d + side) set -> component d fixed on that wall
 __global__ void k_bc_walls(int nx, int ny, int nz, int dim, long N, int wallbits, uint8_t* bc) {
@@ -2082,15 +2135,33 @@ __device__ inline double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+// wave_sum of KM values at once: while more than one is left, each half of the lanes keeps half of
+// the values and hands the other half over, so KM + 5 exchanges take the place of 6 KM.  The lanes
+// whose low bits are zero end with the sum of value (lane KM) / 64 in acc[0], added up in the
+// pairs and order of wave_sum.
+template <int KM, int O = 32>
+__device__ __forceinline__ void wave_sums(double* acc) {
+  if constexpr (O > 0) {
+    if constexpr (KM > 1) {
+      const bool upper = threadIdx.x & O;
+#pragma unroll
+      for (int j = 0; j < KM / 2; j++) {
+        const double keep = upper ? acc[j + KM / 2] : acc[j], give = upper ? acc[j] : acc[j + KM / 2];
+        acc[j] = keep + __shfl_xor(give, O, 64);
+      }
+      wave_sums<KM / 2, O / 2>(acc);
+    } else {
+      acc[0] += __shfl_xor(acc[0], O, 64);
+      wave_sums<1, O / 2>(acc);
+    }
+  }
+}
 // the block's KM sums, in sm[KM][4] (per wave) then partial[j * RB + block] (thread j)
 template <int KM>
 __device__ inline void block_sums(double (&acc)[KM], int k, double (*sm)[4], double* partial) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int j = 0; j < KM; j++) {
-    const double t = wave_sum(acc[j]);
-    if (lane == 0) sm[j][wv] = t;
-  }
+  wave_sums<KM>(acc);
+  if (lane % (64 / KM) == 0) sm[lane / (64 / KM)][wv] = acc[0];
   __syncthreads();
   if (threadIdx.x < KM && threadIdx.x < k) {
     const int j = threadIdx.x;
@@ -2131,13 +2202,20 @@ __global__ __launch_bounds__(256) void k_mdot_pairs(long n, int k, const TX* __r
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n2; i += (long)gridDim.x * blockDim.x) {
     const XV xv = reinterpret_cast<const XV*>(x)[i];
     const double x0 = (double)xv.x, x1 = (double)xv.y;
+    // eight vectors' loads at a time: a branch per vector would let one load fly at a time (the
+    // last group repeats vector k - 1, whose extra sums are not used)
 #pragma unroll
-    for (int j = 0; j < KM; j++)
-      if (j < k) {
-        const YV yv = reinterpret_cast<const YV*>(Y[j])[i];
-        acc[j] += x0 * (double)yv.x;
-        acc[j] += x1 * (double)yv.y;
+    for (int j0 = 0; j0 < KM; j0 += 8) {
+      if (j0 >= k) break;
+      YV yv[8];
+#pragma unroll
+      for (int j = 0; j < 8; j++) yv[j] = reinterpret_cast<const YV*>(Y[j0 + j < k ? j0 + j : k - 1])[i];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        acc[j0 + j] += x0 * (double)yv[j].x;
+        acc[j0 + j] += x1 * (double)yv[j].y;
       }
+    }
   }
   if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
     const double xl = (double)x[n - 1];
@@ -2159,49 +2237,62 @@ __global__ __launch_bounds__(256) void k_sqnorm(long n, const T* __restrict__ x,
   block_sums<1>(acc, 1, sm, partial);
 }
 
-// one block per dot product (block j sums the RB partials of dot j in a fixed order)
-__global__ void k_mdot_final(const double* partial, double* out) {
-  __shared__ double sm[256];
-  const int j = blockIdx.x;
+// blocks of a reduction over n threads' worth of elements: the grid is fixed at RB where there is
+// work for it, and the blocks that would have none are left out (their sums are zeros)
+static int reduce_blocks(long n) { return (int)std::min<long>(RB, std::max<long>(1, (n + 255) / 256)); }
+
+// the sum of nb <= RB partials in a fixed order, in sm[0] of a block of 256
+__device__ __forceinline__ void sum_partials(const double* partial, int nb, double* sm) {
   double a = 0.0;
-  for (int b = threadIdx.x; b < RB; b += 256) a += partial[j * RB + b];
+  for (int b = threadIdx.x; b < nb; b += 256) a += partial[b];
   sm[threadIdx.x] = a;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) sm[threadIdx.x] += sm[threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x < 64) {
+    a = (sm[threadIdx.x] + sm[threadIdx.x + 128]) + (sm[threadIdx.x + 64] + sm[threadIdx.x + 192]);
+    a = wave_sum(a);
+    if (threadIdx.x == 0) sm[0] = a;
   }
-  if (threadIdx.x == 0) out[j] = sm[0];
+  __syncthreads();
+}
+// one block per dot product
+__global__ __launch_bounds__(256) void k_mdot_final(const double* partial, int nb, double* out) {
+  __shared__ double sm[256];
+  sum_partials(partial + blockIdx.x * RB, nb, sm);
+  if (threadIdx.x == 0) out[blockIdx.x] = sm[0];
 }
 template <typename TX, typename TY>
-static void mdot_pass(long n, int k, const TX* x, const TY* const* Y, double* partial, hipStream_t s) {
+static int mdot_pass(long n, int k, const TX* x, const TY* const* Y, double* partial, hipStream_t s) {
+  const int nb = reduce_blocks(n);
   if (k <= 1)
-    hipLaunchKernelGGL((k_mdot<1, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot<1, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
   else if (k <= 4)
-    hipLaunchKernelGGL((k_mdot<4, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot<4, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
   else if (k <= 8)
-    hipLaunchKernelGGL((k_mdot<8, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot<8, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
   else if (k <= 16)
-    hipLaunchKernelGGL((k_mdot<16, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot<16, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
   else
-    hipLaunchKernelGGL((k_mdot<32, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot<32, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
+  return nb;
 }
 template <typename TX, typename TY>
-static void mdot_pairs_pass(long n, int k, const TX* x, const TY* const* Y, double* partial, hipStream_t s) {
+static int mdot_pairs_pass(long n, int k, const TX* x, const TY* const* Y, double* partial, hipStream_t s) {
+  const int nb = reduce_blocks(n >> 1);
   if (k <= 8)
-    hipLaunchKernelGGL((k_mdot_pairs<8, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot_pairs<8, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
   else if (k <= 16)
-    hipLaunchKernelGGL((k_mdot_pairs<16, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot_pairs<16, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
   else
-    hipLaunchKernelGGL((k_mdot_pairs<32, TX, TY>), RB, 256, 0, s, n, k, x, Y, partial);
+    hipLaunchKernelGGL((k_mdot_pairs<32, TX, TY>), nb, 256, 0, s, n, k, x, Y, partial);
+  return nb;
 }
 template <typename T>
 void vk_multi_dot(long n, int k, const T* x, const T* const* Y, double* partial, double* out, hipStream_t s) {
   if (k < 1) return;
   for (int j0 = 0; j0 < k; j0 += KMAX) {
     const int kk = std::min(KMAX, k - j0);
-    mdot_pass<T, T>(n, kk, x, Y + j0, partial, s);
-    hipLaunchKernelGGL(k_mdot_final, kk, 256, 0, s, partial, out + j0);
+    const int nb = mdot_pass<T, T>(n, kk, x, Y + j0, partial, s);
+    hipLaunchKernelGGL(k_mdot_final, kk, 256, 0, s, partial, nb, out + j0);
   }
   UWG_HIP(hipGetLastError());
 }
@@ -2219,6 +2310,7 @@ __global__ void k_gs_update_pairs(long n, int k, const TV* const* V, const doubl
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n2; i += (long)gridDim.x * blockDim.x) {
     const WV wv = reinterpret_cast<const WV*>(w)[i];
     double a0 = (double)wv.x, a1 = (double)wv.y;
+#pragma unroll 8
     for (int j = 0; j < k; j++) {
       const VV v = reinterpret_cast<const VV*>(V[j])[i];
       const double c = -h[j];
@@ -2237,6 +2329,40 @@ __global__ void k_gs_update_pairs(long n, int k, const TV* const* V, const doubl
   }
 }
 
+// the same update with the partial sums of |w|^2 that k_sqnorm forms, one element per thread
+// (n <= 256 RB: k_sqnorm's threads have one element each there)
+template <typename TW, typename TV>
+__global__ __launch_bounds__(256) void k_gs_update_norm(long n, int k, const TV* const* V,
+                                                        const double* __restrict__ h, TW* __restrict__ w,
+                                                        double* partial) {
+  __shared__ double sm[1][4];
+  double acc[1] = {0.0};
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) {
+    double a = (double)w[i];
+#pragma unroll 8
+    for (int j = 0; j < k; j++) a += (-h[j]) * (double)V[j][i];
+    const TW o = (TW)a;
+    w[i] = o;
+    const double xv = (double)o;
+    acc[0] += xv * xv;
+  }
+  block_sums<1>(acc, 1, sm, partial);
+}
+// k_scale_by_norm with the sum of the nb partials of |w|^2, which block 0 leaves in *dot
+template <typename TW, typename TV>
+__global__ __launch_bounds__(256) void k_sum_scale_by_norm(long n, const double* partial, int nb, double* dot,
+                                                           const TW* __restrict__ w, TV* __restrict__ v) {
+  __shared__ double sm[256];
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const TW wi = i < n ? w[i] : (TW)0;
+  sum_partials(partial, nb, sm);
+  const double d = sm[0], hn = sqrt(fmax(0.0, d));
+  if (i == 0) *dot = d;
+  if (!(hn > 0.0) || i >= n) return;
+  v[i] = (TV)((TW)(1.0 / hn) * wi);
+}
+
 // v = w / sqrt(max(0, *dot)) (the scale rounded to TW as vk_scale takes it, the product rounded
 // to the basis type TV); nothing is written when the norm is zero
 template <typename TW, typename TV>
@@ -2251,17 +2377,28 @@ __global__ void k_scale_by_norm(long n, const double* __restrict__ dot, const TW
 
 // The update runs on the streaming grid (a reduction-sized grid holds too few loads in flight
 // for the k-vector gather); |w|^2 is then the one-vector dot of vk_multi_dot.  V[j] and w must
-// be whole allocations (16-byte aligned) for the paired loads of the dot products.
+// be whole allocations (16-byte aligned) for the paired loads of the dot products.  Up to 256 RB
+// elements the norm comes with the update and its sum with the scaling, four launches instead of
+// six, all of them latency.  A step over 30 vectors of 33^3 velocities and 32^3 pressures:
+// dot products 24.9 -> 13.7 us, the rest 24 -> 13 us; 128^3 (two-pass form): dot products
+// 283 -> 198 us (4.4 TB/s).  The sums are the same bits on both paths.
 template <typename TW, typename TV>
 void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, hipStream_t s) {
   for (int j0 = 0; j0 < k; j0 += KMAX) {
     const int kk = std::min(KMAX, k - j0);
-    mdot_pairs_pass<TW, TV>(n, kk, w, V + j0, partial, s);
-    hipLaunchKernelGGL(k_mdot_final, kk, 256, 0, s, partial, h + j0);
+    const int nb = mdot_pairs_pass<TW, TV>(n, kk, w, V + j0, partial, s);
+    hipLaunchKernelGGL(k_mdot_final, kk, 256, 0, s, partial, nb, h + j0);
+  }
+  if (n <= 256L * RB) {
+    const int nb = reduce_blocks(n);
+    hipLaunchKernelGGL((k_gs_update_norm<TW, TV>), nb, 256, 0, s, n, k, V, h, w, partial);
+    hipLaunchKernelGGL((k_sum_scale_by_norm<TW, TV>), nb, 256, 0, s, n, partial, nb, h + k, w, v_next);
+    UWG_HIP(hipGetLastError());
+    return;
   }
   hipLaunchKernelGGL((k_gs_update_pairs<TW, TV>), vgrid(std::max(n >> 1, 1L)), 256, 0, s, n, k, V, h, w);
   hipLaunchKernelGGL(k_sqnorm<TW>, RB, 256, 0, s, n, w, partial);
-  hipLaunchKernelGGL(k_mdot_final, 1, 256, 0, s, partial, h + k);
+  hipLaunchKernelGGL(k_mdot_final, 1, 256, 0, s, partial, RB, h + k);
   hipLaunchKernelGGL((k_scale_by_norm<TW, TV>), vgrid(n), 256, 0, s, n, h + k, w, v_next);
   UWG_HIP(hipGetLastError());
 }
@@ -2274,7 +2411,8 @@ template void vk_multi_dot<double>(long, int, const double*, const double* const
 template void vk_multi_dot<float>(long, int, const float*, const float* const*, double*, double*, hipStream_t);
 
 // dense y = A x (A symmetric, n x n): one block per row, coalesced along the row
-__global__ __launch_bounds__(256) void k_dense_mv(int n, const double* A, const double* x, double* y) {
+template <typename T>
+__global__ __launch_bounds__(256) void k_dense_mv(int n, const double* A, const double* x, T* y) {
   __shared__ double sm[256];
   const int r = blockIdx.x;
   double acc = 0.0;
@@ -2285,7 +2423,7 @@ __global__ __launch_bounds__(256) void k_dense_mv(int n, const double* A, const 
     if (threadIdx.x < w) sm[threadIdx.x] += sm[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) y[r] = sm[0];
+  if (threadIdx.x == 0) y[r] = (T)sm[0];
 }
 // Dense operator of the coarsest multigrid level, one thread per entry (r, c), r = node_r d + i,
 // c = node_c d + j: K[r][c] = sum over the elements holding both nodes (fixed order) and their
@@ -2380,9 +2518,12 @@ void launch_coarse_inverse(const Geom& g, const double* W, const uint8_t* bc, do
   UWG_HIP(hipGetLastError());
 }
 
-void launch_dense_mv(int n, const double* A, const double* x, double* y, hipStream_t s) {
-  hipLaunchKernelGGL(k_dense_mv, n, 256, 0, s, n, A, x, y);
+template <typename T>
+void launch_dense_mv(int n, const double* A, const double* x, T* y, hipStream_t s) {
+  hipLaunchKernelGGL(k_dense_mv<T>, n, 256, 0, s, n, A, x, y);
   UWG_HIP(hipGetLastError());
 }
+template void launch_dense_mv<double>(int, const double*, const double*, double*, hipStream_t);
+template void launch_dense_mv<float>(int, const double*, const double*, float*, hipStream_t);
 
 }  // namespace uwg

@@ -1232,8 +1232,9 @@ template <typename T>
 // Chebyshev(degree) smoothing of K x = b with Jacobi scaling, eigenvalue window
 // [0.12, 1.1] * lmax.  Each step after the first is one fused kernel (apply, residual and
 // update); the iterate alternates between x and the level's r buffer, arranged so that the
-// last step writes x.
-static void chebyshev(Level& A, const T* b, T* x, int degree, bool zero_guess) {
+// last step writes x.  `started`: the first step from a zero guess was done where b was formed
+// (cheb_start).
+static void chebyshev(Level& A, const T* b, T* x, int degree, bool zero_guess, bool started = false) {
   const long n = A.n();
   const double emax = 1.1 * A.lmax, emin = 0.12 * A.lmax;
   const double theta = 0.5 * (emax + emin), delta = 0.5 * (emax - emin);
@@ -1247,7 +1248,7 @@ static void chebyshev(Level& A, const T* b, T* x, int degree, bool zero_guess) {
   if (zero_guess) {
     // x0 = 0: d = dinv b / theta, x1 = d; written where the alternation ends in x
     cur = (steps % 2 == 1) ? tmp : x;
-    vk_cheb_first<T>(n, (T)(1.0 / theta), dinv, b, d, cur, 0);
+    if (!started) vk_cheb_first<T>(n, (T)(1.0 / theta), dinv, b, d, cur, 0);
   }
   for (int k = 0; k < steps; k++) {
     T* nxt = (cur == x) ? tmp : x;
@@ -1265,23 +1266,53 @@ static void chebyshev(Level& A, const T* b, T* x, int degree, bool zero_guess) {
   if (cur != x) vk_copy<T>(n, cur, x, 0);
 }
 
+// the first smoothing step of chebyshev(A, ., x, degree, true) for the pass that forms b
 template <typename T>
-static void coarse_solve(uwg_stokes* st, Level& A, const T* b, T* x);
+static RestrictOut<T> cheb_start(Level& A, T* x, int degree) {
+  const double emax = 1.1 * A.lmax, emin = 0.12 * A.lmax;
+  RestrictOut<T> o;
+  o.c = (T)(1.0 / (0.5 * (emax + emin)));
+  o.dinv = LV<T>::dinv(A);
+  o.d = LV<T>::d(A);
+  o.x = (degree - 1) % 2 == 1 ? LV<T>::r(A) : x;
+  return o;
+}
+
+template <typename T>
+static void coarse_solve(uwg_stokes* st, Level& A, const T* b, T* x, bool started);
 
 template <>
-void coarse_solve<double>(uwg_stokes* st, Level& A, const double* b, double* x) {
+void coarse_solve<double>(uwg_stokes* st, Level& A, const double* b, double* x, bool) {
   if (st->coarse.Ainv)
     launch_dense_mv(st->coarse.n, st->coarse.Ainv, b, x, 0);
   else
     chebyshev<double>(A, b, x, 24, true);
 }
+// FP64 coarsest solve inside the FP32 cycle; started: b is in A.b already
 template <>
-void coarse_solve<float>(uwg_stokes* st, Level& A, const float* b, float* x) {
-  // FP64 coarsest solve inside the FP32 cycle
+void coarse_solve<float>(uwg_stokes* st, Level& A, const float* b, float* x, bool started) {
   const long n = A.n();
-  vk_f2d(n, 1.0, b, A.b, 0);
-  coarse_solve<double>(st, A, A.b, A.x);
+  if (!started) vk_f2d(n, 1.0, b, A.b, 0);
+  if (st->coarse.Ainv) {
+    launch_dense_mv(st->coarse.n, st->coarse.Ainv, A.b, x, 0);
+    return;
+  }
+  coarse_solve<double>(st, A, A.b, A.x, false);
   vk_d2f(n, 1.0, A.x, x, 0);
+}
+
+// b of level l from the residual r of the level above, with what the cycle starts with there
+// unless a network takes the cycle's place
+template <typename T>
+static void restrict_to(uwg_stokes* st, const Geom& fine, const uint8_t* fine_bc, const T* r, int l, bool start) {
+  Level& C = st->L[l];
+  RestrictOut<T> out;
+  if (start && l + 1 < (int)st->L.size()) {
+    out = cheb_start<T>(C, LV<T>::x(C), g_smooth_degree);
+  } else if (start) {
+    if constexpr (std::is_same<T, float>::value) out.wide = C.b;
+  }
+  launch_restrict2<T>(fine, C.g, r, LV<T>::b(C), C.bc, fine_bc, out, 0);
 }
 
 template <typename T>
@@ -1294,25 +1325,27 @@ static void capture_vector(uwg_stokes* st, long n, const T* v) {
   st->captured++;
 }
 
+// started: b came from restrict_to
 template <typename T>
-static void vcycle(uwg_stokes* st, int l, const T* b, T* x) {
+static void vcycle(uwg_stokes* st, int l, const T* b, T* x, bool started = false) {
   Level& A = st->L[l];
   if (l == (int)st->L.size() - 1) {
-    coarse_solve<T>(st, A, b, x);
+    coarse_solve<T>(st, A, b, x, started);
     return;
   }
   Level& C = st->L[l + 1];
-  chebyshev<T>(A, b, x, g_smooth_degree, true);
+  chebyshev<T>(A, b, x, g_smooth_degree, true, started);
   T* r = LV<T>::r(A);
   launch_residual_K<T>(A.g, LV<T>::W(A), x, b, r, A.bc, 0, LV<T>::Wbf(A), LV<T>::S(A));
-  launch_restrict2<T>(A.g, C.g, r, LV<T>::b(C), C.bc, A.bc, 0);
-  const bool capture = st->capture_level == l + 1 && st->captured < st->capture_max &&
-                       (st->capture_seen++ % st->capture_every) == 0;
-  if (capture && st->capture_kind == 0) capture_vector<T>(st, C.n(), LV<T>::b(C));
   bool use_nn = false;
   if constexpr (std::is_same<T, float>::value)
     use_nn = st->nn && !st->nn_disabled && l + 1 == st->nn_level;
-  if (use_nn && st->nn_mode == 0) {
+  const bool cycle = !(use_nn && st->nn_mode == 0);
+  restrict_to<T>(st, A.g, A.bc, r, l + 1, cycle);
+  const bool capture = st->capture_level == l + 1 && st->captured < st->capture_max &&
+                       (st->capture_seen++ % st->capture_every) == 0;
+  if (capture && st->capture_kind == 0) capture_vector<T>(st, C.n(), LV<T>::b(C));
+  if (!cycle) {
     // the learned network stands in for the coarse-grid cycle below this level; its output is
     // scaled by the residual-minimising step on this level
     if constexpr (std::is_same<T, float>::value) {
@@ -1321,7 +1354,7 @@ static void vcycle(uwg_stokes* st, int l, const T* b, T* x) {
       nn_line_search(C.n(), C.b32, C.r32, C.d32, C.x32, false, 0);
     }
   } else {
-    vcycle<T>(st, l + 1, LV<T>::b(C), LV<T>::x(C));
+    vcycle<T>(st, l + 1, LV<T>::b(C), LV<T>::x(C), true);
     if (capture && st->capture_kind == 1) {
       // residual the coarse cycle leaves behind: its error K_C^{-1} r is what an additive
       // correction has to supply
@@ -1404,7 +1437,17 @@ static void top_G(uwg_stokes* st, const T* p, T* y, const uint8_t* bc) {
   if (st->q2)
     launch_q2_apply_G<T>(st->g, st->q2->Gr, p, bc, y, 0);
   else
-    launch_apply_G<T>(st->g, st->Ge, p, bc, y, 0);
+    launch_apply_G<T>(st->g, st->Ge, p, bc, y, false, 0);
+}
+// y += G p; work: a velocity vector, for the kernels that do not add
+template <typename T>
+static void top_G_add(uwg_stokes* st, const T* p, T* y, const uint8_t* bc, T* work) {
+  if (st->q2) {
+    top_G<T>(st, p, work, bc);
+    vk_axpy<T>(st->nu, (T)1, work, y, 0);
+  } else {
+    launch_apply_G<T>(st->g, st->Ge, p, bc, y, true, 0);
+  }
 }
 template <typename T>
 static void top_GT(uwg_stokes* st, const T* u, T* q, const uint8_t* bc) {
@@ -1440,6 +1483,34 @@ static void schur_prec(uwg_stokes* st, const T* diagS, const T* r, T* z) {
     schur_stencil_apply<T>(st->g, st->snn_a, r, z, 0);
   else
     top_schur<T>(st, diagS, r, z);
+}
+// the pressure row of the block preconditioner, z = -S^-1 (r - G^T u); q: a pressure vector, wide: one
+// in T for a narrower r
+template <typename T, typename TR>
+static void pressure_prec(uwg_stokes* st, const T* diagS, const T* u, const TR* r, T* z, T* q, T* wide,
+                          bool learned = true) {
+  const uint8_t* bc = top_bc(st);
+  learned = learned && g_snn_active && st->snn && !st->nn_disabled;
+  if (st->q2) {
+    const T* rt;
+    if constexpr (std::is_same<T, TR>::value) {
+      rt = r;
+    } else {
+      vk_f2d(st->np, 1.0, r, wide, 0);
+      rt = wide;
+    }
+    top_GT<T>(st, u, q, bc);
+    vk_axpby<T>(st->np, (T)1, rt, (T)-1, q, 0);
+    if (learned)
+      schur_stencil_apply<T>(st->g, st->snn_a, q, z, 0);
+    else
+      top_schur<T>(st, diagS, q, z);
+  } else if (learned) {
+    launch_apply_GT<T, TR>(st->g, st->Ge, u, bc, q, 0, r);
+    schur_stencil_apply<T>(st->g, st->snn_a, q, z, 0);
+  } else {
+    launch_apply_GT<T, TR>(st->g, st->Ge, u, bc, z, 0, r, diagS);
+  }
 }
 
 // Chebyshev smoothing on the Q2 level: same window and recurrence as the Q1 smoother
@@ -1481,8 +1552,8 @@ static void q2_vcycle(uwg_stokes* st, const T* b, T* x) {
   q2_chebyshev<T>(st, b, x, g_smooth_degree, true);
   T* r = Q2V<T>::r(A);
   q2_K<T>(st, x, A.bc, Q2Op::residual, Q2Out<T>{r, b});
-  launch_restrict2<T>(A.gn, C.g, r, LV<T>::b(C), C.bc, A.bc, 0);
-  vcycle<T>(st, 0, LV<T>::b(C), LV<T>::x(C));
+  restrict_to<T>(st, A.gn, A.bc, r, 0, true);
+  vcycle<T>(st, 0, LV<T>::b(C), LV<T>::x(C), true);
   launch_prolong_add<T>(A.gn, C.g, LV<T>::x(C), x, A.bc, 0);
   q2_chebyshev<T>(st, b, x, g_smooth_degree, false);
 }
@@ -2137,9 +2208,7 @@ static int solve_schur(uwg_stokes* st, const uwg_solve_opts& o, uwg_solve_stats*
       top_vcycle<float>(st, b32, x32);
       vk_f2d(n, 1.0, x32, y, 0);
     } else {
-      double* b64 = top_buf_b<double>(st);
-      vk_copy<double>(n, x, b64, 0);
-      top_vcycle<double>(st, b64, y);
+      top_vcycle<double>(st, x, y);
     }
   };
   auto inner = [&](const double* rhs, double* x, int* its) {
@@ -2207,8 +2276,7 @@ static int solve_block(uwg_stokes* st, const uwg_solve_opts& o, uwg_solve_stats*
   double* gp = wsbuf<double>(st, WS_BLK_GP, n);
   OpFn Aop = [&](const double* xx, double* yy) {
     top_K<double>(st, xx, yy, bc);
-    top_G<double>(st, xx + n, gp, bc);
-    vk_axpy<double>(n, 1.0, gp, yy, 0);
+    top_G_add<double>(st, xx + n, yy, bc, gp);
     top_GT<double>(st, xx, yy + n, bc);
   };
   OpFn Mop = [&](const double* rr, double* zz) {
@@ -2224,13 +2292,9 @@ static int solve_block(uwg_stokes* st, const uwg_solve_opts& o, uwg_solve_stats*
       inner_solve_fp64(st, rr, zz, st->exact_vel_rtol, &vits);
       st->vcycles += vits - 1;
     } else {
-      double* b64 = top_buf_b<double>(st);
-      vk_copy<double>(n, rr, b64, 0);
-      top_vcycle<double>(st, b64, zz);
+      top_vcycle<double>(st, rr, zz);
     }
-    top_GT<double>(st, zz, q, bc);
-    vk_axpby<double>(E, 1.0, rr + n, -1.0, q, 0);  // q = r_p - G^T z_u
-    schur_prec<double>(st, diagS, q, zz + n);
+    pressure_prec<double>(st, diagS, zz, rr + n, zz + n, q, q);
   };
   int its = 0;
   double rn;
@@ -2285,10 +2349,7 @@ static int solve_block(uwg_stokes* st, const uwg_solve_opts& o, uwg_solve_stats*
       float* x32 = top_buf_x<float>(st);
       top_vcycle<float>(st, rr, x32);
       vk_f2d(n, 1.0, x32, zz, 0);
-      top_GT<double>(st, zz, q, bc);
-      vk_f2d(E, 1.0, rr + n, rp, 0);
-      vk_axpby<double>(E, 1.0, rp, -1.0, q, 0);  // q = r_p - G^T z_u
-      schur_prec<double>(st, diagS, q, zz + n);
+      pressure_prec<double>(st, diagS, zz, rr + n, zz + n, q, rp);
     };
     rc = fgmres<double, float>(st, Kb32, Aop, Mop32, b, x, o.outer_rtol, 1e-300, o.max_outer_its, &its, &rn, true,
                                &mon);
@@ -2332,22 +2393,18 @@ static int solve_block_mixed(uwg_stokes* st, const uwg_solve_opts& o, uwg_solve_
   if (!st->q2) launch_neg_recip<float>(E, st->approxS, diagS32, 0);
   auto A64 = [&](const double* xx, double* yy) {
     top_K<double>(st, xx, yy, bc);
-    top_G<double>(st, xx + n, gp, bc);
-    vk_axpy<double>(n, 1.0, gp, yy, 0);
+    top_G_add<double>(st, xx + n, yy, bc, gp);
     top_GT<double>(st, xx, yy + n, bc);
   };
   OpFn32 A32 = [&](const float* xx, float* yy) {
     top_K<float>(st, xx, yy, bc);
-    top_G<float>(st, xx + n, gp32, bc);
-    vk_axpy<float>(n, 1.0f, gp32, yy, 0);
+    top_G_add<float>(st, xx + n, yy, bc, gp32);
     top_GT<float>(st, xx, yy + n, bc);
   };
   OpFn32 M32 = [&](const float* rr, float* zz) {
     st->vcycles++;
     top_vcycle<float>(st, rr, zz);
-    top_GT<float>(st, zz, q32, bc);
-    vk_axpby<float>(E, 1.0f, rr + n, -1.0f, q32, 0);  // q = r_p - G^T z_u
-    top_schur<float>(st, diagS32, q32, zz + n);
+    pressure_prec<float>(st, diagS32, zz, rr + n, zz + n, q32, q32, false);
   };
   const double bn = sqrt(dev_dot<double>(st, nt, b, b));
   int total = 0, sweeps = 0, status = 0;
@@ -2560,7 +2617,7 @@ extern "C" int uwg_stokes_apply(uwg_stokes* st, int which, int level, const doub
   if (which == 0)
     launch_apply_K<double>(A.g, A.W, dx, dy, A.bc, 0, nullptr, A.S);
   else if (which == 1)
-    launch_apply_G(st->g, st->Ge, dx, st->L[0].bc, dy, 0);
+    launch_apply_G(st->g, st->Ge, dx, st->L[0].bc, dy, false, 0);
   else if (which == 2)
     launch_apply_GT(st->g, st->Ge, dx, st->L[0].bc, dy, 0);
   else {
@@ -2806,9 +2863,7 @@ static int inner_solve_fp64(uwg_stokes* st, const double* b, double* x, double r
   st->kin->init(n, 30);
   OpFn Kop = [&](const double* xx, double* yy) { top_K<double>(st, xx, yy, bc); };
   OpFn Mv = [&](const double* xx, double* yy) {
-    double* b64 = top_buf_b<double>(st);
-    vk_copy<double>(n, xx, b64, 0);
-    top_vcycle<double>(st, b64, yy);
+    top_vcycle<double>(st, xx, yy);
   };
   vk_fill<double>(n, 0.0, x, 0);
   double rn;

@@ -117,15 +117,26 @@ void launch_cheb_step_K(const Geom& g, const T* W, const T* x, T* xn, const T* b
 // FP64 weights [27][Es] -> bfloat16 pairs [14][Es]: word p = bf16(W_2p) | bf16(W_2p+1) << 16
 void launch_pack_w3_bf16(long Es, const double* W, uint32_t* Wb, hipStream_t s);
 template <typename T>
-void launch_apply_G(const Geom& g, const double* Ge, const T* p, const uint8_t* bc, T* y, hipStream_t s);
-template <typename T>
-void launch_apply_GT(const Geom& g, const double* Ge, const T* u, const uint8_t* bc, T* q, hipStream_t s);
+void launch_apply_G(const Geom& g, const double* Ge, const T* p, const uint8_t* bc, T* y, bool add, hipStream_t s);
+// q = G^T u, with r: r - G^T u, and with scale: scale (r - G^T u)
+template <typename T, typename TR = T>
+void launch_apply_GT(const Geom& g, const double* Ge, const T* u, const uint8_t* bc, T* q, hipStream_t s,
+                     const TR* r = nullptr, const T* scale = nullptr);
 template <typename T>
 void launch_prolong_add(const Geom& fine, const Geom& coarse, const T* xc, T* xf, const uint8_t* bcf,
                         hipStream_t s);
+// what a restriction leaves besides the coarse right-hand side b: nothing, the first smoothing step
+// d = x = c dinv b (x set), or b in double precision (wide set)
+template <typename T>
+struct RestrictOut {
+  T c = 0;
+  const T* dinv = nullptr;
+  T *d = nullptr, *x = nullptr;
+  double* wide = nullptr;
+};
 template <typename T>
 void launch_restrict2(const Geom& fine, const Geom& coarse, const T* rf, T* rc, const uint8_t* bcc,
-                      const uint8_t* bcf, hipStream_t s);
+                      const uint8_t* bcf, const RestrictOut<T>& out, hipStream_t s);
 void set_apply_chunk(int kz3, int kz2);
 long dvc_scratch_bytes(int dim, int num, int max_np, int cap);
 bool dvc_wave_supported(int dim, int num);
@@ -251,7 +262,8 @@ void vk_cheb_first(long n, T c, const T* dinv, const T* b, T* d, T* x, hipStream
 // r = b - r  (r holds A x on input)
 template <typename T> void vk_residual(long n, const T* b, T* r, hipStream_t s);
 // dense coarse solve y = Ainv x for a small dense inverse (double)
-void launch_dense_mv(int n, const double* A, const double* x, double* y, hipStream_t s);
+template <typename T>
+void launch_dense_mv(int n, const double* A, const double* x, T* y, hipStream_t s);
 // dense inverse of the coarsest level's operator (identity Dirichlet rows), n = N dim; work:
 // a second n x n buffer
 void launch_coarse_inverse(const Geom& g, const double* W, const uint8_t* bc, double* Ainv, double* work, int* flag,
