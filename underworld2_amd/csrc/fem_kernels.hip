@@ -2489,32 +2489,91 @@ __global__ void k_coarse_dense(Geom g, const double* __restrict__ W, const uint8
   K[t] = acc;
 }
 
-// One Gauss-Jordan step of the inverse of a symmetric positive definite n x n matrix
-// (row-major), pivot k, from A into B (two buffers, so no entry is read after another
-// workgroup overwrote it): with row = A[k][:] / p, row[k] = 1 / p, col = A[:][k],
-//   B[k][j] = row[j],   B[i][j] = (j == k ? 0 : A[i][j]) - col[i] row[j]  (i != k).
-// After steps k = 0 .. n-1 the last buffer holds the inverse (no pivoting, which SPD matrices
-// do not need).  flag[0] = 1 on a non-positive pivot.
-__global__ void k_gj_step(int n, int k, const double* __restrict__ A, double* __restrict__ B, int* __restrict__ flag) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)n * n) return;
-  const double p = A[(long)k * n + k];
-  if (t == 0 && !(p > 0.0)) flag[0] = 1;
-  const int i = (int)(t / n), j = (int)(t % n);
-  const double ip = 1.0 / p;
-  const double rj = j == k ? ip : A[(long)k * n + j] * ip;
-  B[t] = i == k ? rj : (j == k ? 0.0 : A[t]) - A[(long)i * n + k] * rj;
+// Gauss-Jordan steps k .. k + m - 1 (m <= GJ_M) of the inverse of a symmetric positive definite
+// n x n matrix (row-major), from A into B (two buffers, so no entry is read after another
+// workgroup overwrote it).  One step, with pivot k, row = A[k][:] / p, row[k] = 1 / p, is
+//   B[k][j] = row[j],   B[i][j] = (j == k ? 0 : A[i][j]) - A[i][k] row[j]  (i != k).
+// After steps 0 .. n-1 the last buffer holds the inverse (no pivoting, which SPD matrices do not
+// need).  flag[0] = 1 on a non-positive pivot.
+//
+// Entry (i, j) after m steps follows from the pivot rows' and columns' entries at i and j and the
+// m x m pivot block, so a workgroup carries those along for its 16 x 64 entries, each through
+// the same operations as step by step (the same bits).  A launch per step was n launches of
+// 3.2 - 3.8 us for microseconds' worth of traffic: 578 unknowns 2.2 ms, in eights 0.7 ms.
+constexpr int GJ_M = 8, GJ_I = 16, GJ_J = 64;
+__global__ __launch_bounds__(256) void k_gj_steps(int n, int k, int m, const double* __restrict__ A,
+                                                  double* __restrict__ B, int* __restrict__ flag) {
+  __shared__ double R[GJ_M][GJ_J], C[GJ_I][GJ_M], P[GJ_M][GJ_M];
+  const int t = threadIdx.x, i0 = blockIdx.y * GJ_I, j0 = blockIdx.x * GJ_J;
+  const int lj = t & 63, j = j0 + lj, li = t >> 6;  // entries (i0 + li + 4 r, j)
+  for (int q = t; q < GJ_M * GJ_J; q += 256) {
+    const int s = q / GJ_J, c = j0 + q % GJ_J;
+    R[s][q % GJ_J] = s < m && c < n ? A[(long)(k + s) * n + c] : 0.0;
+  }
+  if (t < GJ_I * GJ_M) {
+    const int s = t % GJ_M, r = i0 + t / GJ_M;
+    C[t / GJ_M][s] = s < m && r < n ? A[(long)r * n + k + s] : 0.0;
+  }
+  if (t < GJ_M * GJ_M) {
+    const int s = t / GJ_M, u = t % GJ_M;
+    P[s][u] = s < m && u < m ? A[(long)(k + s) * n + k + u] : 0.0;
+  }
+  double a[GJ_I / 4];
+#pragma unroll
+  for (int r = 0; r < GJ_I / 4; r++) {
+    const int i = i0 + li + 4 * r;
+    a[r] = i < n && j < n ? A[(long)i * n + j] : 0.0;
+  }
+  // one entry through step s: row and column index relative to the pivot (0: the pivot itself)
+  auto step = [](bool prow, bool pcol, double v, double col, double row) {
+    return prow ? row : fma_t(-col, row, pcol ? 0.0 : v);
+  };
+  for (int s = 0; s < m; s++) {
+    __syncthreads();
+    const double p = P[s][s], ip = 1.0 / p;
+    if (t == 0 && blockIdx.x == 0 && blockIdx.y == 0 && !(p > 0.0)) flag[0] = 1;
+    const double rj = j == k + s ? ip : R[s][lj] * ip;
+#pragma unroll
+    for (int r = 0; r < GJ_I / 4; r++) {
+      const int i = li + 4 * r;
+      a[r] = step(i0 + i == k + s, j == k + s, a[r], C[i][s], rj);
+    }
+    double nr[2], nc = 0.0, np = 0.0;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      const int u = li + 4 * r;
+      nr[r] = step(u == s, j == k + s, R[u][lj], P[u][s], rj);
+    }
+    const int cs = t % GJ_M, ci = t / GJ_M;
+    if (t < GJ_I * GJ_M) {
+      const double rp = cs == s ? ip : P[s][cs] * ip;
+      nc = step(i0 + ci == k + s, cs == s, C[ci][cs], C[ci][s], rp);
+      if (t < GJ_M * GJ_M) np = step(ci == s, cs == s, P[ci][cs], P[ci][s], rp);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; r++) R[li + 4 * r][lj] = nr[r];
+    if (t < GJ_I * GJ_M) C[ci][cs] = nc;
+    if (t < GJ_M * GJ_M) P[ci][cs] = np;
+  }
+#pragma unroll
+  for (int r = 0; r < GJ_I / 4; r++) {
+    const int i = i0 + li + 4 * r;
+    if (i < n && j < n) B[(long)i * n + j] = a[r];
+  }
 }
 
 // Ainv (n x n) = inverse of the coarsest level's operator; work: a second n x n buffer
 void launch_coarse_inverse(const Geom& g, const double* W, const uint8_t* bc, double* Ainv, double* work, int* flag,
                            hipStream_t s) {
   const long n = g.N * g.dim;
-  // n steps alternate between the two buffers: start in the one that ends in Ainv
-  double* bufs[2] = {(n % 2) ? work : Ainv, (n % 2) ? Ainv : work};
+  // the launches alternate between the two buffers: start in the one that ends in Ainv
+  const int launches = (int)((n + GJ_M - 1) / GJ_M);
+  double* bufs[2] = {(launches % 2) ? work : Ainv, (launches % 2) ? Ainv : work};
   hipLaunchKernelGGL(k_coarse_dense, nblocks(n * n, 256), 256, 0, s, g, W, bc, bufs[0]);
-  for (int k = 0; k < (int)n; k++)
-    hipLaunchKernelGGL(k_gj_step, nblocks(n * n, 256), 256, 0, s, (int)n, k, bufs[k & 1], bufs[(k + 1) & 1], flag);
+  for (int l = 0; l < launches; l++)
+    hipLaunchKernelGGL(k_gj_steps, dim3(nblocks(n, GJ_J), nblocks(n, GJ_I)), 256, 0, s, (int)n, l * GJ_M,
+                       std::min(GJ_M, (int)n - l * GJ_M), bufs[l & 1], bufs[(l + 1) & 1], flag);
   UWG_HIP(hipGetLastError());
 }
 
