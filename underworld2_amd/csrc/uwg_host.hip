@@ -71,6 +71,70 @@ struct uwg_field {
   double* d;
 };
 
+// Host memory that the device reads and writes, for short lists of points and values: buffers of
+// 64 KB, one per call in progress; up to eight wait for the next call and are freed with the
+// process's last field.
+class HostBuffers {
+ public:
+  static constexpr size_t kBytes = 65536;
+  class Lease {
+   public:
+    Lease() : p_(pool().take()) {}
+    ~Lease() { pool().put(p_); }
+    Lease(const Lease&) = delete;
+    Lease& operator=(const Lease&) = delete;
+    unsigned char* get() const { return p_; }
+
+   private:
+    unsigned char* p_;
+  };
+  static void field_created() {
+    HostBuffers& b = pool();
+    std::lock_guard<std::mutex> lk(b.mu_);
+    b.fields_++;
+  }
+  static void field_destroyed() {
+    HostBuffers& b = pool();
+    std::lock_guard<std::mutex> lk(b.mu_);
+    if (--b.fields_ > 0) return;
+    for (unsigned char* p : b.free_) (void)hipHostFree(p);
+    b.free_.clear();
+  }
+
+ private:
+  HostBuffers() { free_.reserve(8); }
+  static HostBuffers& pool() {
+    static HostBuffers* b = new HostBuffers();  // outlives every field
+    return *b;
+  }
+  unsigned char* take() {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (!free_.empty()) {
+        unsigned char* p = free_.back();
+        free_.pop_back();
+        return p;
+      }
+    }
+    void* p = nullptr;
+    UWG_HIP(hipHostMalloc(&p, kBytes, hipHostMallocPortable));
+    return (unsigned char*)p;
+  }
+  void put(unsigned char* p) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (free_.size() < 8) {
+        free_.push_back(p);
+        return;
+      }
+    }
+    (void)hipHostFree(p);
+  }
+  std::mutex mu_;
+  std::vector<unsigned char*> free_;
+  long fields_ = 0;
+};
+
 struct uwg_swarm {
   uwg_mesh* mesh;
   long P = 0, cap = 0;
@@ -189,6 +253,8 @@ struct uwg_stokes {
   double* red_out = nullptr;
   double* dcoef = nullptr;
   double* dh = nullptr;  // Gram-Schmidt coefficients of the current Arnoldi step (device)
+  HostColumn* hcol = nullptr;  // and where the device reports them
+  unsigned long long hcol_seq = 0;
   const double** dptrs = nullptr;
   int levels_req = 0;
   // learned correction
@@ -388,12 +454,16 @@ extern "C" int uwg_field_create(uwg_mesh* m, int ncomp, int on_elements, uwg_fie
   f->n = nent * ncomp;
   f->d = dalloc<double>(f->n);
   UWG_HIP(hipMemset(f->d, 0, sizeof(double) * f->n));
+  HostBuffers::field_created();
   *out = f;
   return 0;
   API_END
 }
 extern "C" int uwg_field_destroy(uwg_field* f) {
-  if (f) dfree(f->d);
+  if (f) {
+    dfree(f->d);
+    HostBuffers::field_destroyed();
+  }
   delete f;
   return 0;
 }
@@ -792,6 +862,24 @@ extern "C" int uwg_field_interpolate(uwg_field* f, long n, const double* x, doub
   if (f->ncomp < 1 || f->ncomp > 9) return arg_error("fields of 1 to 9 components can be interpolated");
   API_BEGIN
   const int dim = f->mesh->g.dim, nc = f->ncomp;
+  // A short list (64 KB: 1260 points of a 3D vector field) goes through host memory: one launch and
+  // one wait.  Three allocations, three copies and three frees around a kernel of 5 us made a call
+  // of 10 points 57 us; now 23.  Longer lists read the points over the host link more slowly than
+  // a copy moves them.
+  if (n > 0 && (size_t)n <= HostBuffers::kBytes / (sizeof(double) * (dim + nc) + sizeof(int))) {
+    HostBuffers::Lease io;
+    double *hx = (double*)io.get(), *hv = hx + n * dim;
+    int* hok = (int*)(hv + n * nc);
+    memcpy(hx, x, sizeof(double) * n * dim);
+    if (f->mesh->order == 2)
+      launch_q2_interpolate(f->mesh->g, n, f->d, nc, hx, hv, hok, 0);
+    else
+      launch_field_interpolate(f->mesh->g, n, f->d, nc, hx, hv, hok, 0);
+    UWG_HIP(hipStreamSynchronize(0));
+    memcpy(v, hv, sizeof(double) * n * nc);
+    memcpy(ok, hok, sizeof(int) * n);
+    return 0;
+  }
   double* dx = dalloc<double>(n * dim);
   double* dv = dalloc<double>(n * nc);
   int* dok = dalloc<int>(n);
@@ -1634,6 +1722,18 @@ static double dev_dot(uwg_stokes* st, long n, const T* a, const T* b) {
   return r;
 }
 
+// The reported column: polled for 100 us, which covers an iteration on the small grids and saves
+// a copy launch and the wake-up after it, then waited for with the stream.
+static void wait_column(uwg_stokes* st) {
+  const double t0 = now();
+  while (__atomic_load_n(&st->hcol->seq, __ATOMIC_ACQUIRE) != st->hcol_seq)
+    if (now() - t0 > 1e-4) {
+      UWG_HIP(hipStreamSynchronize(0));
+      if (__atomic_load_n(&st->hcol->seq, __ATOMIC_ACQUIRE) != st->hcol_seq)
+        throw std::runtime_error("Gram-Schmidt step did not report its coefficients");
+    }
+}
+
 // Right-preconditioned FGMRES with classical Gram-Schmidt; vectors of type T, the Arnoldi
 // basis of type TV (T, or float under an FP64 iteration), every reduction and the Hessenberg
 // least-squares problem in double.  The preconditioner reads a basis vector.
@@ -1679,8 +1779,9 @@ static int fgmres(uwg_stokes* st, KSpaceT<T, TV>& K, const std::function<void(co
       M(K.V[j], K.Z[j]);
       A(K.Z[j], K.w);
       // Gram-Schmidt on the device; one copy of the Hessenberg column per iteration
-      vk_gs_step<T, TV>(n, j + 1, K.dV, K.w, K.V[j + 1], st->dh, st->red_partial, 0);
-      UWG_HIP(hipMemcpy(hcol.data(), st->dh, sizeof(double) * (j + 2), hipMemcpyDeviceToHost));
+      vk_gs_step<T, TV>(n, j + 1, K.dV, K.w, K.V[j + 1], st->dh, st->red_partial, st->hcol, ++st->hcol_seq, 0);
+      wait_column(st);
+      std::copy(st->hcol->h, st->hcol->h + j + 2, hcol.begin());
       double hn = sqrt(std::max(0.0, hcol[j + 1]));
       hcol[j + 1] = hn;
       // Givens
@@ -1806,6 +1907,8 @@ extern "C" int uwg_stokes_create(uwg_field* vel, uwg_field* p, const unsigned ch
   st->red_out = dalloc<double>(8);
   st->dcoef = dalloc<double>(256);
   st->dh = dalloc<double>(256);
+  UWG_HIP(hipHostMalloc((void**)&st->hcol, sizeof(HostColumn)));
+  st->hcol->seq = 0;
   UWG_HIP(hipMalloc(&st->dptrs, sizeof(double*) * 256));
   *out = st;
   return 0;
@@ -1839,6 +1942,7 @@ extern "C" int uwg_stokes_destroy(uwg_stokes* st) {
                   (void*)st->force_tab, (void*)st->eta_p, (void*)st->force_p, (void*)st->red_partial,
                   (void*)st->red_out, (void*)st->dcoef, (void*)st->dh, (void*)st->dptrs, (void*)st->coarse.Ainv})
     dfree(p);
+  if (st->hcol) (void)hipHostFree(st->hcol);
   delete st;
   return 0;
 }

@@ -251,8 +251,15 @@ void vk_multi_dot(long n, int k, const T* x, const T* const* Y, double* partial,
 // w -= sum h_j V_j, h[k] = |w|^2 (bit-identical to a separate dot), v_next = w / |w| (skipped
 // when |w| = 0).  The basis V (and v_next) may be stored in a narrower type TV than w; every
 // product and sum is in double.  partial holds 32 x vk_reduce_blocks() doubles
+// a Gram-Schmidt step's coefficients in host memory that the device writes; seq is written last.
+// Room for restarts up to 255, as in the device's copy.
+struct HostColumn {
+  double h[256];
+  unsigned long long seq;
+};
 template <typename TW, typename TV>
-void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, hipStream_t s);
+void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, HostColumn* out,
+                unsigned long long seq, hipStream_t s);
 int vk_reduce_blocks();
 // chebyshev helper: d = a*d + b*(dinv .* r) ; x += d  (fused)
 template <typename T>
