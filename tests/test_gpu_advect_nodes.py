@@ -1,0 +1,25 @@
+"""RK2 advection with the axes' node coordinates in a table of up to 4096 nodes and without one: bit
+for bit the oracle on both sides of the limit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("res", [(1, 1), (13, 7), (4093, 1), (4094, 1), (2, 1, 3), (3, 2, 4088), (3, 2, 4089)])
+def test_positions_are_the_oracle_s(res):
+    from oracle import oracle as O
+    import underworld2_amd as uw
+    d = len(res)
+    lo, hi = (-0.3, 0.1, 0.0)[:d], (1.1, 0.9, 2.0)[:d]
+    rng = np.random.default_rng(7)
+    mesh = uw.mesh.FeMesh_Cartesian("Q1/dQ0", res, lo, hi)
+    vel = uw.mesh.MeshVariable(mesh, d)
+    vel.data[:] = rng.standard_normal(vel.data.shape)
+    sw = uw.swarm.Swarm(mesh)
+    x = np.array(lo) + rng.random((3000, d)) * (np.array(hi) - np.array(lo))
+    sw.add_particles_with_coordinates(x)
+    dt = 0.2 * min((h - l) / r for l, h, r in zip(lo, hi, res))  # a few midpoints leave the box
+    want, bad, _ = O.advect_rk2(O.Mesh(res, lo, hi), vel.data.copy(), x, dt)
+    uw.systems.SwarmAdvector(vel, sw, order=2).integrate(dt, update_owners=False)
+    assert np.array_equal(sw.particleCoordinates.data, want)
