@@ -1,5 +1,5 @@
 """Passes joined in the Krylov step and the multigrid cycle: Gram-Schmidt with the norm in the update
-(up to 2^18 unknowns) and separate from it, dot products over 1 to 40 vectors (groups of eight, a
+(up to 2^20 unknowns) and separate from it, dot products over 1 to 40 vectors (groups of eight, a
 second batch after 32), G added into the operator's result, G^T with the pressure preconditioner, the
 restriction with the first smoothing step."""
 import numpy as np
@@ -22,9 +22,9 @@ def _stokes(res):
     return uw, st, vel, p
 
 
-# 4305 (odd) and 214 unknowns; 48^3: 463,539, above 2^18
+# 4305 (odd) and 214 unknowns; 48^3: 463,539, two per thread; 72^3: 1,540,299, above 2^20
 @pytest.mark.parametrize("res,restart", [((6, 10, 14), 3), ((6, 10, 14), 9), ((6, 10, 14), 40), ((10, 6), 17),
-                                         ((48, 48, 48), 40)])
+                                         ((48, 48, 48), 40), ((72, 72, 72), 40)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_residual_of_the_unjoined_operators(res, restart, precision):
     """The residual that uwg_stokes_residuals forms with separate K, G, G^T and vector passes is the

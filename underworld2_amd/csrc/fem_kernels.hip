@@ -2329,16 +2329,15 @@ __global__ void k_gs_update_pairs(long n, int k, const TV* const* V, const doubl
   }
 }
 
-// the same update with the partial sums of |w|^2 that k_sqnorm forms, one element per thread
-// (n <= 256 RB: k_sqnorm's threads have one element each there)
+// the same update, one element at a time in the order of k_sqnorm, with the partial sums of |w|^2
+// that k_sqnorm forms
 template <typename TW, typename TV>
 __global__ __launch_bounds__(256) void k_gs_update_norm(long n, int k, const TV* const* V,
                                                         const double* __restrict__ h, TW* __restrict__ w,
                                                         double* partial) {
   __shared__ double sm[1][4];
   double acc[1] = {0.0};
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) {
+  for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
     double a = (double)w[i];
 #pragma unroll 8
     for (int j = 0; j < k; j++) a += (-h[j]) * (double)V[j][i];
@@ -2390,11 +2389,12 @@ __global__ void k_scale_by_norm(long n, int k, const double* __restrict__ h, con
 
 // The update runs on the streaming grid (a reduction-sized grid holds too few loads in flight
 // for the k-vector gather); |w|^2 is then the one-vector dot of vk_multi_dot.  V[j] and w must
-// be whole allocations (16-byte aligned) for the paired loads of the dot products.  Up to 256 RB
+// be whole allocations (16-byte aligned) for the paired loads of the dot products.  Up to 1024 RB
 // elements the norm comes with the update and its sum with the scaling, four launches instead of
 // six, all of them latency.  A step over 30 vectors of 33^3 velocities and 32^3 pressures:
 // dot products 24.9 -> 13.7 us, the rest 24 -> 13 us; 128^3 (two-pass form): dot products
-// 283 -> 198 us (4.4 TB/s).  The sums are the same bits on both paths.
+// 283 -> 198 us (4.4 TB/s).  With two elements a thread (352,947 unknowns of a Q2 solve) a solve is
+// 1.4 % shorter than with six launches; further up the passes are the cost.  The sums are the same bits on both paths.
 template <typename TW, typename TV>
 void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, HostColumn* out,
                 unsigned long long seq, hipStream_t s) {
@@ -2403,10 +2403,10 @@ void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h,
     const int nb = mdot_pairs_pass<TW, TV>(n, kk, w, V + j0, partial, s);
     hipLaunchKernelGGL(k_mdot_final, kk, 256, 0, s, partial, nb, h + j0);
   }
-  if (n <= 256L * RB) {
+  if (n <= 1024L * RB) {
     const int nb = reduce_blocks(n);
     hipLaunchKernelGGL((k_gs_update_norm<TW, TV>), nb, 256, 0, s, n, k, V, h, w, partial);
-    hipLaunchKernelGGL((k_sum_scale_by_norm<TW, TV>), nb, 256, 0, s, n, partial, nb, k, h, w, v_next, out, seq);
+    hipLaunchKernelGGL((k_sum_scale_by_norm<TW, TV>), (unsigned)((n + 255) / 256), 256, 0, s, n, partial, nb, k, h, w, v_next, out, seq);
     UWG_HIP(hipGetLastError());
     return;
   }
