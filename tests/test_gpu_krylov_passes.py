@@ -22,9 +22,9 @@ def _stokes(res):
     return uw, st, vel, p
 
 
-# 4305 (odd) and 214 unknowns; 48^3: 463,539, two per thread; 72^3: 1,540,299, above 2^20
+# 4305 (odd) and 214 unknowns; 48^3: 463,539, two per thread; 64^3: 1,086,019, above 2^20
 @pytest.mark.parametrize("res,restart", [((6, 10, 14), 3), ((6, 10, 14), 9), ((6, 10, 14), 40), ((10, 6), 17),
-                                         ((48, 48, 48), 40), ((72, 72, 72), 40)])
+                                         ((48, 48, 48), 40), ((64, 64, 64), 40)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_residual_of_the_unjoined_operators(res, restart, precision):
     """The residual that uwg_stokes_residuals forms with separate K, G, G^T and vector passes is the

@@ -87,3 +87,20 @@ def test_divergence_matches_the_gradient(res):
         assert abs(_apply(st, 1, p, n) @ u - q[i]) < 81 * 16 * np.finfo(np.float64).eps * scale
     p = rng.standard_normal(m)
     assert abs(_apply(st, 1, p, n) @ u - q @ p) < 16 * np.sqrt(n) * np.finfo(np.float64).eps * np.abs(q) @ np.abs(p)
+
+
+@pytest.mark.parametrize("res", [(1, 1), (3, 3), (1, 1, 1), (3, 1, 1), (5, 3, 1)])
+def test_schur_blocks_of_ragged_element_counts(res):
+    """approxS blocks against the oracle's where the elements leave workgroups partly empty (four
+    per workgroup in 3D, eight in 2D): sums of 81 terms of one sign pattern, 1e-12 of the largest."""
+    from oracle import q2_oracle as Q
+    import underworld2_amd._lib as L
+    dim = len(res)
+    st, _, _ = _stokes(res)
+    om = Q.Q2Mesh(res, (0.0,) * dim, (1.0, 0.8, 0.7)[:dim])
+    Ke, _ = Q.gauss_assembly(om, lambda X: 1.0 + 3.0 * X[:, 0] * X[:, 1],
+                             lambda X: np.stack([0 * X[:, 0]] * (dim - 1) + [-1.0 + 0 * X[:, 0]], -1))
+    S = np.zeros((om.E, om.npe, om.npe))
+    L.check(L.lib().uwg_stokes_get_assembly(st._h, 0, None, None, L.dptr(S)), "assembly")
+    want = Q.element_approxS(Ke, Q.element_G(om))
+    assert np.abs(S - want).max() < 1e-12 * np.abs(want).max()

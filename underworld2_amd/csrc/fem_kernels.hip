@@ -2394,7 +2394,8 @@ __global__ void k_scale_by_norm(long n, int k, const double* __restrict__ h, con
 // six, all of them latency.  A step over 30 vectors of 33^3 velocities and 32^3 pressures:
 // dot products 24.9 -> 13.7 us, the rest 24 -> 13 us; 128^3 (two-pass form): dot products
 // 283 -> 198 us (4.4 TB/s).  With two elements a thread (352,947 unknowns of a Q2 solve) a solve is
-// 1.4 % shorter than with six launches; further up the passes are the cost.  The sums are the same bits on both paths.
+// 1.4 % shorter than with six launches; further up the passes are the cost.  The sums are the
+// same bits on both paths.
 template <typename TW, typename TV>
 void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, HostColumn* out,
                 unsigned long long seq, hipStream_t s) {

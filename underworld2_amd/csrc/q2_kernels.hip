@@ -1054,25 +1054,35 @@ template void launch_q2_apply_GT<float>(const Geom&, const double*, const float*
 // ---------------------------------------------------------------------------------------
 // approxS_e = G_e^T diag(K_e)^-1 G_e (UzawaPreconditionerTerm.c:124-209), stored inverted
 // ---------------------------------------------------------------------------------------
+// A group of 32 (16 in 2D) lanes per element: a lane per vertex forms its diagonal entries, a lane
+// per block entry sums them over the vertices in order, the first lane inverts the block.  One
+// thread per element walked the 27 x 125 points by itself, 1.40 ms at 24^3 elements on 216
+// one-wave workgroups, against 0.22 ms.
 template <int DIM>
-__global__ void k_q2_approxS(Q2G G, const double* __restrict__ W, const double* __restrict__ Gr,
-                             double* __restrict__ S, double* __restrict__ Sinv, int* __restrict__ bad) {
-  constexpr int NP = DIM + 1, NEN = DIM == 3 ? 27 : 9;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= G.E) return;
-  double M[NP][NP] = {};
-  for (int a = 0; a < NEN; a++) {
+__global__ __launch_bounds__(128) void k_q2_approxS(Q2G G, const double* __restrict__ W, const double* __restrict__ Gr,
+                                                    double* __restrict__ S, double* __restrict__ Sinv,
+                                                    int* __restrict__ bad) {
+  constexpr int NP = DIM + 1, NEN = DIM == 3 ? 27 : 9, LANES = DIM == 3 ? 32 : 16, PER = 128 / LANES;
+  static_assert(NP * NP <= LANES, "a lane per entry");
+  __shared__ double kinv[PER][NEN * DIM], block[PER][NP * NP];
+  const int sub = threadIdx.x / LANES, l = threadIdx.x % LANES;
+  const long e = (long)blockIdx.x * PER + sub;
+  if (l < NEN && e < G.E) {
     double kd[3] = {0.0, 0.0, 0.0};
-    q2_kdiag_elem<DIM>(G, W, e, a, kd);
-    for (int i = 0; i < DIM; i++) {
-      const double* gv = Gr + (a * DIM + i) * NP;
-      const double inv = 1.0 / kd[i];
-      for (int r = 0; r < NP; r++)
-        for (int c = 0; c < NP; c++) M[r][c] += gv[r] * gv[c] * inv;
-    }
+    q2_kdiag_elem<DIM>(G, W, e, l, kd);
+    for (int i = 0; i < DIM; i++) kinv[sub][l * DIM + i] = 1.0 / kd[i];
   }
-  for (int r = 0; r < NP; r++)
-    for (int c = 0; c < NP; c++) S[e * NP * NP + r * NP + c] = M[r][c];
+  __syncthreads();
+  if (l < NP * NP && e < G.E) {
+    const int r = l / NP, c = l % NP;
+    double m = 0.0;
+    for (int k = 0; k < NEN * DIM; k++) m += Gr[k * NP + r] * Gr[k * NP + c] * kinv[sub][k];
+    block[sub][l] = m;
+    S[e * NP * NP + l] = m;
+  }
+  __syncthreads();
+  if (l > 0 || e >= G.E) return;
+  const double(*M)[NP] = reinterpret_cast<const double(*)[NP]>(block[sub]);
   // Gauss-Jordan inverse (symmetric positive definite block)
   double A[NP][2 * NP];
   for (int r = 0; r < NP; r++)
@@ -1112,9 +1122,9 @@ void launch_q2_approxS(const Geom& g, const double* W, const double* Gr, double*
                        hipStream_t s) {
   const Q2G G = q2_pack(g);
   if (g.dim == 3)
-    hipLaunchKernelGGL(k_q2_approxS<3>, q2_blocks(G.E, 64), 64, 0, s, G, W, Gr, S, Sinv, bad);
+    hipLaunchKernelGGL(k_q2_approxS<3>, q2_blocks(G.E, 4), 128, 0, s, G, W, Gr, S, Sinv, bad);
   else
-    hipLaunchKernelGGL(k_q2_approxS<2>, q2_blocks(G.E, 64), 64, 0, s, G, W, Gr, S, Sinv, bad);
+    hipLaunchKernelGGL(k_q2_approxS<2>, q2_blocks(G.E, 8), 128, 0, s, G, W, Gr, S, Sinv, bad);
   UWG_HIP(hipGetLastError());
 }
 
