@@ -1565,13 +1565,6 @@ static void ensure_snn_coefficients(uwg_stokes* st) {
   schur_net_coefficients(st->snn.get(), st->g, st->approxS, st->snn_a, 0);
   st->snn_stamp = st->assembly_stamp;
 }
-template <typename T>
-static void schur_prec(uwg_stokes* st, const T* diagS, const T* r, T* z) {
-  if (g_snn_active && st->snn && !st->nn_disabled)
-    schur_stencil_apply<T>(st->g, st->snn_a, r, z, 0);
-  else
-    top_schur<T>(st, diagS, r, z);
-}
 // the pressure row of the block preconditioner, z = -S^-1 (r - G^T u); q: a pressure vector, wide: one
 // in T for a narrower r
 template <typename T, typename TR>
