@@ -268,9 +268,9 @@ int uwg_snn_eval(uwg_snn *h, long first, long count, float *loss);
 int uwg_stokes_load_schur_nn(uwg_stokes *st, int channels, int layers, long nparams, const float *params);
 /* kernel-apply tuning knob: node levels per workgroup of the 3D K apply (kz3 > 0 fixes it on
  * every grid; kz3 < 0 restores the default, chosen per grid to fill the GPU's resident
- * workgroup slots evenly), element rows per block of the 2D K apply (kz2 > 0; 32, the
- * default, lets the grid decide: the assembled operator up to 150,000 vertices, then at most 32);
- * zero leaves a setting unchanged */
+ * workgroup slots evenly), element rows per block of the 2D K apply (kz2 > 0 fixes it on every
+ * grid; kz2 < 0 restores the default, the assembled operator up to 150,000 vertices and at most
+ * 32 rows above); zero leaves a setting unchanged */
 int uwg_set_apply_chunk(int kz3, int kz2);
 /* 3D Q2 K apply kernel: sum-factorised (2, default), matrix cores (1) or the dense vector
  * kernel (0); uwg_set_q2_mfma(on) selects 1 or 0 */

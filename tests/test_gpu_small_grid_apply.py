@@ -72,8 +72,26 @@ def test_2d_stencil_against_element_kernel(res, mask):
             e = e.ravel()
             diag += e * _apply(st, 0, e)
     finally:
-        L.lib().uwg_set_apply_chunk(0, 32)
+        L.lib().uwg_set_apply_chunk(0, -1)
     bound = 40 * 18 * diag.max() * np.abs(x).max()
     for a, b, u in zip(got, ref, (2.0 ** -53, 2.0 ** -24, 2.0 ** -53, 2.0 ** -24)):
         assert np.abs(a - b).max() <= u * bound
         assert np.linalg.norm(a - b) <= 20 * u * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("res", [(31, 29), (64, 5)])
+def test_2d_chunk_of_32_rows_is_a_chunk(res):
+    """Every chunk size selects the element kernel, whose sums do not depend on it, 32 as well; a
+    negative one restores the automatic choice, here the stencil, whose sums are ordered otherwise."""
+    from underworld2_amd import _lib as L
+    *keep, st, x = _system(res, (1.0, 1.3), 5)
+    auto = _apply(st, 0, x)
+    try:
+        got = []
+        for kz in (31, 32, 33):
+            L.lib().uwg_set_apply_chunk(0, kz)
+            got.append(_apply(st, 0, x))
+    finally:
+        L.lib().uwg_set_apply_chunk(0, -1)
+    assert np.array_equal(got[1], got[0]) and np.array_equal(got[1], got[2])
+    assert not np.array_equal(got[1], auto) and np.array_equal(_apply(st, 0, x), auto)

@@ -1471,9 +1471,8 @@ __global__ __launch_bounds__(128) void k_stencil(int nx, int nd, const T* __rest
 
 static int g_kz3 = 0, g_kz2 = 0;  // 0: automatic
 void set_apply_chunk(int kz3, int kz2) {
-  if (kz3 > 0) g_kz3 = kz3;
-  if (kz3 < 0) g_kz3 = 0;
-  if (kz2 > 0) g_kz2 = kz2 == 32 ? 0 : kz2;
+  if (kz3 != 0) g_kz3 = std::max(kz3, 0);
+  if (kz2 != 0) g_kz2 = std::max(kz2, 0);
 }
 
 // compute units of the current device (cached per device)
