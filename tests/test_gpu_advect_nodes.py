@@ -23,3 +23,23 @@ def test_positions_are_the_oracle_s(res):
     want, bad, _ = O.advect_rk2(O.Mesh(res, lo, hi), vel.data.copy(), x, dt)
     uw.systems.SwarmAdvector(vel, sw, order=2).integrate(dt, update_owners=False)
     assert np.array_equal(sw.particleCoordinates.data, want)
+
+
+def test_advection_that_keeps_owners_takes_no_relocation_workspace():
+    """The workspace (24 bytes per particle) is for calls that update owners; without, a step needs two
+    counters.  Allocations are whole 2 MiB pages."""
+    import ctypes
+    import torch
+    import underworld2_amd as uw
+    from underworld2_amd import _lib as L
+    mesh = uw.mesh.FeMesh_Cartesian("Q1/dQ0", (64, 64, 16), (0.0,) * 3, (1.0,) * 3)
+    vel = uw.mesh.MeshVariable(mesh, 3)
+    vel.data[:] = 0.0
+    sw = uw.swarm.Swarm(mesh)
+    sw.populate_using_layout(uw.swarm.layouts.PerCellRandomLayout(sw, 20, seed=3))  # 1.3 million
+    vel.evaluate(np.full((1, 3), 0.5))  # uploads the field
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    out = ctypes.c_long()
+    L.check(L.lib().uwg_advect_rk2(sw._h, vel._h, 1e-3, 0, ctypes.byref(out)))
+    assert before - torch.cuda.mem_get_info()[0] <= 2 << 20

@@ -38,3 +38,26 @@ def test_gradients_match_oracle(grid, B, C, Ly):
     assert err < 2e-5
     l2, g2 = net.loss_grad(grid, x, r, t)
     assert l2 == lg and np.array_equal(g2, gg)
+
+
+@pytest.mark.parametrize("grid,B,C", [((6, 5, 4), 2, 8), ((23, 20, 19), 1, 8)])  # one chunk, several
+def test_infinite_features_of_inactive_channels(grid, B, C):
+    """An infinite feature whose weights are negative only reaches inactive channels: their gradients
+    are zero there, and a product of the two is left out of the sums instead of making them NaN.  The
+    gradients are those for a large finite feature, which the same ReLUs drop, bit for bit."""
+    from underworld2_amd import learned
+    rng = np.random.default_rng(7)
+    E = int(np.prod(grid))
+    net = learned.StencilNet(C, 1, seed=4)
+    p = net.get_params()
+    w = p[:C * 9 * 27].reshape(C, 9, 27)
+    w[:, 2] = -np.abs(w[:, 2]) - 0.01
+    net.set_params(p)
+    x = rng.standard_normal((B, 9, E)).astype(np.float32)
+    r, t = (rng.standard_normal((B, E)).astype(np.float32) for _ in range(2))
+    out = []
+    for v in (np.inf, 1e30):
+        x[:, 2, E // 2] = v
+        out.append(net.loss_grad(grid, x, r, t))
+    assert np.isfinite(out[0][0]) and np.isfinite(out[0][1]).all()
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])

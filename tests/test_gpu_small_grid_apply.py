@@ -95,3 +95,30 @@ def test_2d_chunk_of_32_rows_is_a_chunk(res):
         L.lib().uwg_set_apply_chunk(0, -1)
     assert np.array_equal(got[1], got[0]) and np.array_equal(got[1], got[2])
     assert not np.array_equal(got[1], auto) and np.array_equal(_apply(st, 0, x), auto)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("where", ["inside", "first column", "last column", "dirichlet"])
+def test_2d_a_value_that_is_not_finite_stays_with_its_elements(where, value):
+    """As in the element kernel: the nodes around it and no others, and none beside its own row where
+    the value stands on a Dirichlet dof, whose column is zero."""
+    from underworld2_amd import _lib as L
+    res = (9, 6)
+    mesh, *keep, st, x = _system(res, (1.0, 1.3), 6)
+    nx = res[0] + 1
+    # free dofs: component 1 on the side walls, both inside; component 0 is fixed on the side walls
+    at = {"inside": 2 * (4 + 3 * nx), "first column": 2 * (3 * nx) + 1, "last column": 2 * (nx - 1 + 2 * nx) + 1,
+          "dirichlet": 2 * (nx - 1 + 3 * nx)}[where]
+    x[at] = value
+    got = [_apply(st, w, x) for w in (0, 4, 6, 7)]
+    try:
+        L.lib().uwg_set_apply_chunk(0, 1)
+        ref = [_apply(st, w, x) for w in (0, 4, 6, 7)]
+    finally:
+        L.lib().uwg_set_apply_chunk(0, -1)
+    assert all(0 < (~np.isfinite(b)).sum() <= 18 for b in ref)
+    for a, b, u in zip(got, ref, (2.0 ** -53, 2.0 ** -24, 2.0 ** -53, 2.0 ** -24)):
+        f = np.isfinite(b)
+        assert np.array_equal(np.isfinite(a), f)
+        # 36 products and sums of rounding u on either side of entries up to the largest row
+        assert np.abs(a[f] - b[f]).max() <= 40 * 18 * u * np.abs(b[f]).max()
