@@ -235,10 +235,9 @@ __global__ void k_conv_bwd_data(int B, int Ci, int Co, Grid3 g, const float* __r
 }
 
 // Sums of NV per-thread values over a workgroup of 256 into res, by halves (128, 64, ... 1): sixteen
-// values at a time cross the waves through LDS, then each wave finishes four of them.
+// values at a time cross the waves through LDS (sm), then each wave finishes four of them.
 template <int NV>
-__device__ __forceinline__ void block_sums(const float (&v)[NV], float* res) {
-  __shared__ float sm[16][256];
+__device__ __forceinline__ void block_sums(const float (&v)[NV], float (*sm)[256], float* res) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int g = 0; g < NV; g += 16) {
@@ -256,18 +255,40 @@ __device__ __forceinline__ void block_sums(const float (&v)[NV], float* res) {
   }
 }
 
+// The weight sums of k_wgrad3's points t0 .. t1 - 1 without the products of zero output gradients,
+// whose inputs may be infinite; one sum at a time, in the same order.
+template <int COB>
+__device__ __noinline__ void wgrad3_active(int Ci, int Co, Grid3 g, const float* dout, const float* in, int ci,
+                                           int co0, int t0, int t1, float (*sm)[256], float* sum) {
+  const int N = (int)g.N(), nx = g.nx, ny = g.ny, nz = g.nz, nxy = nx * ny;
+  for (int c = 0; c < COB; c++)
+    for (int tap = 0; tap < 27; tap++) {
+      float acc[1] = {0.0f};
+      for (int t = t0 + (int)threadIdx.x; t < t1; t += 256) {
+        const int b = t / N, p = t - b * N, k = p / nxy, r = p - k * nxy, j = r / nx, i = r - j * nx;
+        const int ii = i + tap % 3 - 1, jj = j + (tap / 3) % 3 - 1, kk = k + tap / 9 - 1;
+        const float go = dout[(size_t)(b * Co + min(co0 + c, Co - 1)) * N + p];
+        if (go != 0.0f && ii >= 0 && ii < nx && jj >= 0 && jj < ny && kk >= 0 && kk < nz)
+          acc[0] += go * in[(size_t)(b * Ci + ci) * N + ii + nx * jj + nxy * kk];
+      }
+      block_sums<1>(acc, sm, sum + c * 28 + tap);
+    }
+}
+
 // Weight and bias gradients of a 3x3x3 convolution,
 //   dw[co][ci][tap] = sum_b sum_p dout[b][co][p] in[b][ci][p + off(tap)],  db[co] = sum dout,
 // as partial sums part[chunk][Co Ci 27 + Co] of chunks of points, added up in FP64 by k_sum_parts
 // in chunk order (deterministic).  A thread holds COB x 27 sums, so each of the 27 neighbours it
 // loads serves COB products, and the points are split so that every size fills the chip: one
 // workgroup per (co, ci) pair over all points took 6.0 ms for 16 x 16 channels at 4 x 48^3, this
-// 0.2 ms (bound by the loads of the neighbours, which hit the caches).
+// 0.2 ms (bound by the loads of the neighbours, which hit the caches).  An inactive unit's zero
+// gradient has no share in a sum even where the input is infinite: a workgroup with a sum that is
+// NaN forms its sums again without such products (229 us with the test and without).
 template <int COB>
 __global__ __launch_bounds__(256) void k_wgrad3(int B, int Ci, int Co, Grid3 g, const float* __restrict__ dout,
                                                 const float* __restrict__ in, int per, float* __restrict__ part) {
   constexpr int NV = COB * 28;  // the last of 28: the bias
-  __shared__ float sum[NV];
+  __shared__ float sum[NV], sm[16][256];
   const int ci = blockIdx.y, co0 = blockIdx.z * COB;
   const int N = (int)g.N(), nx = g.nx, ny = g.ny, nz = g.nz, nxy = nx * ny;
   const int T = B * N, t0 = blockIdx.x * per, t1 = min(t0 + per, T);
@@ -296,7 +317,9 @@ __global__ __launch_bounds__(256) void k_wgrad3(int B, int Ci, int Co, Grid3 g, 
 #pragma unroll
     for (int c = 0; c < COB; c++) acc[c * 28 + 27] += go[c];
   }
-  block_sums<NV>(acc, sum);
+  block_sums<NV>(acc, sm, sum);
+  if (__syncthreads_or(threadIdx.x < NV && sum[threadIdx.x] != sum[threadIdx.x]))
+    wgrad3_active<COB>(Ci, Co, g, dout, in, ci, co0, t0, t1, sm, sum);
   const long nw = (long)Co * Ci * 27;
   float* out = part + (long)blockIdx.x * (nw + Co);
   for (int q = threadIdx.x; q < NV; q += 256) {
@@ -316,7 +339,7 @@ template <int CB>
 __global__ __launch_bounds__(256) void k_wgrad1(int B, int Ci, long N, const float* __restrict__ gout,
                                                 const float* __restrict__ in, int per, float* __restrict__ part) {
   constexpr int NV = 9 * (CB + 1);
-  __shared__ float sum[NV];
+  __shared__ float sum[NV], sm[16][256];
   const int c0 = blockIdx.y * CB, o0 = blockIdx.z * 9;
   const int n = (int)N, T = B * n, t0 = blockIdx.x * per, t1 = min(t0 + per, T);
   float acc[NV];
@@ -335,7 +358,7 @@ __global__ __launch_bounds__(256) void k_wgrad1(int B, int Ci, long N, const flo
       acc[o * (CB + 1) + CB] += go;
     }
   }
-  block_sums<NV>(acc, sum);
+  block_sums<NV>(acc, sm, sum);
   float* out = part + (long)blockIdx.x * (27L * Ci + 27);
   for (int q = threadIdx.x; q < NV; q += 256) {
     const int o = o0 + q / (CB + 1), c = q % (CB + 1);
