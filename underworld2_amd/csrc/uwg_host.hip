@@ -147,6 +147,7 @@ struct uwg_swarm {
   double* w_slot = nullptr;   // [cap]
   int* slot_cell = nullptr;   // [cap]
   int* dvc_work = nullptr;    // element lists of the DVC, [2 E + 4]
+  int* moves = nullptr;       // counters of an advection step that leaves the owners, [2]
   bool has_mat = false;
   bool has_integration = false;
   long state = 0;             // bumps whenever particles or their materials change (assembly cache)
@@ -520,7 +521,7 @@ extern "C" int uwg_swarm_create(uwg_mesh* m, uwg_swarm** out) {
 extern "C" int uwg_swarm_destroy(uwg_swarm* s) {
   if (!s) return 0;
   for (void* p : {(void*)s->coords, (void*)s->owner, (void*)s->cell_ptr, (void*)s->cell_pid, (void*)s->mat,
-                  (void*)s->xi_slot, (void*)s->w_slot, (void*)s->slot_cell, (void*)s->dvc_work})
+                  (void*)s->xi_slot, (void*)s->w_slot, (void*)s->slot_cell, (void*)s->dvc_work, (void*)s->moves})
     dfree(p);
   reloc_destroy(s->reloc);
   for (int v = 0; v < 8; v++) dfree(s->var[v]);
@@ -820,15 +821,25 @@ extern "C" int uwg_advect_rk2(uwg_swarm* s, uwg_field* vel, double dt, int updat
   if (vel->mesh != s->mesh || vel->on_elements || vel->ncomp != s->mesh->g.dim)
     return arg_error("velocity field must be a nodal vector field on the swarm's mesh");
   API_BEGIN
-  ensure_reloc(s);
-  reloc_begin(s->reloc, 0);
-  launch_advect_rk2(s->mesh->g, s->P, vel->d, s->coords, dt, reloc_counters(s->reloc), 0, vel->mesh->order);
+  // with new owners the counts come back with the relocation's; without, its workspace (24 bytes
+  // per particle) is not needed
+  int* counts;
+  if (update_owners) {
+    ensure_reloc(s);
+    reloc_begin(s->reloc, 0);
+    counts = reloc_counters(s->reloc);
+  } else {
+    if (!s->moves) s->moves = dalloc<int>(2);
+    counts = s->moves;
+    UWG_HIP(hipMemset(counts, 0, sizeof(int) * 2));
+  }
+  launch_advect_rk2(s->mesh->g, s->P, vel->d, s->coords, dt, counts, 0, vel->mesh->order);
   int h[2] = {0, 0};  // particles without a velocity, first-order fallbacks
   long o = 0;
   if (update_owners)
     o = relocate(s->mesh->g, s->P, s->coords, s->owner, s->cell_ptr, s->cell_pid, s->reloc, 0, h);
   else
-    UWG_HIP(hipMemcpy(h, reloc_counters(s->reloc), sizeof(h), hipMemcpyDeviceToHost));
+    UWG_HIP(hipMemcpy(h, counts, sizeof(h), hipMemcpyDeviceToHost));
   s->state++;
   s->geom_state++;
   if (h[0] > 0) {
