@@ -55,3 +55,20 @@ def test_threads_share_a_field():
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not bad
+
+
+def test_a_call_that_reports_an_earlier_error_gives_its_buffer_back_idle():
+    """A failed allocation leaves an error that the next launch reports, with its kernel under way; the
+    call waits for it before the buffer serves another call."""
+    import ctypes
+    import underworld2_amd._lib as L
+    f = _field(1, 3, 3)
+    xs = [np.random.default_rng(k).uniform(0, 1, (1000, 3)) for k in range(2)]
+    ref = [_interp(f, x)[0] for x in xs]
+    for _ in range(20):
+        p = ctypes.c_void_p()
+        assert L.lib().hipMalloc(ctypes.byref(p), ctypes.c_size_t(1 << 60)) != 0
+        with pytest.raises(Exception):
+            _interp(f, xs[0])
+        assert np.array_equal(_interp(f, xs[1])[0], ref[1])
+    assert np.array_equal(_interp(f, xs[0])[0], ref[0])
