@@ -1784,7 +1784,8 @@ template void launch_apply_GT<float, float>(const Geom&, const double*, const fl
 // One thread per dof: on the small grids both kernels are bound by the latency of a few workgroups'
 // dependent loads, and a thread per vertex with three components made a third as many.  Restriction
 // to 17 x 13 x 21 vertices in double precision 13.7 -> 3.6 us including the first smoothing step
-// (a pass of 4.0 us before), to 17^3 in single 4.4 + 2.4 -> 3.6 us; 33^3 prolongation 3.9 -> 2.8 us.
+// (a pass of 4.0 us before), to 17^3 in single 4.4 + 2.4 -> 3.6 us, to 65^3 62.9 + 7.3 -> 26.3 us
+// in double and 13.2 + 5.2 -> 19.1 in single.
 template <typename T, int DIM>
 __global__ __launch_bounds__(128) void k_prolong_add(int fnx, int fny, int cnx, int cny, unsigned nf,
                                                      const T* __restrict__ xc, T* __restrict__ xf,
@@ -1814,6 +1815,35 @@ __global__ __launch_bounds__(128) void k_prolong_add(int fnx, int fny, int cnx, 
   if (odd[1]) wgt *= (T)0.5;
   if (DIM == 3 && odd[2]) wgt *= (T)0.5;
   xf[idx] = ((m >> d) & 1) ? old : old + wgt * acc;
+}
+
+// The same on large grids, a thread per vertex: its index arithmetic and mask serve all components
+// and only the parents there are load, 3.4 on average of the 8 of a thread per dof.  In us, vertex
+// against dof: FP64 49^3 5.4 against 4.4, 65^3 6.3 / 6.7, 97^3 14.0 / 17.9, 129^3 29.5 / 41.8; FP32
+// 4.3 / 4.1, 5.6 / 5.9, 9.7 / 13.7, 17.5 / 28.4; FP64 513^2 5.2 / 4.4, 1025^2 8.9 / 10.3, 2049^2
+// 34.5 / 37.0; FP32 5.0 / 3.6, 7.6 / 7.3, 27.3 / 25.1.
+template <typename T, int DIM>
+__global__ __launch_bounds__(256) void k_prolong_add_vertex(int fnx, int fny, int cnx, int cny, unsigned nf,
+                                                            const T* __restrict__ xc, T* __restrict__ xf,
+                                                            const uint8_t* __restrict__ bcf) {
+  const unsigned n = blockIdx.x * 256u + threadIdx.x;
+  if (n >= nf) return;
+  const unsigned row = n / fnx;
+  const int I = (int)(n % fnx), J = (int)(row % fny), K = (int)(row / fny);
+  T old[DIM], acc[DIM], wgt = (T)1;
+  for (int d = 0; d < DIM; d++) acc[d] = 0;
+  for (int c = 0; c <= (DIM == 3 ? (K & 1) : 0); c++)
+    for (int b = 0; b <= (J & 1); b++)
+      for (int a = 0; a <= (I & 1); a++) {
+        const long p = (I >> 1) + a + (long)cnx * ((J >> 1) + b + (DIM == 3 ? (long)cny * ((K >> 1) + c) : 0));
+        for (int d = 0; d < DIM; d++) acc[d] += xc[p * DIM + d];
+      }
+  const uint8_t m = bcf[n];
+  for (int d = 0; d < DIM; d++) old[d] = xf[(long)n * DIM + d];
+  if (I & 1) wgt *= (T)0.5;
+  if (J & 1) wgt *= (T)0.5;
+  if (DIM == 3 && (K & 1)) wgt *= (T)0.5;
+  for (int d = 0; d < DIM; d++) xf[(long)n * DIM + d] = ((m >> d) & 1) ? old[d] : old[d] + wgt * acc[d];
 }
 
 // OP 1: also the first smoothing step on the coarse level, dd = x = c dinv b (k_cheb_first);
@@ -1867,12 +1897,16 @@ __global__ __launch_bounds__(128) void k_restrict(int fnx, int fny, int fnz, int
 
 template <typename T>
 void launch_prolong_add(const Geom& f, const Geom& c, const T* xc, T* xf, const uint8_t* bcf, hipStream_t s) {
+  auto go = [&](auto kernel, long threads, int block) {
+    hipLaunchKernelGGL(kernel, nblocks(threads, block), block, 0, s, f.nn[0], f.nn[1], c.nn[0], c.nn[1],
+                       (unsigned)f.N, xc, xf, bcf);
+  };
+  // between the sizes measured on either side (figures above)
+  const bool vertex = f.dim == 3 ? f.N > 200000 : sizeof(T) == 8 && f.N > 500000;
   if (f.dim == 3)
-    hipLaunchKernelGGL((k_prolong_add<T, 3>), nblocks(f.N * 3, 128), 128, 0, s, f.nn[0], f.nn[1], c.nn[0], c.nn[1],
-                       (unsigned)f.N, xc, xf, bcf);
+    vertex ? go(k_prolong_add_vertex<T, 3>, f.N, 256) : go(k_prolong_add<T, 3>, f.N * 3, 128);
   else
-    hipLaunchKernelGGL((k_prolong_add<T, 2>), nblocks(f.N * 2, 128), 128, 0, s, f.nn[0], f.nn[1], c.nn[0], c.nn[1],
-                       (unsigned)f.N, xc, xf, bcf);
+    vertex ? go(k_prolong_add_vertex<T, 2>, f.N, 256) : go(k_prolong_add<T, 2>, f.N * 2, 128);
   UWG_HIP(hipGetLastError());
 }
 template void launch_prolong_add<double>(const Geom&, const Geom&, const double*, double*, const uint8_t*, hipStream_t);
