@@ -64,3 +64,18 @@ def test_faces_corners_and_many_elements(d):
     x[:200] = np.round(x[:200])                      # corners of the box
     x[200:400, 0] = np.round(x[200:400, 0] * res[0]) / res[0]  # element faces
     _check(d, res, x)
+
+
+@pytest.mark.parametrize("d", [2, 3])
+def test_many_elements_left_to_the_sequential_kernel(d):
+    """Several workgroups' worth of elements with ties, with 65-130 particles (on either side of the
+    128 that kernel holds) and with none of both, in every order."""
+    res = (29, 23) if d == 2 else (9, 8, 7)
+    E = int(np.prod(res))
+    rng = np.random.default_rng(9)
+    g = (np.arange(2) + 0.5) / 2
+    lat = np.stack(np.meshgrid(*([g] * d), indexing="ij"), -1).reshape(-1, d)
+    kind = rng.integers(0, 4, E)
+    sizes = np.choose(kind, [2 ** d, rng.integers(65, 131, E), rng.integers(33, 65, E), rng.integers(1, 33, E)])
+    it = iter(kind)
+    _check(d, res, _in_cells(res, sizes, rng, lambda n, dd, r: lat if next(it) == 0 else r.random((n, dd))))

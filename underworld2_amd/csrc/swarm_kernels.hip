@@ -426,8 +426,7 @@ template <int DIM, typename MT>
 __global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)) void k_dvc_rounds(long E, const int* __restrict__ cell_ptr,
                                                                         double* __restrict__ xi_slot,
                                                                         double* __restrict__ w_slot,
-                                                                        int* __restrict__ wide,
-                                                                        int* __restrict__ retry,
+                                                                        int* __restrict__ left,
                                                                         int* __restrict__ counts) {
   using D = DvcRound<DIM, MT>;
   constexpr int BS = D::BS, NPM = 8 * (int)sizeof(MT), NB = 2 * DIM;
@@ -451,28 +450,39 @@ __global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)
   const int tid = threadIdx.x, lane = tid & 63;
   const unsigned long long below = (1ull << lane) - 1ull;
   const double dx = (1.0 - -1.0) / kDvcNum, dy = dx, dz = dx;
-  const long n_el = WIDE ? (long)counts[0] : E;
-  if (blockIdx.x >= n_el) return;
+  if (WIDE && counts[5] == 0) return;
   if (tid == 0) {
     // cell centres: X = X + dx accumulation per axis (_DVCWeights_ConstructGrid :527-544)
     double X = -1.0 - dx / 2.0;
     for (int i = 0; i < kDvcNum; i++) { X = X + dx; cen[i] = X; }
     cen[kDvcNum] = 0.0;
   }
-  for (int q = tid; q < D::CELLS; q += BS) mask[q] = 0;
-  for (long it = blockIdx.x; it < n_el; it += gridDim.x) {
-    const long e = WIDE ? (long)wide[it] : it;
+  // An element left to the sequential kernel is marked by plain stores: one counter for them all
+  // serialises its atomics (20 ns each, a tenth of the pass where every element is left).
+  auto leave = [&](long e) {
+    left[e] = 1;
+    counts[0] = 1;
+  };
+  if (!WIDE)
+    for (int q = tid; q < D::CELLS; q += BS) mask[q] = 0;
+  bool clean = !WIDE;
+  for (long e = blockIdx.x; e < E; e += gridDim.x) {
     const int s0 = cell_ptr[e], np = cell_ptr[e + 1] - s0;
-    if (np <= 0 || np > NPM) {
-      if (tid == 0) {
+    if (!WIDE && tid == 0) left[e] = 0;
+    if (np <= (WIDE ? 32 : 0) || np > NPM) {
+      if (!WIDE && tid == 0) {
         if (np <= 0)
           atomicMin(&counts[2], (int)e);
-        else if (!WIDE && np <= 64)
-          wide[atomicAdd(&counts[0], 1)] = (int)e;
+        else if (np > 64)
+          leave(e);
         else
-          retry[atomicAdd(&counts[1], 1)] = (int)e;
+          counts[5] = 1;
       }
       continue;
+    }
+    if (!clean) {  // few elements need this kernel, where it is the second
+      for (int q = tid; q < D::CELLS; q += BS) mask[q] = 0;
+      clean = true;
     }
     __syncthreads();
     {
@@ -637,7 +647,7 @@ __global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)
     if (fail) {
       __syncthreads();
       for (int q = tid; q < D::CELLS; q += BS) mask[q] = 0;
-      if (tid == 0) retry[atomicAdd(&counts[1], 1)] = (int)e;
+      if (tid == 0) leave(e);
       continue;
     }
     // centroids and weights in grid order (_DVCWeights_GetCentroids3D :198-226): the cells are
@@ -721,6 +731,26 @@ __global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)
   }
 }
 
+// the elements left, in list[counts[3]], and the most particles of one of them, in counts[1]
+__global__ __launch_bounds__(256) void k_dvc_left(long E, const int* __restrict__ cell_ptr,
+                                                  const int* __restrict__ left, int* __restrict__ list,
+                                                  int* __restrict__ counts) {
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  const bool on = e < E && left[e];
+  const unsigned long long b = __ballot(on);
+  int np = on ? cell_ptr[e + 1] - cell_ptr[e] : 0;
+  for (int o = 32; o > 0; o >>= 1) np = max(np, __shfl_xor(np, o));
+  if (b == 0) return;
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (lane == 0) {
+    base = atomicAdd(&counts[3], __popcll(b));
+    atomicMax(&counts[1], np);
+  }
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (on) list[base + __popcll(b & ((1ull << lane) - 1ull))] = (int)e;
+}
+
 // One wavefront per element, grid-stride over elements.  The claim grid, a one-bit-per-cell
 // mark and the particles' local coordinates live in LDS (about 8 KB, so many elements are in
 // flight per CU); each particle's boundary chain lives in a per-workgroup global buffer
@@ -734,13 +764,16 @@ __global__ __launch_bounds__((DvcRound<DIM, MT>::BS), (DvcRound<DIM, MT>::WAVES)
 // weights and centroids, summed in grid order at the end - is exactly that of the sequential
 // algorithm above, bit for bit; only the order of cells inside a chain may differ.  Duplicate
 // neighbours are dropped by an atomic test-and-set on the mark bits.  Elements with more than
-// DVCW_MAXNP particles or a chain longer than `cap` are flagged and left to k_dvc.
+// `rows` particles (at most DVCW_MAXNP) or a chain longer than `cap` are listed and left to k_dvc.
+// Chains for the particles there are (rows) and not for 128: the buffer of 4,096 workgroups is
+// 115 KB each in 2D otherwise, and allocating it took as long as the kernel.
 #define DVCW_MAXNC 4096
 #define DVCW_MAXNP 128
 template <int DIM, int NUM>
 __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long nE, const int* __restrict__ elist,
                                                  const int* __restrict__ cell_ptr, double* __restrict__ xi_slot, double* __restrict__ w_slot,
-                                                 short* __restrict__ gbound, int cap, int* __restrict__ flag) {
+                                                 short* __restrict__ gbound, int rows, int cap, int* __restrict__ left,
+                                                 int* __restrict__ n_left) {
   const int num = NUM > 0 ? NUM : num_rt;  // compile-time grid size for the default resolution
   constexpr int NC = NUM > 0 ? (DIM == 3 ? NUM * NUM * NUM : NUM * NUM) : DVCW_MAXNC;  // claim grid cells
   constexpr int NCW = (NC + 31) / 32;                                                 // mark words
@@ -767,7 +800,7 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long nE, const int*
   }
   for (int q = lane; q < NCW; q += 64) mark[q] = 0u;
   // chains: buffer h (0/1) of particle p at gb + (2 p + h) * cap
-  short* gb = gbound + (long)blockIdx.x * 2 * DVCW_MAXNP * cap;
+  short* gb = gbound + (long)blockIdx.x * 2 * rows * cap;
   // neighbour k of cell c in the order S, N, E, W, U, D; -2 outside the grid.  Selects, not a
   // switch: k differs between lanes, and a branch per case costs scalar exec-mask work per lane
   // group
@@ -783,8 +816,8 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long nE, const int*
     const long e = elist ? (long)elist[it] : it;
     const int s0 = cell_ptr[e];
     const int np = cell_ptr[e + 1] - s0;
-    if (np <= 0 || np > DVCW_MAXNP) {
-      if (lane == 0) flag[it] = np <= 0 ? 2 : 1;
+    if (np <= 0 || np > rows) {
+      if (lane == 0) left[atomicAdd(n_left, 1)] = (int)e;
       continue;
     }
     for (int c = lane; c < ncell; c += 64) own[c] = 0xFF;
@@ -893,7 +926,7 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long nE, const int*
     if (overflow) {
       // leave LDS marks clean for the next element
       for (int q = lane; q < NCW; q += 64) mark[q] = 0u;
-      if (lane == 0) flag[it] = 1;
+      if (lane == 0) left[atomicAdd(n_left, 1)] = (int)e;
       __syncthreads();
       continue;
     }
@@ -961,7 +994,6 @@ __global__ __launch_bounds__(64) void k_dvc_wave(int num_rt, long nE, const int*
         if (DIM == 3) out[2] = 0.0;
       }
     }
-    if (lane == 0) flag[it] = 0;
     __syncthreads();
   }
 }
@@ -971,12 +1003,14 @@ bool dvc_wave_supported(int dim, int num) {
   return nc <= DVCW_MAXNC && num <= 32;
 }
 
-// elements elist[0 .. nE) (all elements where it is null)
+// elements elist[0 .. nE) (all elements where it is null), those left out appended to left[*n_left];
+// gbound: dvc_wave_bound_shorts(rows, cap) per workgroup
 void launch_dvc_wave(int dim, int num, long nE, const int* elist, const int* cell_ptr, double* xi_slot, double* w_slot,
-                     short* gbound, int nblk, int cap, int* flag, hipStream_t s) {
+                     short* gbound, int nblk, int rows, int cap, int* left, int* n_left, hipStream_t s) {
   if (nE == 0) return;
   const auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, nblk, 64, 0, s, num, nE, elist, cell_ptr, xi_slot, w_slot, gbound, cap, flag);
+    hipLaunchKernelGGL(kernel, nblk, 64, 0, s, num, nE, elist, cell_ptr, xi_slot, w_slot, gbound, rows, cap, left,
+                       n_left);
   };
   if (dim == 3 && num == 15)
     go(k_dvc_wave<3, 15>);
@@ -990,33 +1024,37 @@ void launch_dvc_wave(int dim, int num, long nE, const int* elist, const int* cel
 }
 
 __global__ void k_dvc_reset(int* counts) {
-  if (threadIdx.x < 2) counts[threadIdx.x] = 0;
-  if (threadIdx.x == 2) counts[2] = 0x7fffffff;
+  if (threadIdx.x < kDvcCounts) counts[threadIdx.x] = threadIdx.x == 2 ? 0x7fffffff : 0;
 }
 
-// DVC of all elements at the default resolution.  work [2 E + 4]: elements with 33-64 particles,
-// elements left to k_dvc_wave, then the counts of both and the first element without particles
-// (0x7fffffff: none).  Returns the counts' address.
+// DVC of all elements at the default resolution.  left [E]: whether an element is left to
+// k_dvc_wave; counts: whether any is, a zero, the first element without particles (0x7fffffff:
+// none), two zeros, and whether any has 33-64 particles.  launch_dvc_left then lists the elements, with the most particles of one
+// in counts[1] and their number in counts[3].
 bool dvc_rounds_supported(int num) { return num == kDvcNum; }
-int* launch_dvc_rounds(int dim, long E, const int* cell_ptr, double* xi_slot, double* w_slot, int cus, int* work,
-                       hipStream_t s) {
-  int *wide = work, *retry = work + E, *counts = work + 2 * E;
+void launch_dvc_rounds(int dim, long E, const int* cell_ptr, double* xi_slot, double* w_slot, int cus, int* left,
+                       int* counts, hipStream_t s) {
   hipLaunchKernelGGL(k_dvc_reset, 1, 64, 0, s, counts);
-  const auto go = [&](auto k32, auto k64, int bs, int per32, int per64) {
-    hipLaunchKernelGGL(k32, (unsigned)std::min(E, (long)cus * per32), bs, 0, s, E, cell_ptr, xi_slot, w_slot, wide,
-                       retry, counts);
-    hipLaunchKernelGGL(k64, (unsigned)std::min(E, (long)cus * per64), bs, 0, s, E, cell_ptr, xi_slot, w_slot, wide,
-                       retry, counts);
+  const auto go = [&](auto kernel, int bs, int per) {
+    hipLaunchKernelGGL(kernel, (unsigned)std::min(E, (long)cus * per), bs, 0, s, E, cell_ptr, xi_slot, w_slot, left,
+                       counts);
   };
-  if (dim == 3)
-    go(k_dvc_rounds<3, unsigned>, k_dvc_rounds<3, unsigned long long>, DvcRound<3, unsigned>::BS, 20, 12);
-  else
-    go(k_dvc_rounds<2, unsigned>, k_dvc_rounds<2, unsigned long long>, DvcRound<2, unsigned>::BS, 64, 48);
+  if (dim == 3) {
+    go(k_dvc_rounds<3, unsigned>, DvcRound<3, unsigned>::BS, 20);
+    go(k_dvc_rounds<3, unsigned long long>, DvcRound<3, unsigned>::BS, 12);
+  } else {
+    go(k_dvc_rounds<2, unsigned>, DvcRound<2, unsigned>::BS, 64);
+    go(k_dvc_rounds<2, unsigned long long>, DvcRound<2, unsigned>::BS, 48);
+  }
   UWG_HIP(hipGetLastError());
-  return counts;
+}
+void launch_dvc_left(long E, const int* cell_ptr, const int* left, int* list, int* counts, hipStream_t s) {
+  hipLaunchKernelGGL(k_dvc_left, nblocks(E, 256), 256, 0, s, E, cell_ptr, left, list, counts);
+  UWG_HIP(hipGetLastError());
 }
 
-long dvc_wave_bound_shorts(int cap) { return 2L * DVCW_MAXNP * cap; }
+int dvc_wave_rows(int max_np) { return std::min(std::max(max_np, 1), DVCW_MAXNP); }
+long dvc_wave_bound_shorts(int rows, int cap) { return 2L * rows * cap; }
 
 long dvc_scratch_bytes(int dim, int num, int max_np, int cap) {
   int ncell = num * num * (dim == 3 ? num : 1);

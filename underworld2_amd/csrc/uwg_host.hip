@@ -157,7 +157,7 @@ struct uwg_swarm {
   double* xi_slot = nullptr;  // [cap][dim]
   double* w_slot = nullptr;   // [cap]
   int* slot_cell = nullptr;   // [cap]
-  int* dvc_work = nullptr;    // element lists of the DVC, [2 E + 4]
+  int* dvc_work = nullptr;    // flags, list and counts of the DVC, [2 E + kDvcCounts]
   int* moves = nullptr;       // counters of an advection step that leaves the owners, [2]
   bool has_mat = false;
   bool has_integration = false;
@@ -692,45 +692,48 @@ static int run_dvc(uwg_swarm* s, int dvc_res) {
   int dev = 0, cus = 0;
   UWG_HIP(hipGetDevice(&dev));
   UWG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+  if (!s->dvc_work) s->dvc_work = dalloc<int>(2 * E + kDvcCounts);
+  int* counts = s->dvc_work + 2 * E;
   long todo = E;               // elements for the kernels below
   const int* elist = nullptr;  // their indices (null: all)
+  int maxc = 0;                // and the most particles of one
   if (dvc_rounds_supported(dvc_res)) {
-    if (!s->dvc_work) s->dvc_work = dalloc<int>(2 * E + 4);
-    const int* counts = launch_dvc_rounds(g.dim, E, s->cell_ptr, s->xi_slot, s->w_slot, cus, s->dvc_work, 0);
-    int h[3];
+    int *left = s->dvc_work, *list = s->dvc_work + E, h[4];
+    launch_dvc_rounds(g.dim, E, s->cell_ptr, s->xi_slot, s->w_slot, cus, left, counts, 0);
     UWG_HIP(hipMemcpy(h, counts, sizeof(h), hipMemcpyDeviceToHost));
     if (h[2] != 0x7fffffff) return underresolved(h[2]);
-    if (h[1] == 0) return 0;
-    todo = h[1];
-    elist = s->dvc_work + E;
-  }
-  // per-cell counts for capacity planning
-  std::vector<int> ptr(E + 1);
-  UWG_HIP(hipMemcpy(ptr.data(), s->cell_ptr, sizeof(int) * (E + 1), hipMemcpyDeviceToHost));
-  int maxc = 0;
-  for (long e = 0; e < E; e++) {
-    int c = ptr[e + 1] - ptr[e];
-    if (c == 0) return underresolved(e);
-    maxc = std::max(maxc, c);
+    if (!h[0]) return 0;
+    launch_dvc_left(E, s->cell_ptr, left, list, counts, 0);
+    UWG_HIP(hipMemcpy(h, counts, sizeof(h), hipMemcpyDeviceToHost));
+    maxc = h[1];
+    todo = h[3];
+    elist = list;
+  } else {
+    std::vector<int> ptr(E + 1);
+    UWG_HIP(hipMemcpy(ptr.data(), s->cell_ptr, sizeof(int) * (E + 1), hipMemcpyDeviceToHost));
+    for (long e = 0; e < E; e++) {
+      int c = ptr[e + 1] - ptr[e];
+      if (c == 0) return underresolved(e);
+      maxc = std::max(maxc, c);
+    }
+    UWG_HIP(hipMemset(counts, 0, sizeof(int) * kDvcCounts));
   }
   const int ncell = dvc_res * dvc_res * (g.dim == 3 ? dvc_res : 1);
   std::vector<int> retry;
   if (dvc_wave_supported(g.dim, dvc_res)) {
-    // one wavefront per element; elements it cannot hold are flagged for the per-thread kernel
-    const int cap = std::min(512, ncell);
+    // one wavefront per element; elements it cannot hold are listed for the per-thread kernel
+    const int cap = std::min(512, ncell), rows = dvc_wave_rows(maxc);
     // 16 workgroups per CU (19 fit in LDS; measured per pass at 128^3: 12 -> 659 ms, 16 -> 559 ms,
     // 19 -> 684 ms)
     const int nblk = (int)std::min<long>(todo, (long)cus * 16);
-    short* gb = dalloc<short>(dvc_wave_bound_shorts(cap) * nblk);
-    int* flag = dalloc<int>(todo);
-    launch_dvc_wave(g.dim, dvc_res, todo, elist, s->cell_ptr, s->xi_slot, s->w_slot, gb, nblk, cap, flag, 0);
-    std::vector<int> hflag(todo), el(elist ? todo : 0);
-    UWG_HIP(hipMemcpy(hflag.data(), flag, sizeof(int) * todo, hipMemcpyDeviceToHost));
-    if (elist) UWG_HIP(hipMemcpy(el.data(), elist, sizeof(int) * todo, hipMemcpyDeviceToHost));
-    for (long t = 0; t < todo; t++)
-      if (hflag[t]) retry.push_back(elist ? el[t] : (int)t);
+    short* gb = dalloc<short>(dvc_wave_bound_shorts(rows, cap) * nblk);
+    launch_dvc_wave(g.dim, dvc_res, todo, elist, s->cell_ptr, s->xi_slot, s->w_slot, gb, nblk, rows, cap, s->dvc_work,
+                    counts + 4, 0);
+    int n = 0;
+    UWG_HIP(hipMemcpy(&n, counts + 4, sizeof(int), hipMemcpyDeviceToHost));
+    retry.resize(n);
+    if (n > 0) UWG_HIP(hipMemcpy(retry.data(), s->dvc_work, sizeof(int) * n, hipMemcpyDeviceToHost));
     dfree(gb);
-    dfree(flag);
   } else {
     int max_np = std::min(std::max(64, ((maxc + 15) / 16) * 16), 32000);
     int cap = std::min(512, ncell);

@@ -140,7 +140,8 @@ void launch_restrict2(const Geom& fine, const Geom& coarse, const T* rf, T* rc, 
 void set_apply_chunk(int kz3, int kz2);
 long dvc_scratch_bytes(int dim, int num, int max_np, int cap);
 bool dvc_wave_supported(int dim, int num);
-long dvc_wave_bound_shorts(int cap);
+int dvc_wave_rows(int max_np);
+long dvc_wave_bound_shorts(int rows, int cap);
 // fn_kernels.hip: per-particle function programs and general field interpolation
 void launch_fn_eval(const Geom& g, long P, const double* coords, const int* mat, const void* prog, int nins,
                     const double* consts, const double* const* fields, const int* field_nc, int nfields,
@@ -149,10 +150,12 @@ void launch_fn_eval(const Geom& g, long P, const double* coords, const int* mat,
 void launch_field_interpolate(const Geom& g, long P, const double* f, int nc, const double* x, double* v, int* ok,
                               hipStream_t s);
 void launch_dvc_wave(int dim, int num, long nE, const int* elist, const int* cell_ptr, double* xi_slot, double* w_slot,
-                     short* gbound, int nblk, int cap, int* flag, hipStream_t s);
+                     short* gbound, int nblk, int rows, int cap, int* left, int* n_left, hipStream_t s);
+constexpr int kDvcCounts = 6;
 bool dvc_rounds_supported(int num);
-int* launch_dvc_rounds(int dim, long E, const int* cell_ptr, double* xi_slot, double* w_slot, int cus, int* work,
-                       hipStream_t s);
+void launch_dvc_rounds(int dim, long E, const int* cell_ptr, double* xi_slot, double* w_slot, int cus, int* left,
+                       int* counts, hipStream_t s);
+void launch_dvc_left(long E, const int* cell_ptr, const int* left, int* list, int* counts, hipStream_t s);
 void launch_dvc_list(int dim, int num, long E0, long nE, const int* elist, const int* cell_ptr,
                      double* xi_slot, double* w_slot, void* scratch, int max_np, int cap, int* d_flag,
                      hipStream_t s);
