@@ -5,8 +5,8 @@ chunk, themselves checked against the oracle in test_gpu_parity3d.py).
 and the order of the node sums, so every value is equal; grids at the tile edges (7 columns), the
 level counts 2, 3 and 4 of its dispatch and one element.
 2D: the assembled stencil sums the same terms in another order: per row 36 products and sums of
-rounding u each, so |dy| <= 40 u sum|K||x| (u = 2^-53, 2^-24); FP32 entries add u.  Irregular
-Dirichlet masks reach every form of the row-sum block."""
+rounding u each, so |dy| <= 40 u sum|K||x| (u = 2^-53, 2^-24), row by row; FP32 entries add u.
+Irregular Dirichlet masks reach every form of the row-sum block."""
 import numpy as np
 import pytest
 
@@ -62,21 +62,16 @@ def test_2d_stencil_against_element_kernel(res, mask):
     try:
         L.lib().uwg_set_apply_chunk(0, 1)
         ref = [_apply(st, w, x) for w in (0, 4, 6, 7)]
-        # sum |K| |x| row by row is bounded by the largest row sum times max |x|; the row sum of
-        # |K| is at most 18 times its largest entry, itself at most the largest diagonal entry
-        n = x.size
-        diag = np.zeros(n)
-        for c in range(18):  # the diagonal by colouring: unit vectors three nodes apart
+        # sum |K| |x| row by row: of the nodes three apart in either direction a row meets one
+        rows = np.abs(x)
+        for c in range(18):
             e = np.zeros((res[1] + 1, res[0] + 1, 2))
             e[(c // 2) // 3::3, (c // 2) % 3::3, c % 2] = 1.0
-            e = e.ravel()
-            diag += e * _apply(st, 0, e)
+            rows = rows + np.abs(_apply(st, 0, e.ravel() * x))
     finally:
         L.lib().uwg_set_apply_chunk(0, -1)
-    bound = 40 * 18 * diag.max() * np.abs(x).max()
     for a, b, u in zip(got, ref, (2.0 ** -53, 2.0 ** -24, 2.0 ** -53, 2.0 ** -24)):
-        assert np.abs(a - b).max() <= u * bound
-        assert np.linalg.norm(a - b) <= 20 * u * np.linalg.norm(b)
+        assert (np.abs(a - b) <= 40 * u * rows).all()
 
 
 @pytest.mark.parametrize("res", [(31, 29), (64, 5)])
