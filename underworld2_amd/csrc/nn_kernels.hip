@@ -13,9 +13,9 @@
 // R is the transpose of P, so the backward pass of a pooling is the other operator.
 //
 // Every convolution is 3x3x3 with zero padding; activations are [B][C][N] (N = nx*ny*nz,
-// x fastest).  Grids here are at most 33^3 nodes, where direct convolution with weights
-// broadcast from the scalar cache is latency-bound rather than FLOP-bound, so MFMA tiles
-// would not pay.
+// x fastest).  The U-net's grids are at most 33^3 nodes, whose convolutions are bound by latency.
+// The Schur-stencil network (below) runs on element grids, 128^3 in the benchmark's solve and 48^3
+// in training, with the same kernels on vector FP32; matrix cores have not been tried there.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -381,7 +381,10 @@ __global__ void k_sum_parts(long n, int nchunk, const float* __restrict__ part, 
 
 // Chunks of T points for `pairs` workgroups per chunk: about 2,048 workgroups (eight per CU), each
 // thread with at least eight points so that the closing sums stay a small part.  Up to kWgradOne
-// points (32 per thread) one workgroup per output pair is as fast, without partial sums.
+// points one workgroup per output pair takes them all, without a launch for partial sums and in
+// the order in which training on such grids has always summed: loss and gradient at 512 points
+// with 8 / 32 channels 236 / 473 us against 262 / 493 in chunks, 4,096 points 260 / 459 against
+// 288 / 477, 8,192 points 300 / 519 against 295 / 504.
 constexpr long kWgradOne = 8192;
 constexpr int kWgradCo = 4, kWgradC = 4;
 static int wgrad_chunks(long T, long pairs) {

@@ -250,16 +250,18 @@ void vk_multi_axpy(long n, int k, const T* const* X, const double* c, T* y, hipS
 // partial sums for dot products: out[j] = <x, Y[j]> for j < k ; deterministic
 template <typename T>
 void vk_multi_dot(long n, int k, const T* x, const T* const* Y, double* partial, double* out, hipStream_t s);
-// one classical Gram-Schmidt step with device-resident coefficients: h[0..k) = V^T w,
-// w -= sum h_j V_j, h[k] = |w|^2 (bit-identical to a separate dot), v_next = w / |w| (skipped
-// when |w| = 0).  The basis V (and v_next) may be stored in a narrower type TV than w; every
-// product and sum is in double.  partial holds 32 x vk_reduce_blocks() doubles
 // a Gram-Schmidt step's coefficients in host memory that the device writes; seq is written last.
 // Room for restarts up to 255, as in the device's copy.
 struct HostColumn {
   double h[256];
   unsigned long long seq;
 };
+// one classical Gram-Schmidt step with device-resident coefficients: h[0..k) = V^T w,
+// w -= sum h_j V_j, h[k] = |w|^2 (bit-identical to a separate dot), v_next = w / |w| (skipped
+// when |w| = 0).  The basis V (and v_next) may be stored in a narrower type TV than w; every
+// product and sum is in double.  partial holds 32 x vk_reduce_blocks() doubles.  out receives
+// h[0..k] and then seq, while the stream may still be writing v_next; the caller gives every step
+// another seq and reads the column when it sees that one (or after waiting for the stream)
 template <typename TW, typename TV>
 void vk_gs_step(long n, int k, const TV* const* V, TW* w, TV* v_next, double* h, double* partial, HostColumn* out,
                 unsigned long long seq, hipStream_t s);
