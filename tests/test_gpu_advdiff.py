@@ -78,6 +78,12 @@ def test_supg_steps_match_oracle(res):
     assert np.array_equal(phi.data[bcmask, 0], p[bcmask])
 
 
+@pytest.mark.parametrize("res", [(1, 1), (16, 8), (43, 3), (17, 15), (1, 1, 1), (4, 4, 8), (43, 3, 1)])
+def test_supg_steps_at_the_edges_of_workgroups(res):
+    """1, 128, 129 and 255 elements, 128 to a workgroup."""
+    test_supg_steps_match_oracle(res)
+
+
 def test_supg_linear_field_closed_form():
     import underworld2_amd as uw
     res = (14, 12)

@@ -131,11 +131,13 @@ __device__ __forceinline__ const SupgRule<DIM>& supg_rule() {
 }
 
 // FP64 arithmetic bound (about 9,000 operations per 3D element: multiplies and adds stay separate,
-// see the build flags).  The rule's tables are wave-uniform and come through scalar registers; the
-// diffusivities, 27 consecutive values per element, are staged in LDS by coalesced loads.  Forming
-// the shape functions per thread with indices the compiler kept in scratch, and reading the
-// diffusivities with a 216-byte stride, took 470 us for 64^3 elements; this takes
-// 108 us.
+// see the build flags).  The rule's tables are wave-uniform and come through scalar registers.  3D:
+// the diffusivities, 27 consecutive values per element, are staged in LDS by coalesced loads.
+// Forming the shape functions per thread with indices the compiler kept in scratch, and reading
+// the diffusivities with a 216-byte stride, took 470 us for 64^3 elements; this takes 108 us.  2D is
+// bound by latency up to some 200^2 elements: its nine values go to registers at once and its
+// points are unrolled, so that no point waits for its tables: 64^2 8.6 us before both, 9.1 with
+// staging and a loop, 6.7 now (256^2 13.2, 12.6, 9.6).
 constexpr int kSupgBlock = 128;
 template <int DIM>
 __global__ __launch_bounds__(kSupgBlock, 2) void k_supg_elem(ADGeom G, const double* __restrict__ phi,
@@ -145,16 +147,21 @@ __global__ __launch_bounds__(kSupgBlock, 2) void k_supg_elem(ADGeom G, const dou
                                                              const double* __restrict__ src, int upwind,
                                                              double* __restrict__ res_e) {
   constexpr int NN = DIM == 3 ? 8 : 4, Q = DIM == 3 ? 27 : 9;
-  __shared__ double ks[kSupgBlock * Q];
+  __shared__ double ks[DIM == 3 ? kSupgBlock * Q : 1];
   const long e0 = (long)blockIdx.x * kSupgBlock, e = e0 + threadIdx.x;
-  {
+  double kr[DIM == 3 ? 1 : Q];
+  if constexpr (DIM == 3) {
     const double* kb = kap + e0 * Q;
     const int n = (int)min((long)kSupgBlock, G.E - e0) * Q;
     for (int q = threadIdx.x; q < n; q += kSupgBlock) ks[q] = kb[q];
+    __syncthreads();
+    if (e >= G.E) return;
+  } else {
+    if (e >= G.E) return;
+#pragma unroll
+    for (int q = 0; q < Q; q++) kr[q] = kap[e * Q + q];
   }
-  __syncthreads();
-  if (e >= G.E) return;
-  const double* kq_ = ks + threadIdx.x * Q;
+  const double* kq_ = DIM == 3 ? ks + threadIdx.x * Q : kr;
   const SupgRule<DIM>& R = supg_rule<DIM>();
   double V[24];
   element_verts<DIM>(G.res, G.lo, G.hi, e, V);
@@ -177,6 +184,7 @@ __global__ __launch_bounds__(kSupgBlock, 2) void k_supg_elem(ADGeom G, const dou
   }
   // upwind diffusivity (element mean diffusivity, velocity at the centre)
   double avg = 0.0;
+#pragma unroll
   for (int q = 0; q < Q; q++) avg += kq_[q];
   avg /= (double)Q;
   if (avg < AD_MIN_DIFFUSIVITY) avg = AD_MIN_DIFFUSIVITY;
@@ -196,7 +204,8 @@ __global__ __launch_bounds__(kSupgBlock, 2) void k_supg_elem(ADGeom G, const dou
 #pragma unroll
   for (int d = 0; d < DIM; d++) sc[d] = 2.0 / h[d];
   double r[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 1
+  constexpr int UNROLL = DIM == 3 ? 1 : Q;
+#pragma unroll UNROLL
   for (int q = 0; q < Q; q++) {
     double dN[3][8];
 #pragma unroll
