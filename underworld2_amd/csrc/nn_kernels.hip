@@ -82,7 +82,7 @@ __global__ void k_conv_fwd(int B, int Ci, int Co, Grid3 g, const float* __restri
 // BWD: the input gradient of the same convolution, din[ci][p] = sum_co sum_tap w[co][ci][tap]
 // dout[co][p - off(tap)]: in is dout (Ci = its channels), out is din (Co = its channels).  Its own
 // kernel with four channels per thread and scalar weight loads took 405 us for 16 x 16 channels at
-// 4 x 48^3, this 150 us.
+// 4 x 48^3, this 178 us.
 template <int COB, bool BWD = false>
 __global__ __launch_bounds__(256) void k_conv_fwd_blk(int B, int Ci, int Co, Grid3 g, const float* __restrict__ in,
                                                       const float* __restrict__ w, const float* __restrict__ bias,
