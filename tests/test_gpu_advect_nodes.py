@@ -26,8 +26,8 @@ def test_positions_are_the_oracle_s(res):
 
 
 def test_advection_that_keeps_owners_takes_no_relocation_workspace():
-    """The workspace (24 bytes per particle) is for calls that update owners; without, a step needs two
-    counters.  Allocations are whole 2 MiB pages."""
+    """The workspace (24 bytes per particle, 31 MB here) is for calls that update owners; without, a step
+    needs two counters.  Allocations are whole 2 MiB pages, and a kernel's first launch may take some."""
     import ctypes
     import underworld2_amd as uw
     from underworld2_amd import _lib as L
@@ -45,4 +45,4 @@ def test_advection_that_keeps_owners_takes_no_relocation_workspace():
     before = free()
     out = ctypes.c_long()
     L.check(L.lib().uwg_advect_rk2(sw._h, vel._h, 1e-3, 0, ctypes.byref(out)))
-    assert before - free() <= 2 << 20
+    assert before - free() <= 8 << 20
